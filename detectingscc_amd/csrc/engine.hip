@@ -88,7 +88,11 @@ scc_status Engine::init(int dev)
     HIP_TRY(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
     HIP_TRY(hipHostMalloc((void **)&h_ctr, CT(kCtrLines) * sizeof(uint32_t), hipHostMallocDefault));
     HIP_TRY(hipMalloc((void **)&st.ctr, CT(kCtrLines) * sizeof(uint32_t)));
-    HIP_TRY(hipMemset(st.ctr, 0, CT(kCtrLines) * sizeof(uint32_t)));
+    // on the engine's stream: it does not wait for the null stream, where a
+    // memset may still be queued (behind another engine's kernels, say) when
+    // this call returns, and would then clear the counters of a later run
+    k_fill_u32(stream, st.ctr, 0u, CT(kCtrLines));
+    HIP_TRY(hipGetLastError());
     // counters published into mapped, coherent host memory: C_COUNT lines
     // plus one line for the sequence word (without it, read-backs copy and
     // synchronise the stream)
