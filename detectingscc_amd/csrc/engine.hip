@@ -332,9 +332,11 @@ __global__ void publish_ctr_kernel(const uint32_t *ctr, uint32_t *pub, uint32_t 
     if (i < C_COUNT) {
         for (int w = 0; w < kPubWords; w++) pub[CT(i) + w] = ctr[CT(i) + w];
         if (spread_index((int)i) >= 0) {
-            uint32_t t = ctr[CT(i)];
-            for (int j = 0; j < kSpread; j++) t += ctr[CSLOT((int)i, j)];
-            pub[CT(i)] = t;
+            // the second word of a 32-bit counter's lines is 0
+            uint64_t t = *reinterpret_cast<const uint64_t *>(ctr + CT(i));
+            for (int j = 0; j < kSpread; j++) t += *reinterpret_cast<const uint64_t *>(ctr + CSLOT((int)i, j));
+            pub[CT(i)] = (uint32_t)t;
+            if (wide_counter((int)i)) pub[CT(i) + 1] = (uint32_t)(t >> 32);
         }
     }
     __threadfence_system();
@@ -366,8 +368,13 @@ scc_status Engine::wait_ctr(uint32_t seq)
         HIP_TRY(hipMemcpyAsync(h_ctr, st.ctr, CT(kCtrLines) * sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
         HIP_TRY(hipStreamSynchronize(stream));
         for (int i = 0; i < C_COUNT; i++)
-            if (spread_index(i) >= 0)
-                for (int j = 0; j < kSpread; j++) h_ctr[CT(i)] += h_ctr[CSLOT(i, j)];
+            if (spread_index(i) >= 0) {
+                uint64_t t = h_ctr[CT(i)] | ((uint64_t)h_ctr[CT(i) + 1] << 32);
+                for (int j = 0; j < kSpread; j++)
+                    t += h_ctr[CSLOT(i, j)] | ((uint64_t)h_ctr[CSLOT(i, j) + 1] << 32);
+                h_ctr[CT(i)] = (uint32_t)t;
+                if (wide_counter(i)) h_ctr[CT(i) + 1] = (uint32_t)(t >> 32);
+            }
         return SCC_OK;
     }
     HIP_TRY(hipGetLastError());
@@ -749,7 +756,7 @@ scc_status Engine::pivot_round(bool first, int expand, int W, scc_stats *stats, 
     if (!first) {
         zero_ctr(C_NPIV, 1);
         k_elect(stream, g, st);
-        k_select(stream, g, st, 1);
+        k_select(stream, g, st);
     }
     mark(SCC_PHASE_REACH, first);   // the first search is always timed
     const int first_mark = (int)nmarks - 1;

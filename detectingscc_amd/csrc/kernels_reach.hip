@@ -759,6 +759,28 @@ __device__ __forceinline__ void bu_level(const DirArgs &D, const uint32_t *__res
     wave_flush_block(wq, nq, cnt_out, qout, qcap, anom);
 }
 
+// Adds the workgroup's work units to slot blockIdx.x % kSpread of the
+// counters C_WORK (the counted run only; every thread of a workgroup of up
+// to 1,024 calls).  With an atomic per wave and unit on one line each, R-MAT
+// scale 20's two widest counted levels took 215 and 205 us; now 28 and 24.
+__device__ __forceinline__ void add_work(uint32_t *ctr, const WorkCount &wc)
+{
+    __shared__ uint32_t s_w[8][16];
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        uint32_t x = wc.n[k];
+        for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
+        if (wlane() == 0) s_w[k][threadIdx.x >> 6] = x;
+    }
+    __syncthreads();
+    if (threadIdx.x >= 8) return;
+    unsigned long long t = 0;
+    for (uint32_t w = 0; w < (blockDim.x >> 6); w++) t += s_w[threadIdx.x][w];
+    if (t)
+        atomicAdd(reinterpret_cast<unsigned long long *>(
+                      ctr + CSLOT(C_WORK, (int)(threadIdx.x * kSpread + blockIdx.x % kSpread))), t);
+}
+
 // ---------------------------------------------------------------------
 // Direction-optimised level decided on the device.  Every workgroup of the
 // level-L launch recomputes each direction's mode from the mode and visited
@@ -767,19 +789,6 @@ __device__ __forceinline__ void bu_level(const DirArgs &D, const uint32_t *__res
 // stores the result in slot L&1 for level L+1.  So the host can queue any
 // number of levels without reading counters in between; a direction that
 // has finished turns its workgroups into no-ops.
-// Adds each lane's work units to the counters, one 64-bit atomic per wave
-// and unit (the counted run only).
-__device__ __forceinline__ void add_work(uint32_t *ctr, const WorkCount &wc)
-{
-#pragma unroll
-    for (int k = 0; k < 8; k++) {
-        uint32_t x = wc.n[k];
-        for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
-        if (wlane() == 0 && x)
-            atomicAdd(reinterpret_cast<unsigned long long *>(ctr + CT(C_WORK + k)), (unsigned long long)x);
-    }
-}
-
 template <bool SINGLE, bool COUNT>
 // At most 80 scalar registers (the compiler moves the rest to vector lanes):
 // with 86 to 102 (the sparse steps' uniform masks) R-MAT scale 24's dense

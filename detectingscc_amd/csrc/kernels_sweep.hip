@@ -19,20 +19,6 @@ namespace sccamd {
 
 __device__ __forceinline__ uint32_t lane() { return threadIdx.x & 63u; }
 
-// pivot key of v from its out-degree and in-degree
-__device__ __forceinline__ uint64_t pivot_key_deg(uint32_t outdeg, uint32_t indeg, uint32_t v)
-{
-    uint64_t p = (uint64_t)outdeg * (uint64_t)indeg;
-    p = p > 0xFFFFFFFFull ? 0xFFFFFFFFull : p;
-    return (p << 32) | (uint64_t)(0xFFFFFFFFu - v);
-}
-
-__device__ __forceinline__ uint64_t pivot_key(const uint32_t *__restrict__ Fr,
-                                              const uint32_t *__restrict__ Br, uint32_t v)
-{
-    return pivot_key_deg(Fr[v + 1] - Fr[v], Br[v + 1] - Br[v], v);
-}
-
 __device__ __forceinline__ uint32_t key_vertex(uint64_t k) { return 0xFFFFFFFFu - (uint32_t)k; }
 
 // visited (or finished) bit of v in fvis / bvis
@@ -753,79 +739,178 @@ void k_init_vis(hipStream_t s, const DevGraph &g, DevState &st, bool elect_first
     }
 }
 
+// ----------------------------------------------- per-id LDS tables ---
+// Reductions into a word per class, label or size (elections, label minima,
+// SCC sizes, the size histogram) meet few large ids (a giant SCC, a few
+// hundred partitions) or many small ones.  A workgroup keeps the running
+// values of up to TAB_SLOTS ids in an LDS table -- an id takes the slot it
+// hashes to, the first to come keeps it -- and adds them to memory once, at
+// its end; only an id whose slot is another's goes to memory lane by lane.
+// The grid is TAB_BLOCKS workgroups at most, which bounds the closing
+// atomics on one address (about 12 ns each, one after another).
+constexpr uint32_t TAB_SLOTS = 1024;
+constexpr uint32_t TAB_BLOCK = 512;
+constexpr uint32_t TAB_BLOCKS = 512;
+constexpr uint32_t TAB_FREE = DEAD;   // no id
+
+static uint32_t tab_blocks(uint32_t V) { return std::min<uint32_t>(TAB_BLOCKS, V / TAB_BLOCK + 1); }
+
+// id's slot, or TAB_SLOTS if another id holds it
+__device__ __forceinline__ uint32_t tab_slot(uint32_t *ids, uint32_t id)
+{
+    const uint32_t slot = (id * 2654435761u) >> 22;
+    uint32_t own = ids[slot];
+    if (own == TAB_FREE) {
+        own = atomicCAS(&ids[slot], TAB_FREE, id);
+        if (own == TAB_FREE) own = id;
+    }
+    return own == id ? slot : TAB_SLOTS;
+}
+static_assert(TAB_SLOTS == 1u << 10, "tab_slot takes the hash's top 10 bits");
+
 // ------------------------------------------------------------ pivots ---
 // pollForPivots / pollForFirstPivot (scc_kernels.cu:57-74, 643-656) with a
 // 64-bit key so the winner is the true argmax and every class elects one
-// vertex (defects D4, D10).  A wave whose live lanes share a class does one
-// atomic.  The key's degree product is DP[v] (built for every live vertex
-// at the start of the decomposition), read with the class word rather than
-// four row offsets after it.  Each chunk reads its classes' current maxima
-// just before its atomics, so most lanes see a maximum an earlier chunk has
-// raised and issue none (deciding four chunks against one read of the
-// maxima, with their atomics issued together, doubled the time on a graph
-// with about 600 classes: more lanes act on maxima that are out of date).
-__global__ void elect_kernel(const uint32_t *__restrict__ DP, const uint32_t *__restrict__ cls,
-                             unsigned long long *piv, uint32_t V)
+// vertex (defects D4, D10).  The key's degree product is DP[v] (built for
+// every live vertex at the start of the decomposition), read with the class
+// word.
+//
+// The largest key of each class goes through the workgroup's LDS table: 200
+// partition classes of 8.4M vertices, ids permuted (a wave's lanes all in
+// different classes), took 165 us with a global atomic per lane that beat
+// the value it had read, 73 us so.
+constexpr uint32_t ELECT_CHUNKS = 2;
+
+__global__ __launch_bounds__(TAB_BLOCK) void elect_kernel(const uint32_t *__restrict__ DP,
+                                                            const uint32_t *__restrict__ cls,
+                                                            unsigned long long *piv, uint32_t V)
 {
-    WAVE_LOOP(v, valid, V)
-    {
-        const uint32_t vv = valid ? v : 0u;   // vertex 0: the dummy, dead
-        const uint32_t c = cls[vv], dp = DP[vv];
-        const bool ok = c != DEAD;
-        const uint64_t live = __ballot(ok);
-        if (!live) continue;
-        const int L = __ffsll((unsigned long long)live) - 1;
-        const uint32_t c0 = __shfl(c, L);
-        const unsigned long long key = ok ? (((uint64_t)dp << 32) | (uint64_t)(0xFFFFFFFFu - v)) : 0ull;
-        if (__all(!ok || c == c0)) {
-            unsigned long long m = key;
-            for (int o = 32; o > 0; o >>= 1) {
-                unsigned long long x = __shfl_xor(m, o);
-                m = x > m ? x : m;
-            }
-            if ((int)lane() == L && m > piv[c0]) atomicMax(&piv[c0], m);
-        } else if (ok && key > piv[c]) {
-            atomicMax(&piv[c], key);
+    __shared__ uint32_t s_cls[TAB_SLOTS];
+    __shared__ unsigned long long s_key[TAB_SLOTS];
+    for (uint32_t i = threadIdx.x; i < TAB_SLOTS; i += TAB_BLOCK) {
+        s_cls[i] = TAB_FREE;
+        s_key[i] = 0;
+    }
+    __syncthreads();
+    auto add = [&](uint32_t c, unsigned long long k) {
+        const uint32_t slot = tab_slot(s_cls, c);
+        if (slot < TAB_SLOTS) {
+            if (k > s_key[slot]) atomicMax(&s_key[slot], k);
+        } else if (k > piv[c]) {
+            atomicMax(&piv[c], k);
         }
+    };
+    const uint32_t stride = gridDim.x * TAB_BLOCK;
+    for (uint32_t base = blockIdx.x * TAB_BLOCK + (threadIdx.x & ~63u); base <= V; base += ELECT_CHUNKS * stride) {
+        uint32_t v[ELECT_CHUNKS], c[ELECT_CHUNKS], dp[ELECT_CHUNKS];
+#pragma unroll
+        for (uint32_t h = 0; h < ELECT_CHUNKS; h++) {
+            v[h] = base + h * stride + lane();
+            const uint32_t vv = v[h] <= V ? v[h] : 0u;   // vertex 0: the dummy, dead
+            c[h] = cls[vv];
+            dp[h] = DP[vv];
+        }
+#pragma unroll
+        for (uint32_t h = 0; h < ELECT_CHUNKS; h++) {
+            const bool ok = c[h] != DEAD;
+            const uint64_t live = __ballot(ok);
+            if (!live) continue;
+            const int L = __ffsll((unsigned long long)live) - 1;
+            const uint32_t c0 = __shfl(c[h], L);
+            unsigned long long k = ok ? (((uint64_t)dp[h] << 32) | (uint64_t)(0xFFFFFFFFu - v[h])) : 0ull;
+            if (__all(!ok || c[h] == c0)) {
+                for (int o = 32; o > 0; o >>= 1) {
+                    const unsigned long long x = __shfl_xor(k, o);
+                    k = x > k ? x : k;
+                }
+                if ((int)lane() == L) add(c0, k);
+            } else if (ok) {
+                add(c[h], k);
+            }
+        }
+    }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < TAB_SLOTS; i += TAB_BLOCK) {
+        const uint32_t c = s_cls[i];
+        if (c != TAB_FREE &&
+            s_key[i] > __hip_atomic_load(&piv[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+            atomicMax(&piv[c], s_key[i]);
     }
 }
 
-// First pivot: every live vertex is in class 0, so each workgroup reduces
-// its maximum key first and issues one atomicMax.
 void k_elect(hipStream_t s, const DevGraph &g, DevState &st)
 {
-    elect_kernel<<<sweep_blocks(g.V), SWEEP_BLOCK, 0, s>>>(g.DP, st.cls,
-                                                           reinterpret_cast<unsigned long long *>(st.piv), g.V);
+    elect_kernel<<<tab_blocks(g.V), TAB_BLOCK, 0, s>>>(g.DP, st.cls,
+                                                       reinterpret_cast<unsigned long long *>(st.piv), g.V);
+}
+
+// Seeds of a round: one vertex per class, possibly millions (a colouring
+// round on an untrimmed power-law graph).  A wave owns 64-aligned chunks, so
+// a seed's visited bit is a plain store by the lane that owns its word, and
+// the seeds go through the wave's LDS queue, one reservation per SEED_WQ of
+// them: with an atomicAdd on the count per wave and an atomicOr per seed the
+// 2.4M roots of untrimmed R-MAT scale 22 took 760 us, bound by same-address
+// and device-wide atomics; now 34 us, bound by its class and colour streams.
+constexpr uint32_t SEED_WQ = 1024;
+constexpr uint32_t SEED_CHUNKS = 2;   // 64-vertex chunks per step
+
+// The chunk's seeds (mask m of its 64 vertices, v this lane's) join the
+// visited words of `vis`: lanes 0 and 32 own one word each.
+__device__ __forceinline__ void mark_seeds(uint32_t *vis, uint64_t m, uint32_t v)
+{
+    const uint32_t mw = lane() < 32 ? (uint32_t)m : (uint32_t)(m >> 32);
+    if ((lane() & 31) == 0 && mw) vis[vword(v)] |= mw;
 }
 
 // selectPivots (scc_kernels.cu:4-19): the winner of each class seeds the
-// FW (and BW) frontier.
-__global__ void select_kernel(const uint32_t *__restrict__ Fr, const uint32_t *__restrict__ Br,
-                              const uint32_t *__restrict__ cls, const uint64_t *__restrict__ piv,
-                              uint32_t *fvis, uint32_t *bvis, uint32_t *qf, uint32_t *qb,
-                              uint32_t *pivlist, uint32_t *ctr, uint32_t V, int seed_bw)
+// FW and BW frontiers.  The key's degree product is DP[v], as in the
+// election.
+__global__ __launch_bounds__(256) void select_kernel(const uint32_t *__restrict__ DP,
+                                                     const uint32_t *__restrict__ cls,
+                                                     const uint64_t *__restrict__ piv, uint32_t *fvis,
+                                                     uint32_t *bvis, uint32_t *qf, uint32_t *qb,
+                                                     uint32_t *pivlist, uint32_t *ctr, uint32_t V)
 {
-    WAVE_LOOP(v, valid, V)
-    {
-        if (!valid) continue;
-        const uint32_t c = cls[v];
-        if (c == DEAD || piv[c] != pivot_key(Fr, Br, v)) continue;
-        uint32_t i = atomicAdd(&ctr[CT(C_NPIV)], 1u);
+    __shared__ uint32_t s_q[4][SEED_WQ];
+    uint32_t *wq = s_q[threadIdx.x >> 6];
+    uint32_t nq = 0;
+    const uint32_t stride = gridDim.x * 256;
+    auto put = [=](uint32_t i, uint32_t v) {
         pivlist[i] = v;
         qf[i] = v;
-        atomicOr(&fvis[vword(v)], 1u << (v & 31));
-        if (seed_bw) {
-            qb[i] = v;
-            atomicOr(&bvis[vword(v)], 1u << (v & 31));
+        qb[i] = v;
+    };
+    for (uint32_t base = blockIdx.x * 256 + (threadIdx.x & ~63u); base <= V; base += SEED_CHUNKS * stride) {
+        if (nq + SEED_CHUNKS * 64 > SEED_WQ) wave_flush_each(wq, nq, &ctr[CT(C_NPIV)], put);
+        uint32_t v[SEED_CHUNKS], c[SEED_CHUNKS], dp[SEED_CHUNKS];
+        uint64_t best[SEED_CHUNKS];
+#pragma unroll
+        for (uint32_t h = 0; h < SEED_CHUNKS; h++) {
+            v[h] = base + h * stride + lane();
+            const uint32_t vv = v[h] <= V ? v[h] : 0u;   // vertex 0: the dummy, dead
+            c[h] = cls[vv];
+            dp[h] = DP[vv];
+        }
+#pragma unroll
+        for (uint32_t h = 0; h < SEED_CHUNKS; h++) best[h] = piv[c[h] != DEAD ? c[h] : 0u];
+#pragma unroll
+        for (uint32_t h = 0; h < SEED_CHUNKS; h++) {
+            const bool win = c[h] != DEAD && best[h] == (((uint64_t)dp[h] << 32) | (uint64_t)(0xFFFFFFFFu - v[h]));
+            const uint64_t m = __ballot(win);
+            if (!m) continue;
+            mark_seeds(fvis, m, v[h]);
+            mark_seeds(bvis, m, v[h]);
+            wave_push(wq, nq, win, v[h]);
         }
     }
+    wave_flush_block_each(wq, nq, &ctr[CT(C_NPIV)], put);
 }
 
 // Queue counts for level 0 and the two counters after it.
-__global__ void seed_counts_kernel(uint32_t *ctr, const uint32_t *pivlist, int seed_bw)
+__global__ void seed_counts_kernel(uint32_t *ctr, const uint32_t *seeds, int seed_bw)
 {
     uint32_t n = ctr[CT(C_NPIV)];
-    ctr[CT(C_PIV0)] = n ? pivlist[0] : 0u;
+    ctr[CT(C_PIV0)] = n ? seeds[0] : 0u;
     ctr[CT(C_FWCNT + 0)] = n;
     ctr[CT(C_FWCNT + 1)] = 0;
     ctr[CT(C_FWCNT + 2)] = 0;
@@ -835,12 +920,11 @@ __global__ void seed_counts_kernel(uint32_t *ctr, const uint32_t *pivlist, int s
     zero_hub_counts(ctr);
 }
 
-void k_select(hipStream_t s, const DevGraph &g, DevState &st, int seed_bw)
+void k_select(hipStream_t s, const DevGraph &g, DevState &st)
 {
-    select_kernel<<<sweep_blocks(g.V), SWEEP_BLOCK, 0, s>>>(g.Fr, g.Br, st.cls, st.piv, st.fvis,
-                                                            st.bvis, st.qf[0], st.qb[0],
-                                                            st.pivlist, st.ctr, g.V, seed_bw);
-    seed_counts_kernel<<<1, 1, 0, s>>>(st.ctr, st.pivlist, seed_bw);
+    select_kernel<<<sweep_blocks(g.V), SWEEP_BLOCK, 0, s>>>(g.DP, st.cls, st.piv, st.fvis, st.bvis, st.qf[0],
+                                                            st.qb[0], st.pivlist, st.ctr, g.V);
+    seed_counts_kernel<<<1, 1, 0, s>>>(st.ctr, st.pivlist, 1);
 }
 
 // A single source for the phase entry point: vertex src seeds direction dir.
@@ -1240,28 +1324,40 @@ void k_color_prop(hipStream_t s, const DevGraph &g, DevState &st)
 
 // selectPivotColoring (scc_kernels.cu:567-580): class = colour; a vertex
 // whose colour is its own id is a root and seeds the FW frontier.
-__global__ void color_roots_kernel(uint32_t *cls, const uint32_t *__restrict__ aux, uint32_t *fvis,
-                                   uint32_t *qf, uint32_t *pivlist, uint32_t *ctr, uint32_t V)
+__global__ __launch_bounds__(256) void color_roots_kernel(uint32_t *cls, const uint32_t *__restrict__ aux,
+                                                          uint32_t *fvis, uint32_t *qf, uint32_t *ctr, uint32_t V)
 {
-    WAVE_LOOP(v, valid, V)
-    {
-        if (!valid || cls[v] == DEAD) continue;
-        const uint32_t c = aux[v];
-        cls[v] = c;
-        if (c == v) {
-            uint32_t i = atomicAdd(&ctr[CT(C_NPIV)], 1u);
-            pivlist[i] = v;
-            qf[i] = v;
-            atomicOr(&fvis[vword(v)], 1u << (v & 31));
+    __shared__ uint32_t s_q[4][SEED_WQ];
+    uint32_t *wq = s_q[threadIdx.x >> 6];
+    uint32_t nq = 0;
+    const uint32_t stride = gridDim.x * 256;
+    for (uint32_t base = blockIdx.x * 256 + (threadIdx.x & ~63u); base <= V; base += SEED_CHUNKS * stride) {
+        if (nq + SEED_CHUNKS * 64 > SEED_WQ) wave_flush(wq, nq, &ctr[CT(C_NPIV)], qf);
+        uint32_t v[SEED_CHUNKS], c[SEED_CHUNKS], k[SEED_CHUNKS];
+#pragma unroll
+        for (uint32_t h = 0; h < SEED_CHUNKS; h++) {
+            v[h] = base + h * stride + lane();
+            const uint32_t vv = v[h] <= V ? v[h] : 0u;   // vertex 0: the dummy, dead
+            c[h] = cls[vv];
+            k[h] = aux[vv];
+        }
+#pragma unroll
+        for (uint32_t h = 0; h < SEED_CHUNKS; h++) {
+            if (c[h] != DEAD) cls[v[h]] = k[h];
+            const bool root = c[h] != DEAD && k[h] == v[h];
+            const uint64_t m = __ballot(root);
+            if (!m) continue;
+            mark_seeds(fvis, m, v[h]);
+            wave_push(wq, nq, root, v[h]);
         }
     }
+    wave_flush_block(wq, nq, &ctr[CT(C_NPIV)], qf);
 }
 
 void k_color_roots(hipStream_t s, const DevGraph &g, DevState &st)
 {
-    color_roots_kernel<<<sweep_blocks(g.V), SWEEP_BLOCK, 0, s>>>(st.cls, st.aux, st.fvis, st.qf[0],
-                                                                 st.pivlist, st.ctr, g.V);
-    seed_counts_kernel<<<1, 1, 0, s>>>(st.ctr, st.pivlist, 0);
+    color_roots_kernel<<<sweep_blocks(g.V), SWEEP_BLOCK, 0, s>>>(st.cls, st.aux, st.fvis, st.qf[0], st.ctr, g.V);
+    seed_counts_kernel<<<1, 1, 0, s>>>(st.ctr, st.qf[0], 0);
 }
 
 // fwdColoring marks each vertex it expands as finished (scc_kernels.cu:607):
@@ -1315,33 +1411,35 @@ __global__ void canon_reset_kernel(uint32_t *aux, uint32_t V, const uint32_t *ga
     for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v <= V; v += gridDim.x * blockDim.x) aux[v] = DEAD;
 }
 
-// Lanes of a wave that share a label are combined before touching memory:
-// up to MATCH_ROUNDS times the lowest pending lane leads and every lane with
-// its label joins; what is left (a wave with many distinct labels) goes
-// lane by lane.  A giant SCC's members then cost one atomic per wave
-// instead of one per vertex.
-constexpr int MATCH_ROUNDS = 8;
-
 // Each lane takes CANON_CHUNKS vertices per step, one per 64-vertex chunk
 // of its wave, with all their label loads in flight together (then, in the
 // apply pass, all their representative loads): one load per step leaves
 // these passes waiting on memory latency.
 constexpr uint32_t CANON_CHUNKS = 8;
 
-// Like the size counts below, each wave keeps a running minimum for one
-// label several of its lanes shared and writes it once at the end.
-__global__ __launch_bounds__(256) void canon_min_kernel(uint32_t *lab, uint32_t *aux, uint32_t *ctr, uint32_t V,
-                                                        const uint32_t *gate)
+// The smallest vertex of each label, through the workgroup's LDS table: a
+// label's minimum is set by the first few vertices of its members that the
+// workgroup meets, and every later member only reads its slot (lanes that
+// share a label combined by up to eight rounds of shuffles per wave before:
+// 8.4M vertices in 200 local SCCs 115 -> 28 us, untrimmed R-MAT scale 22
+// 74 -> 36 us).
+__global__ __launch_bounds__(TAB_BLOCK) void canon_min_kernel(uint32_t *lab, uint32_t *aux, uint32_t *ctr,
+                                                              uint32_t V, const uint32_t *gate)
 {
     if (gate_closed(gate)) return;
-    uint32_t heavy = DEAD, hmin = DEAD;
-    const uint32_t stride = gridDim.x * blockDim.x;
-    for (uint32_t base = blockIdx.x * blockDim.x + (threadIdx.x & ~63u); base < V; base += CANON_CHUNKS * stride) {
+    __shared__ uint32_t s_lab[TAB_SLOTS], s_min[TAB_SLOTS];
+    for (uint32_t i = threadIdx.x; i < TAB_SLOTS; i += TAB_BLOCK) {
+        s_lab[i] = TAB_FREE;
+        s_min[i] = DEAD;
+    }
+    __syncthreads();
+    const uint32_t stride = gridDim.x * TAB_BLOCK;
+    for (uint32_t base = blockIdx.x * TAB_BLOCK + (threadIdx.x & ~63u); base < V; base += CANON_CHUNKS * stride) {
         uint32_t vs[CANON_CHUNKS], rs[CANON_CHUNKS];
 #pragma unroll
         for (uint32_t h = 0; h < CANON_CHUNKS; h++) {
             vs[h] = base + h * stride + lane() + 1;
-            rs[h] = vs[h] <= V ? lab[vs[h]] : DEAD;
+            rs[h] = lab[vs[h] <= V ? vs[h] : 0u];
         }
 #pragma unroll
         for (uint32_t h = 0; h < CANON_CHUNKS; h++) {
@@ -1355,54 +1453,22 @@ __global__ __launch_bounds__(256) void canon_min_kernel(uint32_t *lab, uint32_t 
                 atomicAdd(&ctr[CT(C_ANOM)], 1u);
                 lab[v] = r = v | LAB_FINAL;
             }
-            bool pending = valid && !(r & LAB_FINAL);
-            for (int it = 0; it < MATCH_ROUNDS; it++) {
-                const uint64_t pm = __ballot(pending);
-                if (!pm) break;
-                const int L = __ffsll((unsigned long long)pm) - 1;
-                const uint32_t rl = __shfl(r, L);
-                const bool mine = pending && r == rl;
-                const uint64_t mm = __ballot(mine);
-                uint32_t m = mine ? v : DEAD;
-                for (int o = 32; o > 0; o >>= 1) {
-                    uint32_t x = __shfl_xor(m, o);
-                    m = x < m ? x : m;
-                }
-                if (rl == heavy) {
-                    hmin = m < hmin ? m : hmin;
-                } else if (heavy == DEAD && __popcll(mm) > 1) {
-                    heavy = rl;
-                    hmin = m;
-                } else if ((int)lane() == L && m < aux[rl]) {
-                    atomicMin(&aux[rl], m);
-                }
-                pending = pending && !mine;
+            if (!valid || (r & LAB_FINAL)) continue;
+            const uint32_t slot = tab_slot(s_lab, r);
+            if (slot < TAB_SLOTS) {
+                if (v < s_min[slot]) atomicMin(&s_min[slot], v);
+            } else if (v < aux[r]) {
+                atomicMin(&aux[r], v);
             }
-            if (pending && v < aux[r]) atomicMin(&aux[r], v);
         }
-    }
-    // The waves' running minima (every wave of a giant SCC's decomposition
-    // holds one for the same label) are combined per workgroup, and one
-    // lane adds it only if a coherent read shows it still lowers the value:
-    // a plain read sees a stale cached copy, and thousands of waves ending
-    // together with an atomic each on one address serialise.
-    __shared__ uint32_t s_heavy[4], s_hmin[4];
-    const uint32_t wv = threadIdx.x >> 6;
-    if (lane() == 0) {
-        s_heavy[wv] = heavy;
-        s_hmin[wv] = hmin;
     }
     __syncthreads();
-    if (lane() == 0 && heavy != DEAD) {
-        uint32_t m = hmin;
-        bool lead = true;   // the lowest wave holding this label adds for all of them
-        for (uint32_t w = 0; w < (blockDim.x >> 6); w++) {
-            if (w == wv || s_heavy[w] != heavy) continue;
-            if (w < wv) lead = false;
-            m = s_hmin[w] < m ? s_hmin[w] : m;
-        }
-        if (lead && m < __hip_atomic_load(&aux[heavy], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-            atomicMin(&aux[heavy], m);
+    // a coherent read first: a plain one may see a stale copy, and an atomic
+    // from every workgroup on a giant SCC's word serialises
+    for (uint32_t i = threadIdx.x; i < TAB_SLOTS; i += TAB_BLOCK) {
+        const uint32_t r = s_lab[i];
+        if (r != TAB_FREE && s_min[i] < __hip_atomic_load(&aux[r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+            atomicMin(&aux[r], s_min[i]);
     }
 }
 
@@ -1481,7 +1547,7 @@ void k_canon(hipStream_t s, const DevGraph &g, DevState &st, bool sizes, bool ga
     const uint32_t *gate = gated ? st.ctr : nullptr;
     const uint32_t b = sweep_blocks(g.V);
     canon_reset_kernel<<<b, SWEEP_BLOCK, 0, s>>>(st.aux, g.V, gate);
-    canon_min_kernel<<<b, SWEEP_BLOCK, 0, s>>>(st.lab, st.aux, st.ctr, g.V, gate);
+    canon_min_kernel<<<tab_blocks(g.V), TAB_BLOCK, 0, s>>>(st.lab, st.aux, st.ctr, g.V, gate);
     canon_apply_kernel<<<b, SWEEP_BLOCK, 0, s>>>(st.lab, st.aux, st.ctr, g.V, gate);
     if (sizes) k_sizes(s, g, st, gated);
 }
@@ -1490,8 +1556,9 @@ void k_canon(hipStream_t s, const DevGraph &g, DevState &st, bool sizes, bool ga
 // From canonical labels (lab[v] = the smallest vertex of v's SCC): cnt[r]
 // counts the members of r's SCC other than r itself, so a singleton (most
 // SCCs of a power-law graph: trim-1's) costs no atomic at all, and the
-// members of a large SCC are combined per wave (MATCH_ROUNDS leaders, then
-// one running count per wave for a recurring label) before touching memory.
+// members of a large SCC are counted in the workgroup's LDS table (one
+// running count per wave, added by 4,096 waves to one address, before: R-MAT
+// scale 20 49 -> 8 us, and 49 -> 9 us for the histogram's counts).
 // The size of the SCC of root r (lab[r] == r) is cnt[r] + 1.  cnt is the
 // class-word array, free once the labels are final.
 __global__ void size_reset_kernel(uint32_t *cnt, uint32_t V, const uint32_t *gate)
@@ -1500,104 +1567,114 @@ __global__ void size_reset_kernel(uint32_t *cnt, uint32_t V, const uint32_t *gat
     for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v <= V; v += gridDim.x * blockDim.x) cnt[v] = 0;
 }
 
-__global__ __launch_bounds__(256) void size_count_kernel(const uint32_t *__restrict__ lab, uint32_t *cnt,
-                                                         uint32_t V, const uint32_t *gate)
+// x added to id's value: the lanes that share the first pending lane's id
+// (a giant SCC's members, the singletons of the histogram) as one add, the
+// others lane by lane.  All 64 lanes of a wave call.
+__device__ __forceinline__ void tab_count(uint32_t *ids, uint32_t *vals, uint32_t *mem, bool pending, uint32_t id)
+{
+    const uint64_t pm = __ballot(pending);
+    if (!pm) return;
+    const int L = __ffsll((unsigned long long)pm) - 1;
+    const uint32_t first = __shfl(id, L);
+    const uint32_t n = (uint32_t)__popcll(__ballot(pending && id == first));
+    if (!pending || (id == first && (int)lane() != L)) return;
+    const uint32_t add = id == first ? n : 1u;
+    const uint32_t slot = tab_slot(ids, id);
+    if (slot < TAB_SLOTS) atomicAdd(&vals[slot], add);
+    else atomicAdd(&mem[id], add);
+}
+
+// The table's counts to memory, at the end (the whole workgroup calls).
+__device__ __forceinline__ void tab_add(const uint32_t *ids, const uint32_t *vals, uint32_t *mem)
+{
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < TAB_SLOTS; i += TAB_BLOCK)
+        if (ids[i] != TAB_FREE && vals[i]) atomicAdd(&mem[ids[i]], vals[i]);
+}
+
+__global__ __launch_bounds__(TAB_BLOCK) void size_count_kernel(const uint32_t *__restrict__ lab, uint32_t *cnt,
+                                                               uint32_t V, const uint32_t *gate)
 {
     if (gate_closed(gate)) return;
-    uint32_t heavy = DEAD, hcount = 0;
-    const uint32_t stride = gridDim.x * blockDim.x;
-    for (uint32_t base = blockIdx.x * blockDim.x + (threadIdx.x & ~63u); base < V; base += CANON_CHUNKS * stride) {
+    __shared__ uint32_t s_id[TAB_SLOTS], s_n[TAB_SLOTS];
+    for (uint32_t i = threadIdx.x; i < TAB_SLOTS; i += TAB_BLOCK) {
+        s_id[i] = TAB_FREE;
+        s_n[i] = 0;
+    }
+    __syncthreads();
+    const uint32_t stride = gridDim.x * TAB_BLOCK;
+    for (uint32_t base = blockIdx.x * TAB_BLOCK + (threadIdx.x & ~63u); base < V; base += CANON_CHUNKS * stride) {
         uint32_t vs[CANON_CHUNKS], rs[CANON_CHUNKS];
 #pragma unroll
         for (uint32_t h = 0; h < CANON_CHUNKS; h++) {
             vs[h] = base + h * stride + lane() + 1;
-            rs[h] = vs[h] <= V ? lab[vs[h]] : 0u;
+            rs[h] = lab[vs[h] <= V ? vs[h] : 0u];
         }
 #pragma unroll
-        for (uint32_t h = 0; h < CANON_CHUNKS; h++) {
-            const uint32_t r = rs[h];
-            bool pending = vs[h] <= V && r != vs[h] && r >= 1 && r <= V;
-            for (int it = 0; it < MATCH_ROUNDS; it++) {
-                const uint64_t pm = __ballot(pending);
-                if (!pm) break;
-                const int L = __ffsll((unsigned long long)pm) - 1;
-                const uint32_t rl = __shfl(r, L);
-                const uint32_t n = (uint32_t)__popcll(__ballot(pending && r == rl));
-                if (rl == heavy) {
-                    hcount += n;
-                } else if (heavy == DEAD && n > 1) {
-                    heavy = rl;
-                    hcount = n;
-                } else if ((int)lane() == L) {
-                    atomicAdd(&cnt[rl], n);
-                }
-                pending = pending && r != rl;
-            }
-            if (pending) atomicAdd(&cnt[r], 1u);
-        }
+        for (uint32_t h = 0; h < CANON_CHUNKS; h++)
+            tab_count(s_id, s_n, cnt, vs[h] <= V && rs[h] != vs[h] && rs[h] >= 1 && rs[h] <= V, rs[h]);
     }
-    if (hcount && lane() == 0) atomicAdd(&cnt[heavy], hcount);
+    tab_add(s_id, s_n, cnt);
 }
 
-// Largest SCC: the largest cnt[r] + 1 over roots r.
-__global__ void size_largest_kernel(const uint32_t *__restrict__ lab, const uint32_t *__restrict__ cnt,
-                                    uint32_t *ctr, uint32_t V, const uint32_t *gate)
+// Largest SCC: the largest cnt[r] + 1 over roots r, one atomic per workgroup
+// whose maximum beats a coherent read (an atomic per wave on the one address
+// took 49 us on R-MAT scale 20, all of it serialised; now 4 to 7 us).
+__global__ __launch_bounds__(TAB_BLOCK) void size_largest_kernel(const uint32_t *__restrict__ lab,
+                                                                 const uint32_t *__restrict__ cnt, uint32_t *ctr,
+                                                                 uint32_t V, const uint32_t *gate)
 {
     if (gate_closed(gate)) return;
+    __shared__ uint32_t s_max[TAB_BLOCK / 64];
     uint32_t m = 0;
-    for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x + 1; v <= V; v += gridDim.x * blockDim.x)
-        if (lab[v] == v) m = cnt[v] + 1 > m ? cnt[v] + 1 : m;
+    for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x + 1; v <= V; v += gridDim.x * blockDim.x) {
+        const uint32_t l = lab[v], c = cnt[v];
+        if (l == v) m = c + 1 > m ? c + 1 : m;
+    }
     for (int o = 32; o > 0; o >>= 1) {
         uint32_t x = __shfl_xor(m, o);
         m = x > m ? x : m;
     }
-    if (lane() == 0 && m) atomicMax(&ctr[CT(C_LARGEST)], m);
+    if (lane() == 0) s_max[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    for (uint32_t w = 1; w < TAB_BLOCK / 64; w++) m = s_max[w] > m ? s_max[w] : m;
+    if (m > __hip_atomic_load(&ctr[CT(C_LARGEST)], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMax(&ctr[CT(C_LARGEST)], m);
 }
 
 void k_sizes(hipStream_t s, const DevGraph &g, DevState &st, bool gated)
 {
     const uint32_t *gate = gated ? st.ctr : nullptr;
-    const uint32_t b = sweep_blocks(g.V);
-    size_reset_kernel<<<b, SWEEP_BLOCK, 0, s>>>(st.cls, g.V, gate);
-    size_count_kernel<<<b, SWEEP_BLOCK, 0, s>>>(st.lab, st.cls, g.V, gate);
-    size_largest_kernel<<<b, SWEEP_BLOCK, 0, s>>>(st.lab, st.cls, st.ctr, g.V, gate);
+    const uint32_t b = tab_blocks(g.V);
+    size_reset_kernel<<<sweep_blocks(g.V), SWEEP_BLOCK, 0, s>>>(st.cls, g.V, gate);
+    size_count_kernel<<<b, TAB_BLOCK, 0, s>>>(st.lab, st.cls, g.V, gate);
+    size_largest_kernel<<<b, TAB_BLOCK, 0, s>>>(st.lab, st.cls, st.ctr, g.V, gate);
 }
 
 // Size histogram from the sizes pass: hist[k] = number of SCCs of k
-// vertices (hist has V + 1 words, cleared here), combined per wave like
-// the counts (a power-law graph has millions of roots of size 1), then the
-// non-zero entries compacted into (size, count) pairs: `pairs` holds up to
-// `cap` of them (64-bit words, size then count), *npairs (a counter line)
-// the number found.  At most about sqrt(2V) sizes occur, so the list is
-// short; the host sorts it.
-__global__ __launch_bounds__(256) void hist_count_kernel(const uint32_t *__restrict__ lab,
-                                                         const uint32_t *__restrict__ cnt, uint32_t *hist,
-                                                         uint32_t V)
+// vertices (hist has V + 1 words, cleared here), counted in the workgroup's
+// LDS table like the sizes (a power-law graph has millions of roots of size
+// 1), then the non-zero entries compacted into (size, count) pairs: `pairs`
+// holds up to `cap` of them (64-bit words, size then count), *npairs (a
+// counter line) the number found.  At most about sqrt(2V) sizes occur, so
+// the list is short; the host sorts it.
+__global__ __launch_bounds__(TAB_BLOCK) void hist_count_kernel(const uint32_t *__restrict__ lab,
+                                                               const uint32_t *__restrict__ cnt, uint32_t *hist,
+                                                               uint32_t V)
 {
-    uint32_t heavy = 0, hcount = 0;
-    for (uint32_t v0 = blockIdx.x * blockDim.x + (threadIdx.x & ~63u); v0 < V; v0 += gridDim.x * blockDim.x) {
-        const uint32_t v = v0 + lane() + 1;
-        const uint32_t k = (v <= V && lab[v] == v) ? cnt[v] + 1 : 0u;
-        bool pending = k != 0;
-        for (int it = 0; it < MATCH_ROUNDS; it++) {
-            const uint64_t pm = __ballot(pending);
-            if (!pm) break;
-            const int L = __ffsll((unsigned long long)pm) - 1;
-            const uint32_t kl = __shfl(k, L);
-            const uint32_t n = (uint32_t)__popcll(__ballot(pending && k == kl));
-            if (kl == heavy) {
-                hcount += n;
-            } else if (heavy == 0 && n > 1) {
-                heavy = kl;
-                hcount = n;
-            } else if ((int)lane() == L) {
-                atomicAdd(&hist[kl], n);
-            }
-            pending = pending && k != kl;
-        }
-        if (pending) atomicAdd(&hist[k], 1u);
+    __shared__ uint32_t s_id[TAB_SLOTS], s_n[TAB_SLOTS];
+    for (uint32_t i = threadIdx.x; i < TAB_SLOTS; i += TAB_BLOCK) {
+        s_id[i] = TAB_FREE;
+        s_n[i] = 0;
     }
-    if (hcount && lane() == 0) atomicAdd(&hist[heavy], hcount);
+    __syncthreads();
+    for (uint32_t v0 = blockIdx.x * TAB_BLOCK + (threadIdx.x & ~63u); v0 < V; v0 += gridDim.x * TAB_BLOCK) {
+        const uint32_t v = v0 + lane() + 1, vv = v <= V ? v : 0u;
+        const uint32_t l = lab[vv], c = cnt[vv];
+        tab_count(s_id, s_n, hist, v <= V && l == v, c + 1);
+    }
+    tab_add(s_id, s_n, hist);
 }
 
 __global__ void hist_compact_kernel(const uint32_t *__restrict__ hist, uint64_t *pairs, uint32_t cap,
@@ -1625,7 +1702,7 @@ void k_size_histogram(hipStream_t s, const DevGraph &g, DevState &st, uint32_t *
 {
     const uint32_t b = sweep_blocks(g.V);
     size_reset_kernel<<<b, SWEEP_BLOCK, 0, s>>>(hist, g.V, nullptr);
-    hist_count_kernel<<<b, SWEEP_BLOCK, 0, s>>>(st.lab, st.cls, hist, g.V);
+    hist_count_kernel<<<tab_blocks(g.V), TAB_BLOCK, 0, s>>>(st.lab, st.cls, hist, g.V);
     hist_compact_kernel<<<b, SWEEP_BLOCK, 0, s>>>(hist, pairs, cap, npairs, g.V);
 }
 

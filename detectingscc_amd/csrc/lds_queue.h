@@ -71,11 +71,10 @@ __device__ __forceinline__ void wave_push(uint32_t *wq, uint32_t &nq, bool p, ui
     nq += (uint32_t)__popcll(m);
 }
 
-// Entries at or past `cap` are not written, and a reservation that passes
-// it counts one in *anom (a caller whose bound says that cannot happen
-// passes its region's size; the region's reader clamps its count to cap).
-__device__ __forceinline__ void wave_flush(uint32_t *wq, uint32_t &nq, uint32_t *gcnt, uint32_t *gout,
-                                           uint32_t cap = ~0u, uint32_t *anom = nullptr)
+// One reservation of nq entries, then store(index, entry) for each of them.
+template <class Store>
+__device__ __forceinline__ void wave_flush_each(uint32_t *wq, uint32_t &nq, uint32_t *gcnt, Store store,
+                                                uint32_t cap = ~0u, uint32_t *anom = nullptr)
 {
     if (!nq) return;
     const uint32_t lane = threadIdx.x & 63u;
@@ -87,15 +86,25 @@ __device__ __forceinline__ void wave_flush(uint32_t *wq, uint32_t &nq, uint32_t 
     }
     b = __shfl(b, 0);
     for (uint32_t i = lane; i < nq; i += 64)
-        if (b + i < cap) gout[b + i] = wq[i];
+        if (b + i < cap) store(b + i, wq[i]);
     nq = 0;
     wave_sync();
 }
 
+// Entries at or past `cap` are not written, and a reservation that passes
+// it counts one in *anom (a caller whose bound says that cannot happen
+// passes its region's size; the region's reader clamps its count to cap).
+__device__ __forceinline__ void wave_flush(uint32_t *wq, uint32_t &nq, uint32_t *gcnt, uint32_t *gout,
+                                           uint32_t cap = ~0u, uint32_t *anom = nullptr)
+{
+    wave_flush_each(wq, nq, gcnt, [gout](uint32_t i, uint32_t v) { gout[i] = v; }, cap, anom);
+}
+
 // End of kernel: the four waves' remainders with one atomic (every thread
 // of the 256-lane workgroup calls).  cap and anom as for wave_flush.
-__device__ __forceinline__ void wave_flush_block(const uint32_t *wq, uint32_t nq, uint32_t *gcnt, uint32_t *gout,
-                                                 uint32_t cap = ~0u, uint32_t *anom = nullptr)
+template <class Store>
+__device__ __forceinline__ void wave_flush_block_each(const uint32_t *wq, uint32_t nq, uint32_t *gcnt, Store store,
+                                                      uint32_t cap = ~0u, uint32_t *anom = nullptr)
 {
     __shared__ uint32_t s_n[4], s_base;
     const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
@@ -110,7 +119,13 @@ __device__ __forceinline__ void wave_flush_block(const uint32_t *wq, uint32_t nq
     uint32_t off = s_base;
     for (uint32_t w = 0; w < wv; w++) off += s_n[w];
     for (uint32_t i = lane; i < nq; i += 64)
-        if (off + i < cap) gout[off + i] = wq[i];
+        if (off + i < cap) store(off + i, wq[i]);
+}
+
+__device__ __forceinline__ void wave_flush_block(const uint32_t *wq, uint32_t nq, uint32_t *gcnt, uint32_t *gout,
+                                                 uint32_t cap = ~0u, uint32_t *anom = nullptr)
+{
+    wave_flush_block_each(wq, nq, gcnt, [gout](uint32_t i, uint32_t v) { gout[i] = v; }, cap, anom);
 }
 
 } // namespace sccamd

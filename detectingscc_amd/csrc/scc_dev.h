@@ -79,18 +79,21 @@ enum : int {
 // after the C_COUNT counter lines: workgroup b uses slot b % kSpread.  Its
 // value is its own word plus its slots (the counter publication folds them
 // for the host).  The spread counters are C_CHANGED..C_NSCC, the trim-1
-// list counts C_TLIST..C_TLIST+2 and the search queue counts
+// list counts C_TLIST..C_TLIST+2, the search queue counts
 // C_FWCNT..C_BWCNT+2 (the slots of each direction's three counts are
-// consecutive: count k's slot j is CSLOT(first, k * kSpread + j)).
+// consecutive: count k's slot j is CSLOT(first, k * kSpread + j)) and the
+// work units C_WORK..C_WORK+7 (64-bit: words 0 and 1 of each line).
 constexpr int kSpread = 32;
 __host__ __device__ constexpr int spread_index(int c)
 {
     return (c >= C_CHANGED && c <= C_NSCC) ? c - C_CHANGED
            : (c >= C_TLIST && c < C_TLIST + 3) ? C_NSCC - C_CHANGED + 1 + (c - C_TLIST)
            : (c >= C_FWCNT && c < C_BWCNT + 3) ? C_NSCC - C_CHANGED + 4 + (c - C_FWCNT)
+           : (c >= C_WORK && c < C_WORK + 8)   ? C_NSCC - C_CHANGED + 10 + (c - C_WORK)
                                                 : -1;
 }
-constexpr int kSpreadCounters = C_NSCC - C_CHANGED + 1 + 3 + 6;
+constexpr int kSpreadCounters = C_NSCC - C_CHANGED + 1 + 3 + 6 + 8;
+__host__ __device__ constexpr bool wide_counter(int c) { return c >= C_WORK && c < C_WORK + 8; }   // 64-bit slots
 constexpr int kCtrLines = C_COUNT + kSpreadCounters * kSpread;   // lines of the counters block
 // word of slot j of spread counter c
 __host__ __device__ constexpr int CSLOT(int c, int j) { return CT(C_COUNT + spread_index(c) * kSpread + j); }
@@ -372,7 +375,7 @@ void k_init_vis(hipStream_t s, const DevGraph &g, DevState &st, bool elect_first
                 const uint32_t *live_bits = nullptr);
 // single_class: every live vertex is in class 0 (the first pivot)
 void k_elect(hipStream_t s, const DevGraph &g, DevState &st);
-void k_select(hipStream_t s, const DevGraph &g, DevState &st, int seed_bw);
+void k_select(hipStream_t s, const DevGraph &g, DevState &st);
 // scc_min: a round with one pivot (C_PIV0) also leaves its SCC's smallest
 // vertex in aux[pivot]
 // live_bits as for k_init_vis; lazy (a first round after a label-less
