@@ -14,7 +14,7 @@ struct BatchDev {
     uint32_t *cls = nullptr, *lab = nullptr, *aux = nullptr;
     uint32_t *fvis = nullptr, *bvis = nullptr;        // bit voff[i]+v
     uint64_t *piv = nullptr;                           // 3*voff[i] + class
-    uint32_t *q = nullptr;                             // 4*voff[i]: FW in/out, BW in/out
+    uint32_t *q = nullptr;                             // 4*voff[i]: four arrays of V+2 words (G1::q)
     uint32_t *pivlist = nullptr;                       // voff[i]
     const uint32_t *cfg = nullptr;                     // per graph
     const uint32_t *order = nullptr;                   // processing order (indices)
@@ -27,7 +27,7 @@ struct BatchDev {
 constexpr uint32_t BATCH_ANOMALY = 0xFFFFFFFFu;
 
 // cfg word of one graph
-uint32_t batch_cfg(int lanes, bool trim1, bool trim2, bool slota);
+uint32_t batch_cfg(bool trim1, bool trim2, bool slota);
 
 // Persistent launch over order[first .. first+count) with `block` lanes per
 // workgroup (256, 512 or 1024) and `grid` workgroups; *B.next must be 0.

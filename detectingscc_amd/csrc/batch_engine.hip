@@ -256,7 +256,11 @@ scc_status BatchEngine::launch(const std::vector<uint32_t> &idx, const std::vect
                                uint32_t *launches)
 {
     BHIP(hipSetDevice(dev));
-    // group by block size, each group ordered by size (largest first)
+    // group by block size, each group ordered by expected time, longest
+    // first.  The time of a graph follows its vertices more than its arcs
+    // (bottom-up levels stop at a vertex's first visited parent, and sparse
+    // graphs take more levels and trim passes): 63,665 vertices with 131,651
+    // arcs take as long as 61,414 with 930,397
     std::vector<uint32_t> order;
     std::vector<std::pair<int, std::pair<uint32_t, uint32_t>>> groups;   // block, (first, count)
     for (int bs : {1024, 512, 256}) {
@@ -265,7 +269,7 @@ scc_status BatchEngine::launch(const std::vector<uint32_t> &idx, const std::vect
             if (block[k] == bs) mine.push_back(idx[k]);
         if (mine.empty()) continue;
         std::stable_sort(mine.begin(), mine.end(), [&](uint32_t a, uint32_t c) {
-            return (uint64_t)V[a] + E[a] > (uint64_t)V[c] + E[c];
+            return 16 * (uint64_t)V[a] + E[a] > 16 * (uint64_t)V[c] + E[c];
         });
         groups.push_back({bs, {(uint32_t)order.size(), (uint32_t)mine.size()}});
         order.insert(order.end(), mine.begin(), mine.end());
@@ -350,7 +354,7 @@ scc_status BatchEngine::run(const scc_batch_opts &o, scc_batch_stats *out)
             cfg[i] = best_cfg[bucket[i]];
             blk[i] = best_block[bucket[i]];
         } else {
-            cfg[i] = batch_cfg(o.lanes, o.trim1, o.trim2, o.algo == 'h');
+            cfg[i] = batch_cfg(o.trim1, o.trim2, o.algo == 'h');
             blk[i] = o.block;
         }
     }
@@ -415,7 +419,7 @@ scc_status BatchEngine::run_serial(Engine &eng, const scc_opts &o, scc_batch_sta
     return SCC_OK;
 }
 
-// Candidates per bucket: lanes x workgroup size x strategy.  Each candidate
+// Candidates per bucket: workgroup size x strategy.  Each candidate
 // runs up to `sample` graphs of the bucket in one persistent launch, so the
 // graphs share the chip as they do in a full batch; cost = elapsed time of
 // that launch (best of two).  A bucket with many graphs is then costed by
@@ -425,18 +429,17 @@ scc_status BatchEngine::autotune(int sample, std::string *report)
     if (!G) return fail(SCC_ERR_NOTREADY, "no batch uploaded");
     if (sample < 1) sample = 1;
     struct Cand {
-        int lanes, block;
+        int block;
         bool t1, t2, slota;
         const char *name;
     };
     std::vector<Cand> cands;
-    for (int lanes : {4, 16, 64})
-        for (int blk : {256, 512, 1024}) {
-            cands.push_back({lanes, blk, true, true, false, "hong+trim1+trim2"});
-            cands.push_back({lanes, blk, true, false, false, "hong+trim1"});
-            cands.push_back({lanes, blk, true, false, true, "slota+trim1"});
-        }
-    best_cfg.assign(NBUCKETS, batch_cfg(16, true, false, true));
+    for (int blk : {256, 512, 1024}) {
+        cands.push_back({blk, true, true, false, "hong+trim1+trim2"});
+        cands.push_back({blk, true, false, false, "hong+trim1"});
+        cands.push_back({blk, true, false, true, "slota+trim1"});
+    }
+    best_cfg.assign(NBUCKETS, batch_cfg(true, false, true));
     best_block.assign(NBUCKETS, 1024);
     char line[256];
     for (int bk = 0; bk < NBUCKETS; bk++) {
@@ -448,7 +451,7 @@ scc_status BatchEngine::autotune(int sample, std::string *report)
         int bi = 0;
         for (size_t c = 0; c < cands.size(); c++) {
             const Cand &cd = cands[c];
-            std::vector<uint32_t> cfg(members.size(), batch_cfg(cd.lanes, cd.t1, cd.t2, cd.slota));
+            std::vector<uint32_t> cfg(members.size(), batch_cfg(cd.t1, cd.t2, cd.slota));
             std::vector<int> blk(members.size(), cd.block);
             double cost = 1e300;
             for (int rep = 0; rep < 2; rep++) {
@@ -462,14 +465,13 @@ scc_status BatchEngine::autotune(int sample, std::string *report)
                 bi = (int)c;
             }
         }
-        best_cfg[bk] = batch_cfg(cands[bi].lanes, cands[bi].t1, cands[bi].t2, cands[bi].slota);
+        best_cfg[bk] = batch_cfg(cands[bi].t1, cands[bi].t2, cands[bi].slota);
         best_block[bk] = cands[bi].block;
         if (report) {
             static const char *sz[] = {"2^8-2^10", "2^10-2^12", "2^12-2^14", ">=2^14"};
             static const char *dg[] = {"deg<6", "deg 6-11", "deg>=11"};
-            snprintf(line, sizeof line, "bucket V %s %s (%zu graphs): lanes %d, block %d, %s, %.3f ms\n",
-                     sz[bk / 3], dg[bk % 3], members.size(), cands[bi].lanes, cands[bi].block,
-                     cands[bi].name, best);
+            snprintf(line, sizeof line, "bucket V %s %s (%zu graphs): block %d, %s, %.3f ms\n",
+                     sz[bk / 3], dg[bk % 3], members.size(), cands[bi].block, cands[bi].name, best);
             *report += line;
         }
     }

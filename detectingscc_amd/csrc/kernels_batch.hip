@@ -8,11 +8,25 @@
 // to the host until the batch is done.
 //
 // Phase orders are the reference's: vHong (scc_WCC.cu:573-998) and vSlota
-// (scc_Coloring.cu:403-701); the kernels inside each phase mirror the
-// single-graph engine (kernels_sweep.hip, kernels_reach.hip) at workgroup
-// scope.  Per graph the configuration word selects the algorithm, the trims
-// and the lanes per frontier vertex (chosen by the autotuner per size and
-// degree bucket).
+// (scc_Coloring.cu:403-701).  The first round (trim-1, the first pivot's FW
+// and BW search) has one class only and runs on bitmaps; a graph that it
+// finishes gets its labels from them.  Otherwise the vertices it left are
+// listed, and the later phases run over that list.  Per graph the
+// configuration word selects the algorithm and the trims (with the workgroup
+// size chosen by the autotuner per size and degree bucket).
+//
+// What bounds it: one graph's chain of dependent loads (a workgroup waits
+// for some hundreds of them one after another) and, for the large graphs of
+// a batch, HBM (6.5 GB for the 4.4 GB of the 4,096-graph mix).  Hence:
+// several chunks' loads in flight per lane (four 64-vertex chunks and all
+// their list walks side by side: 2.45 -> 1.95 ms on the mix, although its
+// registers leave one 1,024-lane workgroup per CU instead of two), the two
+// directions of a search on two halves of the waves, a frontier's arcs
+// balanced over its wave, hubs over the workgroup, bottom-up levels where
+// the degree pays for them, no gather of first neighbours where trim-1 would
+// remove little, and nothing run for vertices that are finished.  The mix
+// (47.6M vertices, 434M arcs, 1,024 lanes) 11.1 -> 1.9 ms; 700 graphs of 2^8
+// to 2^12 vertices with 256 lanes 1.31 -> 0.19 ms.
 //
 // Layout: graph i's per-vertex arrays start at slot voff[i] (a multiple of
 // 64, so bitmap words never straddle two graphs) and span V_i+2 slots; its
@@ -22,67 +36,123 @@
 
 namespace sccamd {
 
-// cfg word: bits 0-2 log2(lanes per frontier vertex), bit 3 trim-1, bit 4
-// trim-2, bit 5 Slota (colouring) instead of Hong
-__host__ __device__ inline uint32_t cfg_lanes(uint32_t c) { return 1u << (c & 7u); }
-__host__ __device__ inline bool cfg_t1(uint32_t c) { return (c >> 3) & 1u; }
-__host__ __device__ inline bool cfg_t2(uint32_t c) { return (c >> 4) & 1u; }
-__host__ __device__ inline bool cfg_slota(uint32_t c) { return (c >> 5) & 1u; }
+// cfg word: bit 0 trim-1, bit 1 trim-2, bit 2 Slota (colouring) instead of Hong
+__host__ __device__ inline bool cfg_t1(uint32_t c) { return c & 1u; }
+__host__ __device__ inline bool cfg_t2(uint32_t c) { return (c >> 1) & 1u; }
+__host__ __device__ inline bool cfg_slota(uint32_t c) { return (c >> 2) & 1u; }
 
 namespace {
 
 __device__ __forceinline__ uint32_t ln() { return threadIdx.x & 63u; }
 
-__device__ __forceinline__ uint64_t bkey(const uint32_t *Fr, const uint32_t *Br, uint32_t v)
+// A value every lane holds alike (read from LDS, say), as a scalar: the
+// views' pointers and the loop bounds then live in scalar registers.
+__device__ __forceinline__ uint32_t uni(uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); }
+
+__device__ __forceinline__ uint64_t bkey_deg(uint32_t outdeg, uint32_t indeg, uint32_t v)
 {
-    uint64_t p = (uint64_t)(Fr[v + 1] - Fr[v]) * (uint64_t)(Br[v + 1] - Br[v]);
+    uint64_t p = (uint64_t)outdeg * (uint64_t)indeg;
     p = p > 0xFFFFFFFFull ? 0xFFFFFFFFull : p;
     return (p << 32) | (uint64_t)(0xFFFFFFFFu - v);
+}
+
+__device__ __forceinline__ uint64_t bkey(const uint32_t *Fr, const uint32_t *Br, uint32_t v)
+{
+    return bkey_deg(Fr[v + 1] - Fr[v], Br[v + 1] - Br[v], v);
 }
 
 __device__ __forceinline__ uint32_t bkey_vertex(uint64_t k) { return 0xFFFFFFFFu - (uint32_t)k; }
 
 __device__ __forceinline__ bool bbit(const uint32_t *bm, uint32_t v) { return (bm[v >> 5] >> (v & 31)) & 1u; }
 
+// A frontier vertex of at least HUB_DEG arcs is walked by the whole
+// workgroup (one lane group alone would walk the pivot of a power-law graph
+// for hundreds of steps); up to HUB_CAP of them per level.
+constexpr uint32_t HUB_DEG = 512;
+constexpr uint32_t HUB_CAP = 128;
+
 // per-workgroup scratch in LDS
 struct Lds {
     uint32_t graph;
-    uint32_t flag;
-    uint32_t cnt[4];          // queue counts: FW in, FW out, BW in, BW out
+    uint32_t tail[2];         // entries in the FW and BW queues
     uint32_t npiv;
-    uint32_t live;
+    uint32_t nact;            // listed vertices
+    uint32_t nhub;
     uint32_t anom;            // a class without a recorded pivot was seen
-    uint32_t red[16];
+    uint32_t red[2][16];
     unsigned long long key;
+    uint32_t hub[HUB_CAP];    // vertex | direction << 31
 };
 
 // one graph's views
 struct G1 {
     uint32_t V;
+    uint32_t E;
     const uint32_t *Fr, *Fc, *Br, *Bc;
     uint32_t *cls, *lab, *aux;
-    uint32_t *fvis, *bvis;
+    uint32_t *live, *fvis, *bvis;   // one bit per vertex
     uint64_t *piv;
-    uint32_t *q;          // four queues of V+2 entries: FW in/out, BW in/out
-    // queue k (0..3) by arithmetic: a runtime index into a pointer array
-    // would put the whole struct in scratch memory
+    // four arrays of V+2 words: 0 and 2 are the FW and BW queues (each
+    // vertex enters a search's queue once, so a queue is never reused within
+    // a search), 1 holds the first out-neighbours and then the list of the
+    // vertices the first round left, 3 the live bitmap of a graph too large
+    // for LDS
+    uint32_t *q;
     __device__ __forceinline__ uint32_t *queue(uint32_t k) const { return q + (size_t)k * (V + 2); }
+    __device__ __forceinline__ uint32_t *f1() const { return queue(1); }
+    __device__ __forceinline__ uint32_t *b1() const { return aux; }   // first in-neighbours (first round only)
+    __device__ __forceinline__ uint32_t *list() const { return queue(1); }
     uint32_t *pivlist;
 };
 
-template <int BS> __device__ __forceinline__ uint32_t wg_sum(Lds &L, uint32_t x)
+// Workgroup sum; L.red is double-buffered by `k`, so consecutive sums with
+// alternating k need one barrier each.
+template <int BS> __device__ __forceinline__ uint32_t wg_sum(Lds &L, uint32_t x, uint32_t k)
 {
     for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
-    __syncthreads();
-    if (ln() == 0) L.red[threadIdx.x >> 6] = x;
+    if (ln() == 0) L.red[k][threadIdx.x >> 6] = x;
     __syncthreads();
     uint32_t t = 0;
-    for (int w = 0; w < BS / 64; w++) t += L.red[w];
+    for (int w = 0; w < BS / 64; w++) t += L.red[k][w];
+    return uni(t);
+}
+
+template <int BS> __device__ __forceinline__ uint32_t wg_sum1(Lds &L, uint32_t x)
+{
+    __syncthreads();
+    const uint32_t t = wg_sum<BS>(L, x, 0);
     __syncthreads();
     return t;
 }
 
-// LDS-counter push (wave-aggregated)
+template <int BS> __device__ __forceinline__ uint32_t wg_min1(Lds &L, uint32_t x)
+{
+    for (int o = 32; o > 0; o >>= 1) {
+        const uint32_t y = __shfl_xor(x, o);
+        x = y < x ? y : x;
+    }
+    __syncthreads();
+    if (ln() == 0) L.red[0][threadIdx.x >> 6] = x;
+    __syncthreads();
+    uint32_t t = DEAD;
+    for (int w = 0; w < BS / 64; w++) t = L.red[0][w] < t ? L.red[0][w] : t;
+    __syncthreads();
+    return uni(t);
+}
+
+// a[i] for a per-vertex array (i < 2^30, so the byte offset fits 32 bits and
+// the address is a scalar base and one vector register)
+__device__ __forceinline__ uint32_t at(const uint32_t *a, uint32_t i)
+{
+    return *reinterpret_cast<const uint32_t *>(reinterpret_cast<const char *>(a) + (uint32_t)(i << 2));
+}
+
+__device__ __forceinline__ void put(uint32_t *a, uint32_t i, uint32_t x)
+{
+    *reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(a) + (uint32_t)(i << 2)) = x;
+}
+
+// LDS-counter push (wave-aggregated over the active lanes)
 __device__ __forceinline__ void lpush(bool p, uint32_t v, uint32_t *q, uint32_t *cnt)
 {
     const uint64_t act = __ballot(1);
@@ -92,26 +162,75 @@ __device__ __forceinline__ void lpush(bool p, uint32_t v, uint32_t *q, uint32_t 
     uint32_t b = 0;
     if ((int)ln() == leader) b = atomicAdd(cnt, (uint32_t)__popcll(m));
     b = __shfl(b, leader);
-    if (p) q[b + (uint32_t)__popcll(m & ((1ull << ln()) - 1))] = v;
-}
-
-template <int BS> __device__ void g_init_vis(const G1 &g)
-{
-    const uint32_t nch = (g.V + 64) / 64;
-    for (uint32_t ch = threadIdx.x >> 6; ch < nch; ch += BS / 64) {
-        const uint32_t v = ch * 64 + ln();
-        const bool dead = v > g.V || g.cls[v] == DEAD;
-        const uint64_t m = __ballot(dead);
-        if (ln() < 2) g.fvis[2 * ch + ln()] = ln() ? (uint32_t)(m >> 32) : (uint32_t)m;
-        else if (ln() < 4) g.bvis[2 * ch + (ln() & 1)] = (ln() & 1) ? (uint32_t)(m >> 32) : (uint32_t)m;
-    }
+    if (p) put(q, b + (uint32_t)__popcll(m & ((1ull << ln()) - 1)), v);
 }
 
 // Per-vertex list walks: a step loads GK columns and then issues every
 // probe of the step before using any (indexes past the end repeat the last
 // arc, which changes no minimum, maximum or existence test).  A walk of
 // one arc per step waits for two dependent loads per arc.
-constexpr uint32_t GK = 4;
+constexpr uint32_t GK = 2;
+
+// For each of a lane's K lists, a vertex of C[k][i[k]..e[k]) whose bit is set
+// in bm, 0 if none (i == e: nothing to look up; all 64 lanes of the wave
+// call).  The lane's lists are walked side by side, GK arcs of each in
+// flight, for ROW_LANE arcs; what is left of longer lists the wave walks
+// together, one list after the other: a lane alone took milliseconds for a
+// power-law graph's hub whose neighbours are nearly all unset, and its graph
+// finished last by as much.
+constexpr uint32_t ROW_LANE = 32;
+
+template <uint32_t K>
+__device__ __forceinline__ void g_any_bit(const uint32_t *const (&C)[K], uint32_t (&i)[K], const uint32_t (&e)[K],
+                                          const uint32_t *bm, uint32_t (&hit)[K])
+{
+    uint32_t own[K];
+    bool any = false;
+#pragma unroll
+    for (uint32_t k = 0; k < K; k++) {
+        hit[k] = 0;
+        own[k] = min(e[k], i[k] + ROW_LANE);
+        any |= i[k] < e[k];
+    }
+    while (any) {
+        uint32_t w[K][GK];
+#pragma unroll
+        for (uint32_t k = 0; k < K; k++) {
+#pragma unroll
+            for (uint32_t n = 0; n < GK; n++) w[k][n] = 0;   // the dummy: never set
+            if (!hit[k] && i[k] < own[k]) {
+#pragma unroll
+                for (uint32_t n = 0; n < GK; n++) w[k][n] = C[k][min(i[k] + n, e[k] - 1)];
+            }
+        }
+        any = false;
+#pragma unroll
+        for (uint32_t k = 0; k < K; k++) {
+#pragma unroll
+            for (uint32_t n = 0; n < GK; n++)
+                if (!hit[k] && bbit(bm, w[k][n])) hit[k] = w[k][n];
+            i[k] = hit[k] ? own[k] : min(i[k] + GK, own[k]);
+            any |= i[k] < own[k];
+        }
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < K; k++) {
+        uint64_t todo = __ballot(!hit[k] && i[k] < e[k]);
+        while (todo) {
+            const int l = __ffsll((unsigned long long)todo) - 1;
+            todo &= todo - 1;
+            const uint32_t end = (uint32_t)__builtin_amdgcn_readlane((int)e[k], l);
+            uint32_t found = 0;
+            for (uint32_t j = (uint32_t)__builtin_amdgcn_readlane((int)i[k], l); !found && j < end; j += 128) {
+                const uint32_t w0 = C[k][min(j + ln(), end - 1)], w1 = C[k][min(j + 64 + ln(), end - 1)];
+                const uint32_t w = bbit(bm, w0) ? w0 : bbit(bm, w1) ? w1 : 0u;
+                const uint64_t m = __ballot(w != 0);
+                if (m) found = (uint32_t)__builtin_amdgcn_readlane((int)w, __ffsll((unsigned long long)m) - 1);
+            }
+            if ((int)ln() == l) hit[k] = found;
+        }
+    }
+}
 
 // whether some arc of col[i..e) leads to a vertex of class c
 __device__ __forceinline__ bool g_any_cls(const uint32_t *C, uint32_t i, uint32_t e, const uint32_t *cls,
@@ -145,39 +264,411 @@ __device__ __forceinline__ uint32_t g_fold(const uint32_t *C, uint32_t i, uint32
     return m;
 }
 
-// trim-1 (scc_kernels.cu:187-233) to its fixpoint or one pass
-template <int BS> __device__ uint32_t g_trim1(Lds &L, const G1 &g, bool fixpoint)
+// ------------------------------------------------- the first round ---
+// A wave owns the 64-vertex chunks w, w + BS/64, ... and with them the two
+// words of each bitmap, which it writes with plain stores.
+
+// Degrees: the live bitmap (vertices with an in- and an out-arc; all of them
+// with the trims off) and the best pivot key among them, which goes to
+// L.key.  Returns the number of vertices that are not live.
+constexpr uint32_t DEG_CHUNKS = 4;
+
+template <int BS> __device__ __forceinline__ uint32_t g_degrees(Lds &L, const G1 &g, bool trim)
 {
-    uint32_t total = 0;
+    const uint32_t nch = (g.V + 64) / 64;
+    unsigned long long best = 0;
+    uint32_t gone = 0;
+    for (uint32_t c0 = uni(threadIdx.x >> 6); c0 < nch; c0 += DEG_CHUNKS * (BS / 64)) {
+        uint32_t fb[DEG_CHUNKS], fe[DEG_CHUNKS], bb[DEG_CHUNKS], be[DEG_CHUNKS];
+#pragma unroll
+        for (uint32_t h = 0; h < DEG_CHUNKS; h++) {
+            const uint32_t v = (c0 + h * (BS / 64)) * 64 + ln(), vv = v <= g.V ? v : 0u;   // row 0 is empty
+            fb[h] = at(g.Fr, vv);
+            fe[h] = at(g.Fr, vv + 1);
+            bb[h] = at(g.Br, vv);
+            be[h] = at(g.Br, vv + 1);
+        }
+#pragma unroll
+        for (uint32_t h = 0; h < DEG_CHUNKS; h++) {
+            const uint32_t ch = c0 + h * (BS / 64), v = ch * 64 + ln();
+            const bool in = v >= 1 && v <= g.V;
+            const bool alive = in && (!trim || (fe[h] > fb[h] && be[h] > bb[h]));
+            gone += in && !alive;
+            const uint64_t m = __ballot(alive);
+            if (ch < nch && ln() < 2) g.live[2 * ch + ln()] = ln() ? (uint32_t)(m >> 32) : (uint32_t)m;
+            if (alive) {
+                const unsigned long long k = bkey_deg(fe[h] - fb[h], be[h] - bb[h], v);
+                best = k > best ? k : best;
+            }
+        }
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        const unsigned long long x = __shfl_xor(best, o);
+        best = x > best ? x : best;
+    }
+    if (ln() == 0 && best) atomicMax(&L.key, best);
+    return wg_sum1<BS>(L, gone);
+}
+
+// trim-1 (scc_kernels.cu:187-233) on the live bitmap.  A vertex tests its
+// first in- and out-neighbour (pass 0 gathers them); where one is gone it
+// walks the list and keeps the live neighbour it finds as its first one,
+// which the next pass and the bottom-up levels then test.  A pass reads
+// every live vertex's first neighbours, so it stops when a pass removes less
+// than 1/TRIM_STOP of the vertices: what a fixpoint would still remove (the
+// long chains of a sparse graph, a few vertices per pass for dozens of
+// passes) is left to the list phases, whose passes read the listed vertices
+// only (stopping at 1/128 instead of 1/32 of the vertices, and not at all,
+// made the mix's sparsest graphs its last to end).  A graph of which the
+// degrees alone removed less than 1/TRIM_MIN is not trimmed here at all: the
+// gather of its first neighbours, one line of columns per vertex and
+// direction, costs more than what it would remove (mix 3.05 -> 2.69 ms).
+constexpr uint32_t TRIM_CHUNKS = 4;
+constexpr uint32_t TRIM_STOP = 32;
+constexpr uint32_t TRIM_MIN = 8;
+
+template <int BS> __device__ __forceinline__ void g_trim_bits(Lds &L, const G1 &g)
+{
+    const uint32_t nch = (g.V + 64) / 64;
+    uint32_t *F1 = g.f1(), *B1 = g.b1();
+    for (uint32_t pass = 0; pass <= g.V; pass++) {   // each pass removes a vertex or ends
+        uint32_t removed = 0;                        // wave-uniform
+        for (uint32_t c0 = uni(threadIdx.x >> 6); c0 < nch; c0 += TRIM_CHUNKS * (BS / 64)) {
+            uint32_t word[TRIM_CHUNKS], pin[TRIM_CHUNKS], pout[TRIM_CHUNKS];
+            bool any = false;
+#pragma unroll
+            for (uint32_t h = 0; h < TRIM_CHUNKS; h++) {
+                const uint32_t ch = c0 + h * (BS / 64);
+                word[h] = ch < nch ? g.live[2 * ch + (ln() >> 5)] : 0u;
+                any |= word[h] != 0;
+            }
+            if (!__ballot(any)) continue;
+            if (pass == 0) {
+                uint32_t fb[TRIM_CHUNKS], bb[TRIM_CHUNKS];
+#pragma unroll
+                for (uint32_t h = 0; h < TRIM_CHUNKS; h++) {
+                    const uint32_t v = (c0 + h * (BS / 64)) * 64 + ln(), vv = v <= g.V ? v : 0u;
+                    fb[h] = at(g.Fr, vv);
+                    bb[h] = at(g.Br, vv);
+                }
+#pragma unroll
+                for (uint32_t h = 0; h < TRIM_CHUNKS; h++) {
+                    pin[h] = pout[h] = 0;
+                    if ((word[h] >> (ln() & 31)) & 1u) {   // live: both lists have an arc
+                        pin[h] = g.Bc[bb[h]];
+                        pout[h] = g.Fc[fb[h]];
+                    }
+                }
+#pragma unroll
+                for (uint32_t h = 0; h < TRIM_CHUNKS; h++) {
+                    const uint32_t v = (c0 + h * (BS / 64)) * 64 + ln();
+                    if ((word[h] >> (ln() & 31)) & 1u) {
+                        put(B1, v, pin[h]);
+                        put(F1, v, pout[h]);
+                    }
+                }
+            } else {
+#pragma unroll
+                for (uint32_t h = 0; h < TRIM_CHUNKS; h++) {
+                    const uint32_t v = (c0 + h * (BS / 64)) * 64 + ln(), vv = v <= g.V ? v : 0u;
+                    pin[h] = at(B1, vv);
+                    pout[h] = at(F1, vv);
+                }
+            }
+            // lists 2h and 2h + 1: chunk h's in- and out-list, where the first
+            // neighbour is gone (a vertex that is not live has no entry in B1
+            // and F1)
+            const uint32_t *C[2 * TRIM_CHUNKS];
+            uint32_t i[2 * TRIM_CHUNKS], e[2 * TRIM_CHUNKS], x[2 * TRIM_CHUNKS];
+            bool walk = false;
+#pragma unroll
+            for (uint32_t h = 0; h < TRIM_CHUNKS; h++) {
+                const bool alive = (word[h] >> (ln() & 31)) & 1u;
+                C[2 * h] = g.Bc;
+                C[2 * h + 1] = g.Fc;
+                x[2 * h] = !alive || bbit(g.live, pin[h]);
+                x[2 * h + 1] = !alive || bbit(g.live, pout[h]);
+                walk |= !x[2 * h] || !x[2 * h + 1];
+            }
+            if (__ballot(walk)) {
+#pragma unroll
+                for (uint32_t h = 0; h < TRIM_CHUNKS; h++) {
+                    const uint32_t v = (c0 + h * (BS / 64)) * 64 + ln();
+                    const uint32_t ri = x[2 * h] ? 0u : v, ro = x[2 * h + 1] ? 0u : v;   // row 0 is empty
+                    i[2 * h] = at(g.Br, ri);
+                    e[2 * h] = at(g.Br, ri + 1);
+                    i[2 * h + 1] = at(g.Fr, ro);
+                    e[2 * h + 1] = at(g.Fr, ro + 1);
+                }
+                uint32_t y[2 * TRIM_CHUNKS];
+                g_any_bit<2 * TRIM_CHUNKS>(C, i, e, g.live, y);
+#pragma unroll
+                for (uint32_t h = 0; h < TRIM_CHUNKS; h++) {
+                    const uint32_t v = (c0 + h * (BS / 64)) * 64 + ln();
+                    if (y[2 * h]) put(B1, v, y[2 * h]);
+                    if (y[2 * h + 1]) put(F1, v, y[2 * h + 1]);
+                    x[2 * h] |= y[2 * h];
+                    x[2 * h + 1] |= y[2 * h + 1];
+                }
+#pragma unroll
+                for (uint32_t h = 0; h < TRIM_CHUNKS; h++) {
+                    const uint32_t ch = c0 + h * (BS / 64);
+                    const uint64_t m = __ballot(!x[2 * h] || !x[2 * h + 1]);
+                    const uint32_t mw = ln() < 32 ? (uint32_t)m : (uint32_t)(m >> 32);
+                    if ((ln() & 31) == 0 && mw) g.live[2 * ch + (ln() >> 5)] = word[h] & ~mw;
+                    removed += (uint32_t)__popcll(m);
+                }
+            }
+        }
+        if ((uint64_t)wg_sum<BS>(L, ln() == 0 ? removed : 0u, pass & 1) * TRIM_STOP <= g.V) break;
+    }
+    __syncthreads();
+}
+
+// The arcs of frontier entries [lo, hi) of direction d's queue.  SINGLE: every live vertex is in one class, a neighbour is taken
+// if it is live and not visited; otherwise if it is in the vertex's class
+// (a finished vertex is in none) and not visited.
+template <bool SINGLE>
+__device__ __forceinline__ bool g_claim(const G1 &g, uint32_t *vis, uint32_t w, uint32_t c)
+{
+    const uint32_t bit = 1u << (w & 31);
+    const uint32_t word = vis[w >> 5];
+    const bool ok = SINGLE ? (g.live[w >> 5] & ~word & bit) != 0 : (!(word & bit) && g.cls[w] == c);
+    return ok && !(atomicOr(&vis[w >> 5], bit) & bit);
+}
+
+// A wave takes up to 64 frontier vertices, scans their degrees and walks
+// their arcs one after the other with all lanes (consecutive lanes read
+// consecutive columns, EXP_UNR steps in flight), whatever the degree mix: an
+// arc's vertex is the first lane whose running degree sum exceeds the arc's
+// index, found with six shuffles.  w of nw: this wave among the waves that
+// work on this direction.
+constexpr uint32_t EXP_UNR = 2;
+
+template <bool SINGLE>
+__device__ __forceinline__ void g_expand(Lds &L, const G1 &g, uint32_t d, uint32_t lo, uint32_t hi, uint32_t w,
+                                         uint32_t nw)
+{
+    const uint32_t *R = d ? g.Br : g.Fr, *C = d ? g.Bc : g.Fc;
+    uint32_t *vis = d ? g.bvis : g.fvis, *q = g.queue(2 * d);
+    const uint32_t per = min(64u, (hi - lo + nw - 1) / nw);   // vertices per wave and step
+    for (uint32_t t = lo + per * w; t < hi; t += per * nw) {
+        const uint32_t v = ln() < per && t + ln() < hi ? at(q, t + ln()) : 0u;   // row 0 is empty
+        const uint32_t b = at(R, v);
+        uint32_t n = at(R, v + 1) - b;
+        const uint32_t c = SINGLE ? 0u : g.cls[v];
+        if (n >= HUB_DEG) {
+            const uint32_t k = atomicAdd(&L.nhub, 1u);
+            if (k < HUB_CAP) {
+                L.hub[k] = v | (d << 31);
+                n = 0;
+            }
+        }
+        uint32_t sum = n;   // inclusive
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t y = __shfl_up(sum, o);
+            if ((int)ln() >= o) sum += y;
+        }
+        const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)sum, 63);
+        const uint32_t start = b - (sum - n);   // arc j of the tile is C[start + j], modulo 2^32
+        for (uint32_t j0 = 0; j0 < total; j0 += 64 * EXP_UNR) {
+            uint32_t x[EXP_UNR], cx[EXP_UNR];
+            bool ok[EXP_UNR];
+#pragma unroll
+            for (uint32_t u = 0; u < EXP_UNR; u++) {
+                const uint32_t j = j0 + u * 64 + ln();
+                uint32_t own = 0;
+#pragma unroll
+                for (uint32_t o = 32; o >= 1; o >>= 1)
+                    own += (uint32_t)__shfl((int)sum, (int)(own + o - 1)) <= j ? o : 0u;
+                // past the end `own` is 63, and the load is skipped
+                const uint32_t st = __shfl(start, (int)own);
+                cx[u] = SINGLE ? 0u : __shfl(c, (int)own);
+                ok[u] = j < total;
+                x[u] = 0;
+                if (ok[u]) x[u] = C[st + j];
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < EXP_UNR; u++)
+                lpush(ok[u] && g_claim<SINGLE>(g, vis, x[u], cx[u]), x[u], q, &L.tail[d]);
+        }
+    }
+}
+
+// The hubs the level listed, a workgroup's width of arcs at a time (between
+// two barriers).
+template <int BS, bool SINGLE> __device__ __forceinline__ void g_hubs(Lds &L, const G1 &g)
+{
+    const uint32_t nh = uni(min(L.nhub, HUB_CAP));
+    for (uint32_t k = 0; k < nh; k++) {
+        const uint32_t e = uni(L.hub[k]), v = e & 0x7FFFFFFFu, d = e >> 31;
+        const uint32_t *R = d ? g.Br : g.Fr, *C = d ? g.Bc : g.Fc;
+        uint32_t *vis = d ? g.bvis : g.fvis;
+        const uint32_t c = SINGLE ? 0u : g.cls[v];
+        for (uint32_t j = at(R, v) + threadIdx.x, end = at(R, v + 1); j < end; j += BS) {
+            const uint32_t w = C[j];
+            lpush(g_claim<SINGLE>(g, vis, w, c), w, g.queue(2 * d), &L.tail[d]);
+        }
+    }
+}
+
+// A bottom-up level of direction d: a live vertex not yet visited joins if
+// one of its parents is visited: its first parent, if trim-1 has left the
+// array of them (`first`), or one of its row.  A parent that joins in this same level may or may not
+// be seen; if not, it is in the queue that the next level starts from.
+// A level goes bottom-up when its frontier holds more than 1/BU_SWITCH of
+// the vertices left to visit (1/BU_BURST right after growing kBurst-fold), in
+// graphs of at least BU_DEGREE arcs per vertex.  The share is larger than
+// the single-graph engine's 1/16: here a top-down claim is an LDS operation,
+// while a bottom-up level walks the list of nearly every vertex whose first
+// parent is not visited (mix: 1/16 2.93 ms, 1/4 2.77, 1/2 2.69, 1/1 2.66,
+// untrimmed 4.5 to 4.6).  In sparser graphs a whole search top-down costs
+// less than two bottom-up sweeps: 63,665 vertices of 2.07 arcs 1.20 -> 0.66
+// ms for the search; from 8 arcs on it costs more (mix 1.91 -> 2.32 ms with
+// BU_DEGREE at 8).
+constexpr uint32_t BU_CHUNKS = 4;
+constexpr uint64_t BU_SWITCH = 3, BU_BURST = 8, BU_DEGREE = 3;
+
+__device__ __forceinline__ void g_bottom_up(Lds &L, const G1 &g, uint32_t d, uint32_t w, uint32_t nw,
+                                            bool first)
+{
+    const uint32_t *R = d ? g.Fr : g.Br, *C = d ? g.Fc : g.Bc, *P = d ? g.f1() : g.b1();
+    uint32_t *vis = d ? g.bvis : g.fvis, *q = g.queue(2 * d);
+    const uint32_t nch = (g.V + 64) / 64;
+    for (uint32_t c0 = w; c0 < nch; c0 += BU_CHUNKS * nw) {
+        uint32_t word[BU_CHUNKS], cand[BU_CHUNKS], p[BU_CHUNKS];
+        bool any = false;
+#pragma unroll
+        for (uint32_t h = 0; h < BU_CHUNKS; h++) {
+            const uint32_t ch = c0 + h * nw, i = 2 * ch + (ln() >> 5);
+            word[h] = ch < nch ? vis[i] : ~0u;
+            cand[h] = ch < nch ? g.live[i] & ~word[h] : 0u;
+            any |= cand[h] != 0;
+        }
+        if (!__ballot(any)) continue;
+        if (first) {
+#pragma unroll
+            for (uint32_t h = 0; h < BU_CHUNKS; h++) {
+                const uint32_t v = (c0 + h * nw) * 64 + ln();
+                p[h] = at(P, v <= g.V ? v : 0u);
+            }
+        }
+        bool hit[BU_CHUNKS], more[BU_CHUNKS];
+        bool anym = false;
+#pragma unroll
+        for (uint32_t h = 0; h < BU_CHUNKS; h++) {
+            const bool is = (cand[h] >> (ln() & 31)) & 1u;
+            hit[h] = first && is && bbit(vis, p[h]);   // a live vertex has a first parent
+            more[h] = is && !hit[h];
+            anym |= more[h];
+        }
+        if (__ballot(anym)) {
+            const uint32_t *Ck[BU_CHUNKS];
+            uint32_t b[BU_CHUNKS], e[BU_CHUNKS], x[BU_CHUNKS];
+#pragma unroll
+            for (uint32_t h = 0; h < BU_CHUNKS; h++) {
+                const uint32_t r = more[h] ? (c0 + h * nw) * 64 + ln() : 0u;   // row 0 is empty
+                Ck[h] = C;
+                b[h] = at(R, r);
+                e[h] = at(R, r + 1);
+            }
+            g_any_bit<BU_CHUNKS>(Ck, b, e, vis, x);
+#pragma unroll
+            for (uint32_t h = 0; h < BU_CHUNKS; h++) hit[h] |= x[h] != 0;
+        }
+#pragma unroll
+        for (uint32_t h = 0; h < BU_CHUNKS; h++) {
+            const uint32_t ch = c0 + h * nw;
+            const uint64_t m = __ballot(hit[h]);
+            if (!m) continue;
+            const uint32_t mw = ln() < 32 ? (uint32_t)m : (uint32_t)(m >> 32);
+            if ((ln() & 31) == 0 && mw) vis[2 * ch + (ln() >> 5)] = word[h] | mw;
+            lpush(hit[h], ch * 64 + ln(), q, &L.tail[d]);
+        }
+    }
+}
+
+// The waves of a level that has both directions to run are split between
+// them (the two searches do not touch each other's state, so their chains of
+// loads overlap); with one direction left every wave works on it.
+template <int BS, class Level>
+__device__ __forceinline__ void g_both(const uint32_t *lo, const uint32_t *hi, Level level)
+{
+    const uint32_t wv = uni(threadIdx.x >> 6), nwv = BS / 64;
+    if (lo[0] != hi[0] && lo[1] != hi[1]) level(wv & 1, wv >> 1, nwv / 2);
+    else level(lo[0] != hi[0] ? 0u : 1u, wv, nwv);
+}
+
+// The first pivot's FW and BW search, each level of a direction top-down or
+// bottom-up (`dense`: the graph has the arcs for it).
+template <int BS> __device__ __forceinline__ void g_first_search(Lds &L, const G1 &g, uint32_t nlive, bool first, bool dense)
+{
+    uint32_t lo[2] = {0, 0}, hi[2] = {1, 1}, prev[2] = {1, 1};
+    bool bu[2] = {false, false};
+    for (uint32_t level = 0; level <= g.V; level++) {   // each level claims a vertex or ends
+        if (lo[0] == hi[0] && lo[1] == hi[1]) break;
+        g_both<BS>(lo, hi, [&](uint32_t d, uint32_t w, uint32_t nw) {
+            if (d ? bu[1] : bu[0]) g_bottom_up(L, g, d, w, nw, first);
+            else g_expand<true>(L, g, d, d ? lo[1] : lo[0], d ? hi[1] : hi[0], w, nw);
+        });
+        __syncthreads();
+        if (uni(L.nhub)) {
+            g_hubs<BS, true>(L, g);
+            __syncthreads();
+            if (threadIdx.x == 0) L.nhub = 0;
+        }
+        for (uint32_t d = 0; d < 2; d++) {
+            if (lo[d] == hi[d]) continue;
+            lo[d] = hi[d];
+            hi[d] = uni(L.tail[d]);
+            const uint64_t nf = hi[d] - lo[d], left = nlive - hi[d];
+            if (!bu[d])
+                bu[d] = dense && nf * (nf > kBurst * (uint64_t)prev[d] ? BU_BURST : BU_SWITCH) > left &&
+                        nf * kBottomUpFloor >= nlive;
+            else
+                bu[d] = nf * kToTopDown >= nlive;
+            prev[d] = (uint32_t)nf;
+        }
+        __syncthreads();   // every lane has read the tails and the hub count
+    }
+}
+
+// ----------------------------------------------- the later phases ---
+// Over the `n` vertices the first round left (g.list()), in classes.
+
+#define LIST_LOOP(v)                                                                        \
+    for (uint32_t _i = threadIdx.x, v; _i < n && (v = at(list, _i), true); _i += BS)
+
+template <int BS> __device__ __forceinline__ void g_trim1(Lds &L, const G1 &g, uint32_t n)
+{
+    const uint32_t *list = g.list();
     for (uint32_t pass = 0; pass <= g.V; pass++) {   // each pass removes a vertex or ends
         uint32_t removed = 0;
-        for (uint32_t v = threadIdx.x + 1; v <= g.V; v += BS) {
+        LIST_LOOP(v)
+        {
             // class and both rows' offsets together; a dead vertex scans
             // empty ranges, so the offsets are used on every path and are
             // not loaded after the class test or the first scan
             const uint32_t c = g.cls[v];
-            const uint32_t bb = g.Br[v], be = g.Br[v + 1], fb = g.Fr[v], fe = g.Fr[v + 1];
+            const uint32_t bb = at(g.Br, v), be = at(g.Br, v + 1), fb = at(g.Fr, v), fe = at(g.Fr, v + 1);
             const bool act = c != DEAD;
             const bool kin = g_any_cls(g.Bc, bb, act ? be : bb, g.cls, c);
             const bool keep = kin && g_any_cls(g.Fc, fb, fe, g.cls, c);
-            if (act && !keep) {
-                g.lab[v] = v | LAB_FINAL;
+            if (act && !keep) {   // its label is still the v | LAB_FINAL it was listed with
                 __hip_atomic_store(&g.cls[v], DEAD, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                 removed++;
             }
         }
-        const uint32_t n = wg_sum<BS>(L, removed);
-        total += n;
-        if (!fixpoint || !n) break;
+        if (!wg_sum<BS>(L, removed, pass & 1)) break;
     }
-    return total;
+    __syncthreads();
 }
 
 __device__ __forceinline__ int g_deg2(const uint32_t *R, const uint32_t *C, const uint32_t *cls,
                                       uint32_t v, uint32_t c, uint32_t *k)
 {
     int d = 0;
-    for (uint32_t i = R[v], e = R[v + 1]; i < e; i++) {
+    for (uint32_t i = at(R, v), e = at(R, v + 1); i < e; i++) {
         const uint32_t w = C[i];
         if (cls[w] != c) continue;
         if (++d == 2) return 2;
@@ -188,15 +679,17 @@ __device__ __forceinline__ int g_deg2(const uint32_t *R, const uint32_t *C, cons
 
 __device__ __forceinline__ bool g_arc(const uint32_t *R, const uint32_t *C, uint32_t v, uint32_t k)
 {
-    for (uint32_t i = R[v], e = R[v + 1]; i < e; i++)
+    for (uint32_t i = at(R, v), e = at(R, v + 1); i < e; i++)
         if (C[i] == k) return true;
     return false;
 }
 
 // trim-2 (scc_kernels.cu:236-357), claim by CAS on the smaller id
-template <int BS> __device__ void g_trim2(const G1 &g)
+template <int BS> __device__ __forceinline__ void g_trim2(const G1 &g, uint32_t n)
 {
-    for (uint32_t v = threadIdx.x + 1; v <= g.V; v += BS) {
+    const uint32_t *list = g.list();
+    LIST_LOOP(v)
+    {
         const uint32_t c = g.cls[v];
         if (c == DEAD) continue;
         uint32_t k = 0, kk = 0;
@@ -219,123 +712,72 @@ template <int BS> __device__ void g_trim2(const G1 &g)
     __syncthreads();
 }
 
-// FW and/or BW level loop from queues [0] with counts L.cnt[0] / L.cnt[2]
-template <int BS> __device__ void g_reach(Lds &L, const G1 &g, bool do_bw, bool single, uint32_t W)
+// no vertex visited (finished ones are told apart by their class)
+template <int BS> __device__ __forceinline__ void g_clear_vis(const G1 &g)
 {
-    int in = 0;
-    for (uint32_t level = 0; level <= g.V; level++) {   // each level claims a vertex or ends
-        const uint32_t nf = L.cnt[0], nb = do_bw ? L.cnt[2] : 0u;
-        if (!nf && !nb) break;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            L.cnt[1] = 0;
-            L.cnt[3] = 0;
-        }
-        __syncthreads();
-        const uint32_t grp = threadIdx.x / W, sub = threadIdx.x % W, ngrp = BS / W;
-        for (int d = 0; d < 2; d++) {
-            const uint32_t n = d ? nb : nf;
-            const uint32_t *R = d ? g.Br : g.Fr, *C = d ? g.Bc : g.Fc;
-            uint32_t *vis = d ? g.bvis : g.fvis;
-            const uint32_t *qin = g.queue(2 * d + in);
-            uint32_t *qout = g.queue(2 * d + (in ^ 1));
-            uint32_t *cnt = &L.cnt[d ? 3 : 1];
-            // two frontier vertices per lane group in flight: their queue
-            // entries, rows, columns and probes are loaded side by side
-            // (vertex 0, the dummy, stands for "none": its row is empty)
-            for (uint32_t i0 = grp; i0 < n; i0 += 2 * ngrp) {
-                uint32_t v[2], b[2], e[2], c[2];
-#pragma unroll
-                for (uint32_t u = 0; u < 2; u++) v[u] = i0 + u * ngrp < n ? qin[i0 + u * ngrp] : 0u;
-#pragma unroll
-                for (uint32_t u = 0; u < 2; u++) {
-                    b[u] = R[v[u]];
-                    e[u] = R[v[u] + 1];
-                    c[u] = single ? 0u : g.cls[v[u]];
-                }
-                const uint32_t d0 = e[0] - b[0], d1 = e[1] - b[1];
-                const uint32_t dm = d0 > d1 ? d0 : d1;
-                for (uint32_t j = sub; j < dm; j += W) {
-                    uint32_t w[2] = {0u, 0u};
-                    bool ok[2] = {j < d0, j < d1};
-#pragma unroll
-                    for (uint32_t u = 0; u < 2; u++)
-                        if (ok[u]) w[u] = C[b[u] + j];
-                    uint32_t word[2] = {~0u, ~0u}, wc[2] = {0u, 0u};
-#pragma unroll
-                    for (uint32_t u = 0; u < 2; u++)
-                        if (ok[u]) {
-                            word[u] = vis[w[u] >> 5];
-                            if (!single) wc[u] = g.cls[w[u]];
-                        }
-                    bool claimed[2] = {false, false};
-#pragma unroll
-                    for (uint32_t u = 0; u < 2; u++) {
-                        const uint32_t bit = 1u << (w[u] & 31);
-                        if (ok[u] && !(word[u] & bit) && (single || wc[u] == c[u]))
-                            claimed[u] = !(atomicOr(&vis[w[u] >> 5], bit) & bit);
-                    }
-#pragma unroll
-                    for (uint32_t u = 0; u < 2; u++) lpush(claimed[u], w[u], qout, cnt);
-                }
-            }
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            L.cnt[0] = L.cnt[1];
-            L.cnt[2] = L.cnt[3];
-        }
-        __syncthreads();
-        in ^= 1;
+    const uint32_t nw = 2 * ((g.V + 64) / 64);
+    for (uint32_t i = threadIdx.x; i < nw; i += BS) {
+        g.fvis[i] = 0;
+        g.bvis[i] = 0;
     }
 }
 
-// pivots: one per live class (first = single class, reduced in LDS)
-template <int BS> __device__ uint32_t g_pivots(Lds &L, const G1 &g, bool first)
+// FW and, with do_bw, BW top-down levels from the seeded queues
+template <int BS> __device__ __forceinline__ void g_reach(Lds &L, const G1 &g, bool do_bw)
 {
-    if (first) {
-        unsigned long long m = 0;
-        for (uint32_t v = threadIdx.x + 1; v <= g.V; v += BS)
-            if (g.cls[v] != DEAD) {
-                const unsigned long long k = bkey(g.Fr, g.Br, v);
-                m = k > m ? k : m;
-            }
-        for (int o = 32; o > 0; o >>= 1) {
-            unsigned long long x = __shfl_xor(m, o);
-            m = x > m ? x : m;
+    uint32_t lo[2] = {0, 0};
+    uint32_t hi[2] = {uni(L.tail[0]), do_bw ? uni(L.tail[1]) : 0u};
+    __syncthreads();
+    for (uint32_t level = 0; level <= g.V; level++) {   // each level claims a vertex or ends
+        if (lo[0] == hi[0] && lo[1] == hi[1]) break;
+        g_both<BS>(lo, hi, [&](uint32_t d, uint32_t w, uint32_t nw) {
+            g_expand<false>(L, g, d, d ? lo[1] : lo[0], d ? hi[1] : hi[0], w, nw);
+        });
+        __syncthreads();
+        if (uni(L.nhub)) {
+            g_hubs<BS, false>(L, g);
+            __syncthreads();
+            if (threadIdx.x == 0) L.nhub = 0;
         }
-        if (threadIdx.x == 0) L.key = 0;
+        for (uint32_t d = 0; d < 2; d++) {
+            if (lo[d] == hi[d]) continue;
+            lo[d] = hi[d];
+            hi[d] = uni(L.tail[d]);
+        }
         __syncthreads();
-        if (ln() == 0 && m) atomicMax(&L.key, m);
-        __syncthreads();
-        if (threadIdx.x == 0) g.piv[0] = L.key;
-    } else {
-        // a wave whose live lanes share a class does one atomic
-        unsigned long long *piv = reinterpret_cast<unsigned long long *>(g.piv);
-        for (uint32_t base = threadIdx.x & ~63u; base <= g.V; base += BS) {
-            const uint32_t v = base + ln();
-            const uint32_t c = (v >= 1 && v <= g.V) ? g.cls[v] : DEAD;
-            const bool ok = c != DEAD;
-            const uint64_t live = __ballot(ok);
-            if (!live) continue;
-            const int lead = __ffsll((unsigned long long)live) - 1;
-            const uint32_t c0 = __shfl(c, lead);
-            unsigned long long k = ok ? bkey(g.Fr, g.Br, v) : 0ull;
-            if (__all(!ok || c == c0)) {
-                for (int o = 32; o > 0; o >>= 1) {
-                    const unsigned long long x = __shfl_xor(k, o);
-                    k = x > k ? x : k;
-                }
-                if ((int)ln() == lead && k > __hip_atomic_load(&piv[c0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-                    atomicMax(&piv[c0], k);
-            } else if (ok && k > __hip_atomic_load(&piv[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-                atomicMax(&piv[c], k);
+    }
+}
+
+// One pivot per live class, seeded in both directions.
+template <int BS> __device__ __forceinline__ void g_pivots(Lds &L, const G1 &g, uint32_t n)
+{
+    const uint32_t *list = g.list();
+    // a wave whose live lanes share a class does one atomic
+    unsigned long long *piv = reinterpret_cast<unsigned long long *>(g.piv);
+    for (uint32_t i0 = threadIdx.x & ~63u; i0 < n; i0 += BS) {
+        const uint32_t v = i0 + ln() < n ? at(list, i0 + ln()) : 0u;   // vertex 0, the dummy, is dead
+        const uint32_t c = g.cls[v];
+        const bool ok = c != DEAD;
+        const uint64_t live = __ballot(ok);
+        if (!live) continue;
+        const int lead = __ffsll((unsigned long long)live) - 1;
+        const uint32_t c0 = __shfl(c, lead);
+        unsigned long long k = ok ? bkey(g.Fr, g.Br, v) : 0ull;
+        if (__all(!ok || c == c0)) {
+            for (int o = 32; o > 0; o >>= 1) {
+                const unsigned long long x = __shfl_xor(k, o);
+                k = x > k ? x : k;
             }
+            if ((int)ln() == lead && k > __hip_atomic_load(&piv[c0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                atomicMax(&piv[c0], k);
+        } else if (ok && k > __hip_atomic_load(&piv[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+            atomicMax(&piv[c], k);
         }
     }
     if (threadIdx.x == 0) L.npiv = 0;
     __syncthreads();
-    for (uint32_t v = threadIdx.x + 1; v <= g.V; v += BS) {
+    LIST_LOOP(v)
+    {
         const uint32_t c = g.cls[v];
         const bool win = c != DEAD && g.piv[c] == bkey(g.Fr, g.Br, v);
         if (win) {
@@ -345,24 +787,25 @@ template <int BS> __device__ uint32_t g_pivots(Lds &L, const G1 &g, bool first)
         lpush(win, v, g.pivlist, &L.npiv);
     }
     __syncthreads();
-    const uint32_t n = L.npiv;
-    for (uint32_t i = threadIdx.x; i < n; i += BS) {
+    const uint32_t np = uni(L.npiv);
+    for (uint32_t i = threadIdx.x; i < np; i += BS) {
         g.queue(0)[i] = g.pivlist[i];
         g.queue(2)[i] = g.pivlist[i];
     }
     if (threadIdx.x == 0) {
-        L.cnt[0] = n;
-        L.cnt[2] = n;
+        L.tail[0] = np;
+        L.tail[1] = np;
     }
     __syncthreads();
-    return n;
 }
 
 // update (scc_kernels.cu:124-142) + clear the next round's pivot slots
-template <int BS> __device__ uint32_t g_update(Lds &L, const G1 &g)
+template <int BS> __device__ __forceinline__ uint32_t g_update(Lds &L, const G1 &g, uint32_t n)
 {
+    const uint32_t *list = g.list();
     uint32_t live = 0;
-    for (uint32_t v = threadIdx.x + 1; v <= g.V; v += BS) {
+    LIST_LOOP(v)
+    {
         const uint32_t c = g.cls[v];
         if (c == DEAD) continue;
         uint32_t p = bkey_vertex(g.piv[c]);
@@ -379,7 +822,7 @@ template <int BS> __device__ uint32_t g_update(Lds &L, const G1 &g)
             live++;
         }
     }
-    const uint32_t n = wg_sum<BS>(L, live);
+    const uint32_t left = wg_sum1<BS>(L, live);
     for (uint32_t i = threadIdx.x; i < L.npiv; i += BS) {
         const uint32_t p = g.pivlist[i];
         g.piv[3ull * p] = 0;
@@ -387,34 +830,27 @@ template <int BS> __device__ uint32_t g_update(Lds &L, const G1 &g)
         g.piv[3ull * p + 2] = 0;
     }
     __syncthreads();
-    return n;
-}
-
-template <int BS> __device__ void g_pivot_round(Lds &L, const G1 &g, bool first, uint32_t W, uint32_t *live)
-{
-    g_init_vis<BS>(g);
-    __syncthreads();
-    g_pivots<BS>(L, g, first);
-    g_reach<BS>(L, g, true, first, W);
-    *live = g_update<BS>(L, g);
+    return left;
 }
 
 // "WCC" min reachable label with pointer jumping (scc_kernels.cu:477-536)
-template <int BS> __device__ void g_minlabel(Lds &L, const G1 &g)
+template <int BS> __device__ __forceinline__ void g_minlabel(Lds &L, const G1 &g, uint32_t n)
 {
-    for (uint32_t v = threadIdx.x + 1; v <= g.V; v += BS)
+    const uint32_t *list = g.list();
+    LIST_LOOP(v)
         if (g.cls[v] != DEAD) g.cls[v] = v;
     __syncthreads();
     for (uint32_t it = 0; it <= g.V; it++) {   // labels only decrease
         uint32_t changed = 0;
-        for (uint32_t v = threadIdx.x + 1; v <= g.V; v += BS) {
+        LIST_LOOP(v)
+        {
             // label and row offsets together (an inactive lane folds an
             // empty range, so the offsets are used on every path)
-            const uint32_t m0 = g.cls[v], b = g.Fr[v], e = g.Fr[v + 1];
+            const uint32_t m0 = g.cls[v], b = at(g.Fr, v), e = at(g.Fr, v + 1);
             const bool act = m0 != DEAD;
             uint32_t m = g_fold<false>(g.Fc, b, act ? e : b, g.cls, m0);
             if (!act) continue;
-            for (int it = 0; it < 32; it++) {
+            for (int jump = 0; jump < 32; jump++) {
                 const uint32_t x = g.cls[m];
                 if (x >= m) break;
                 m = x;
@@ -424,9 +860,11 @@ template <int BS> __device__ void g_minlabel(Lds &L, const G1 &g)
                 changed = 1;
             }
         }
-        if (!wg_sum<BS>(L, changed)) break;
+        if (!wg_sum<BS>(L, changed, it & 1)) break;
     }
-    for (uint32_t v = threadIdx.x + 1; v <= g.V; v += BS) {
+    __syncthreads();
+    LIST_LOOP(v)
+    {
         const uint32_t m = g.cls[v];
         if (m == DEAD) continue;
         if (m == v) g.piv[3ull * v] = 0;
@@ -435,21 +873,26 @@ template <int BS> __device__ void g_minlabel(Lds &L, const G1 &g)
     __syncthreads();
 }
 
-// vSlota colouring loop (scc_Coloring.cu:590-637)
-template <int BS> __device__ void g_color_loop(Lds &L, const G1 &g, uint32_t W, uint32_t live)
+// vSlota colouring loop (scc_Coloring.cu:590-637); aux is 0 for every
+// vertex outside the list
+template <int BS> __device__ __forceinline__ void g_color_loop(Lds &L, const G1 &g, uint32_t n)
 {
+    const uint32_t *list = g.list();
+    uint32_t live = n;
     for (uint32_t round = 0; live && round <= g.V; round++) {   // a round finishes >= 1 SCC
-        for (uint32_t v = threadIdx.x; v <= g.V; v += BS) g.aux[v] = (v && g.cls[v] != DEAD) ? v : 0u;
+        LIST_LOOP(v)
+            g.aux[v] = g.cls[v] != DEAD ? v : 0u;
         __syncthreads();
         for (uint32_t it = 0; it <= g.V; it++) {   // colours only increase
             uint32_t changed = 0;
-            for (uint32_t v = threadIdx.x + 1; v <= g.V; v += BS) {
+            LIST_LOOP(v)
+            {
                 // as in g_minlabel
-                const uint32_t m0 = g.aux[v], b = g.Fr[v], e = g.Fr[v + 1];
+                const uint32_t m0 = g.aux[v], b = at(g.Fr, v), e = at(g.Fr, v + 1);
                 const bool act = m0 != 0;
                 uint32_t m = g_fold<true>(g.Fc, b, act ? e : b, g.aux, m0);
                 if (!act) continue;
-                for (int it = 0; it < 32; it++) {
+                for (int jump = 0; jump < 32; jump++) {
                     const uint32_t x = g.aux[m];
                     if (x <= m) break;
                     m = x;
@@ -459,12 +902,14 @@ template <int BS> __device__ void g_color_loop(Lds &L, const G1 &g, uint32_t W, 
                     changed = 1;
                 }
             }
-            if (!wg_sum<BS>(L, changed)) break;
+            if (!wg_sum<BS>(L, changed, it & 1)) break;
         }
-        g_init_vis<BS>(g);
-        if (threadIdx.x == 0) L.cnt[0] = 0;
         __syncthreads();
-        for (uint32_t v = threadIdx.x + 1; v <= g.V; v += BS) {
+        g_clear_vis<BS>(g);
+        if (threadIdx.x == 0) L.tail[0] = 0;
+        __syncthreads();
+        LIST_LOOP(v)
+        {
             bool root = false;
             if (g.cls[v] != DEAD) {
                 const uint32_t c = g.aux[v];
@@ -472,12 +917,13 @@ template <int BS> __device__ void g_color_loop(Lds &L, const G1 &g, uint32_t W, 
                 root = c == v;
                 if (root) atomicOr(&g.fvis[v >> 5], 1u << (v & 31));
             }
-            lpush(root, v, g.queue(0), &L.cnt[0]);
+            lpush(root, v, g.queue(0), &L.tail[0]);
         }
         __syncthreads();
-        g_reach<BS>(L, g, false, false, W);
+        g_reach<BS>(L, g, false);
         uint32_t lv = 0;
-        for (uint32_t v = threadIdx.x + 1; v <= g.V; v += BS) {
+        LIST_LOOP(v)
+        {
             const uint32_t c = g.cls[v];
             if (c == DEAD) continue;
             if (bbit(g.fvis, v)) {
@@ -487,22 +933,24 @@ template <int BS> __device__ void g_color_loop(Lds &L, const G1 &g, uint32_t W, 
                 lv++;
             }
         }
-        live = wg_sum<BS>(L, lv);
+        live = wg_sum1<BS>(L, lv);
     }
 }
 
-// canonical labels; returns the number of SCCs
+// Canonical labels of the listed vertices; returns their number of SCCs.
 // The minimum per label: lanes of a wave that share a label combine first
 // (up to four labels per wave step, then lane by lane), and the guard reads
 // the current minimum at agent scope (the CU's L1 may hold a stale copy),
 // so a large SCC costs about one atomic per wave instead of one per vertex.
-template <int BS> __device__ uint32_t g_canon(Lds &L, const G1 &g)
+template <int BS> __device__ __forceinline__ uint32_t g_canon(Lds &L, const G1 &g, uint32_t n)
 {
-    for (uint32_t v = threadIdx.x; v <= g.V; v += BS) g.aux[v] = DEAD;
+    const uint32_t *list = g.list();
+    LIST_LOOP(v)
+        g.aux[v] = DEAD;
     __syncthreads();
-    for (uint32_t base = threadIdx.x & ~63u; base <= g.V; base += BS) {
-        const uint32_t v = base + ln();
-        const uint32_t l = (v >= 1 && v <= g.V) ? g.lab[v] : LAB_FINAL;
+    for (uint32_t i0 = threadIdx.x & ~63u; i0 < n; i0 += BS) {
+        const uint32_t v = i0 + ln() < n ? at(list, i0 + ln()) : 0u;
+        const uint32_t l = v ? g.lab[v] : LAB_FINAL;
         bool pending = !(l & LAB_FINAL);
         for (int it = 0; it < 4; it++) {
             const uint64_t pm = __ballot(pending);
@@ -525,104 +973,194 @@ template <int BS> __device__ uint32_t g_canon(Lds &L, const G1 &g)
     }
     __syncthreads();
     uint32_t roots = 0;
-    for (uint32_t v = threadIdx.x + 1; v <= g.V; v += BS) {
+    LIST_LOOP(v)
+    {
         const uint32_t l = g.lab[v];
         const uint32_t r = (l & LAB_FINAL) ? (l & ~LAB_FINAL) : g.aux[l];
         g.lab[v] = r;
         roots += r == v;
     }
-    if (threadIdx.x == 0) g.lab[0] = 0;
-    return wg_sum<BS>(L, roots);
+    return wg_sum1<BS>(L, roots);
+}
+
+// The whole pipeline of one graph; returns its number of SCCs.  LDS_BITS /
+// LDS_CLS only say which memory the views point to: the code is the same,
+// and inlined per case so that the accesses are LDS instructions.
+template <int BS> __device__ __forceinline__ uint32_t g_solve(Lds &L, const G1 &g, uint32_t cfg)
+{
+    const uint32_t nch = (g.V + 64) / 64, nw = 2 * nch;
+    if (threadIdx.x == 0) {
+        L.key = 0;
+        L.nhub = 0;
+        L.nact = 0;
+        L.anom = 0;
+    }
+    __syncthreads();
+    const uint32_t ndeg = g_degrees<BS>(L, g, cfg_t1(cfg));
+    const bool first = (uint64_t)ndeg * TRIM_MIN > g.V;   // never with the trims off
+    if (first) g_trim_bits<BS>(L, g);
+    uint32_t nl = 0;
+    for (uint32_t i = threadIdx.x; i < nw; i += BS) {
+        nl += (uint32_t)__popc(g.live[i]);
+        g.fvis[i] = 0;
+        g.bvis[i] = 0;
+    }
+    const uint32_t nlive = wg_sum1<BS>(L, nl);
+    // the best key of the degree pass may name a vertex the trim removed
+    if (nlive && !bbit(g.live, bkey_vertex(L.key))) {
+        __syncthreads();
+        if (threadIdx.x == 0) L.key = 0;
+        __syncthreads();
+        unsigned long long best = 0;
+        for (uint32_t v = threadIdx.x; v <= g.V; v += BS)
+            if (bbit(g.live, v)) {
+                const unsigned long long k = bkey(g.Fr, g.Br, v);
+                best = k > best ? k : best;
+            }
+        for (int o = 32; o > 0; o >>= 1) {
+            const unsigned long long x = __shfl_xor(best, o);
+            best = x > best ? x : best;
+        }
+        if (ln() == 0 && best) atomicMax(&L.key, best);
+        __syncthreads();
+    }
+    const uint32_t p0 = nlive ? uni(bkey_vertex(L.key)) : 0u;
+    if (nlive) {
+        if (threadIdx.x == 0) {
+            g.fvis[p0 >> 5] |= 1u << (p0 & 31);
+            g.bvis[p0 >> 5] |= 1u << (p0 & 31);
+            g.queue(0)[0] = p0;
+            g.queue(2)[0] = p0;
+            L.tail[0] = 1;
+            L.tail[1] = 1;
+        }
+        __syncthreads();
+        g_first_search<BS>(L, g, nlive, first, g.E >= BU_DEGREE * (uint64_t)g.V);
+    }
+    // the pivot's SCC: its size, its smallest vertex
+    uint32_t members = 0, least = DEAD;
+    for (uint32_t i = threadIdx.x; i < nw; i += BS) {
+        const uint32_t m = g.live[i] & g.fvis[i] & g.bvis[i];
+        members += (uint32_t)__popc(m);
+        if (m && least == DEAD) least = 32 * i + (uint32_t)(__ffs(m) - 1);
+    }
+    const uint32_t nmem = wg_sum1<BS>(L, members), root = wg_min1<BS>(L, least);
+    const uint32_t singles = g.V - nlive;   // trim-1's
+    if (nmem == nlive) {
+        for (uint32_t v = threadIdx.x; v <= g.V; v += BS) g.lab[v] = bbit(g.live, v) ? root : v;
+        return singles + (nmem ? 1u : 0u);
+    }
+    // Vertices are left: their classes and the list of them.  Every other
+    // label is final.  Class 3 p0 + k needs its pivot key cleared.
+    const bool slota = cfg_slota(cfg);
+    uint32_t *list = g.list();   // the first out-neighbours are not needed any more
+    for (uint32_t c0 = uni(threadIdx.x >> 6); c0 < nch; c0 += BS / 64) {
+        const uint32_t v = c0 * 64 + ln(), i = 2 * c0 + (ln() >> 5), sh = ln() & 31;
+        const uint32_t lw = g.live[i], f = (g.fvis[i] >> sh) & 1u, b = (g.bvis[i] >> sh) & 1u;
+        const bool alive = (lw >> sh) & 1u, rest = alive && !(f && b);
+        if (v <= g.V) {
+            g.lab[v] = alive && !rest ? root : (rest ? v | LAB_FINAL : v);
+            g.cls[v] = rest ? 3u * p0 + f + 2u * b : DEAD;
+            if (slota) g.aux[v] = 0;
+        }
+        lpush(rest, v, list, &L.nact);
+    }
+    if (threadIdx.x < 3) g.piv[3ull * p0 + threadIdx.x] = 0;
+    __syncthreads();
+    const uint32_t n = uni(L.nact);
+    if (!slota) {
+        if (cfg_t1(cfg)) g_trim1<BS>(L, g, n);
+        if (cfg_t2(cfg)) {
+            g_trim2<BS>(g, n);
+            if (cfg_t1(cfg)) g_trim1<BS>(L, g, n);
+        }
+        g_minlabel<BS>(L, g, n);
+        for (uint32_t round = 0; round <= g.V + 1; round++) {
+            g_clear_vis<BS>(g);
+            __syncthreads();
+            g_pivots<BS>(L, g, n);
+            g_reach<BS>(L, g, true);
+            if (!g_update<BS>(L, g, n)) break;
+        }
+    } else {
+        g_color_loop<BS>(L, g, n);
+    }
+    return singles + (nmem ? 1u : 0u) + g_canon<BS>(L, g, n);
 }
 
 } // namespace
 
-// LDS tiers.  A graph whose visited bitmaps fit `vis_words` words each keeps
-// them in LDS, so probes and claims are LDS operations (a device-wide
-// atomic costs a share of a chip-wide rate of about 10 G/s); a graph whose
-// class words fit `cls_words` keeps those in LDS as well, so the
-// neighbour-class tests of the trims, searches and colouring stay on the
-// CU.  Larger graphs use their slots in global memory (the views are
-// generic pointers, so the phase code is the same either way).  The tiers
-// shrink with the workgroup so that smaller workgroups share a CU:
-//   1,024 lanes: bitmaps up to 2^16 vertices, classes up to 2^15 (about
-//                145 KB: one workgroup per CU, which its registers allow)
-//     512 lanes: bitmaps up to 2^15, classes up to 2^14 (about 74 KB: two)
-//     256 lanes: bitmaps up to 2^15, classes up to 2^13 (about 41 KB: three)
+// LDS tiers.  A graph whose bitmaps (live, FW and BW visited) fit `words`
+// words each keeps them in LDS, so probes and claims are LDS operations (a
+// device-wide atomic costs a share of a chip-wide rate of about 10 G/s); a
+// graph whose class words fit `cls_words` keeps those in LDS as well for the
+// phases after the first round.  Larger graphs use their slots in global
+// memory.  The tiers leave room for several workgroups per CU:
+// (their number is set by registers before LDS at 1,024 and 512 lanes):
+//   1,024 lanes: bitmaps up to 2^16 vertices, classes up to 2^13 (58 KB)
+//     512 lanes: bitmaps up to 2^16, classes up to 2^12 (42 KB)
+//     256 lanes: bitmaps up to 2^16, classes up to 2^11 (34 KB)
 template <int BS> struct BTier;
 template <> struct BTier<1024> {
-    static constexpr uint32_t vis_words = 2 * ((65536 + 64) / 64);
-    static constexpr uint32_t cls_words = (1u << 15) + 2;
+    static constexpr uint32_t words = 2 * ((65536 + 64) / 64);
+    static constexpr uint32_t cls_words = (1u << 13) + 2;
 };
 template <> struct BTier<512> {
-    static constexpr uint32_t vis_words = 2 * ((32768 + 64) / 64);
-    static constexpr uint32_t cls_words = (1u << 14) + 2;
+    static constexpr uint32_t words = 2 * ((65536 + 64) / 64);
+    static constexpr uint32_t cls_words = (1u << 12) + 2;
 };
 template <> struct BTier<256> {
-    static constexpr uint32_t vis_words = 2 * ((32768 + 64) / 64);
-    static constexpr uint32_t cls_words = (1u << 13) + 2;
+    static constexpr uint32_t words = 2 * ((65536 + 64) / 64);
+    static constexpr uint32_t cls_words = (1u << 11) + 2;
 };
 
 template <int BS>
 __global__ __launch_bounds__(BS) void batch_scc_kernel(BatchDev B, uint32_t first, uint32_t count)
 {
     __shared__ Lds L;
-    __shared__ uint32_t s_vis[2][BTier<BS>::vis_words];
+    __shared__ uint32_t s_bits[3][BTier<BS>::words];
     __shared__ uint32_t s_cls[BTier<BS>::cls_words];
     for (;;) {
         __syncthreads();
         if (threadIdx.x == 0) L.graph = atomicAdd(B.next, 1u);
         __syncthreads();
-        const uint32_t k = L.graph;
+        const uint32_t k = uni(L.graph);
         if (k >= count) break;
         const uint32_t gi = B.order[first + k];
         const uint64_t vo = B.voff[gi], eo = B.eoff[gi];
+        const uint32_t cfg = B.cfg[gi];
+        const uint64_t t0 = wall_clock64();
         G1 g;
         g.V = B.Vn[gi];
+        g.E = (uint32_t)(B.eoff[gi + 1] - eo);
         g.Fr = B.Fr + vo;
         g.Br = B.Br + vo;
         g.Fc = B.Fc + eo;
         g.Bc = B.Bc + eo;
-        g.cls = g.V + 1 <= BTier<BS>::cls_words ? s_cls : B.cls + vo;
         g.lab = B.lab + vo;
         g.aux = B.aux + vo;
-        // g_init_vis writes 2 * ((V + 64) / 64) words of each bitmap
-        const bool lds_vis = 2 * ((g.V + 64) / 64) <= BTier<BS>::vis_words;
-        g.fvis = lds_vis ? s_vis[0] : B.fvis + vo / 32;
-        g.bvis = lds_vis ? s_vis[1] : B.bvis + vo / 32;
         g.piv = B.piv + 3 * vo;
         g.q = B.q + 4 * vo;
         g.pivlist = B.pivlist + vo;
-        const uint32_t cfg = B.cfg[gi];
-        const uint32_t W = cfg_lanes(cfg);
-        const uint64_t t0 = wall_clock64();
-        for (uint32_t v = threadIdx.x; v <= g.V; v += BS) {
-            g.cls[v] = v ? 0u : DEAD;
-            g.lab[v] = v ? (v | LAB_FINAL) : 0u;
-        }
-        if (threadIdx.x == 0) {
-            g.piv[0] = 0;
-            L.anom = 0;
-        }
-        __syncthreads();
-        uint32_t live = g.V;
-        if (!cfg_slota(cfg)) {
-            if (cfg_t1(cfg)) g_trim1<BS>(L, g, true);
-            g_pivot_round<BS>(L, g, true, W, &live);
-            if (cfg_t1(cfg)) g_trim1<BS>(L, g, true);
-            if (cfg_t2(cfg)) g_trim2<BS>(g);
-            if (cfg_t1(cfg)) g_trim1<BS>(L, g, true);
-            g_minlabel<BS>(L, g);
-            for (uint32_t round = 0; round <= g.V + 1; round++) {
-                g_pivot_round<BS>(L, g, false, W, &live);
-                if (!live) break;
-            }
+        uint32_t n;
+        if (2 * ((g.V + 64) / 64) > BTier<BS>::words) {
+            g.live = g.queue(3);
+            g.fvis = B.fvis + vo / 32;
+            g.bvis = B.bvis + vo / 32;
+            g.cls = B.cls + vo;
+            n = g_solve<BS>(L, g, cfg);
         } else {
-            if (cfg_t1(cfg)) g_trim1<BS>(L, g, false);
-            g_pivot_round<BS>(L, g, true, W, &live);
-            g_color_loop<BS>(L, g, W, live);
+            g.live = s_bits[0];
+            g.fvis = s_bits[1];
+            g.bvis = s_bits[2];
+            if (g.V + 1 > BTier<BS>::cls_words) {
+                g.cls = B.cls + vo;
+                n = g_solve<BS>(L, g, cfg);
+            } else {
+                g.cls = s_cls;
+                n = g_solve<BS>(L, g, cfg);
+            }
         }
-        const uint32_t n = g_canon<BS>(L, g);
         if (threadIdx.x == 0) {
             B.nscc[gi] = L.anom ? BATCH_ANOMALY : n;
             B.tstart[gi] = t0;
@@ -631,11 +1169,9 @@ __global__ __launch_bounds__(BS) void batch_scc_kernel(BatchDev B, uint32_t firs
     }
 }
 
-uint32_t batch_cfg(int lanes, bool trim1, bool trim2, bool slota)
+uint32_t batch_cfg(bool trim1, bool trim2, bool slota)
 {
-    uint32_t lg = 0;
-    while ((1 << (lg + 1)) <= lanes && lg < 6) lg++;
-    return lg | (trim1 ? 8u : 0u) | (trim2 ? 16u : 0u) | (slota ? 32u : 0u);
+    return (trim1 ? 1u : 0u) | (trim2 ? 2u : 0u) | (slota ? 4u : 0u);
 }
 
 int batch_occupancy(int block)

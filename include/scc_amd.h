@@ -295,7 +295,8 @@ scc_status scc_gen_serving_mix(uint32_t num_graphs, double median_v, double sigm
 typedef struct {
     char algo;       /* 'g' Hong phase order or 'h' Slota colouring */
     int trim1, trim2;
-    int lanes;       /* lanes per frontier vertex, 1..64 */
+    int lanes;       /* 1, 2, 4, ... 64; checked and otherwise unused (a frontier's
+                        arcs are balanced over whole waves) */
     int block;       /* workgroup size: 256, 512 or 1024 */
     int autotuned;   /* 1: per size/degree bucket choices of scc_batch_autotune */
 } scc_batch_opts;
@@ -316,7 +317,7 @@ scc_status scc_batch_run(scc_ctx *ctx, const scc_batch_opts *opts, scc_batch_sta
 /* Baseline: one graph at a time through the single-graph engine with its
  * host-synchronised phase loop (the reference's style of driving). */
 scc_status scc_batch_run_serial(scc_ctx *ctx, const scc_opts *opts, scc_batch_stats *stats);
-/* Pick lanes, workgroup size and trim/colouring strategy per size and
+/* Pick the workgroup size and trim/colouring strategy per size and
  * degree bucket by timing each candidate on up to `sample` graphs of the
  * bucket in one launch; a text report of the choices goes to `report`
  * (may be NULL).  Labels of the uploaded batch are overwritten. */

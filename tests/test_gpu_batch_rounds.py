@@ -1,0 +1,64 @@
+"""The batched kernel's first round and list phases at the sizes and shapes
+where they change path: graphs at the edges of a chunk (64 vertices) and of
+the LDS tiers, with hubs walked by the whole workgroup, sparse enough to be
+trimmed and searched top-down only, dense enough for bottom-up levels, and
+with thousands of SCCs that the first round leaves to the list phases."""
+import numpy as np
+import pytest
+
+import detectingscc_amd as scc
+from oracle import pyoracle as orc
+from helpers import assert_same_labels, random_graph
+
+pytestmark = pytest.mark.gpu
+
+EDGES = (1, 2, 63, 64, 65, 127, 129, 2047, 2050, 4097, 8193, 65535, 65536, 65537)
+
+
+def _islands(V, rng):
+    """Disjoint cycles of 1 to 9 vertices over permuted ids, joined by arcs
+    from an island to a random later one: every cycle is an SCC."""
+    perm = rng.permutation(V) + 1
+    cuts = np.unique(np.concatenate([[0, V], np.cumsum(rng.integers(1, 10, V))]))
+    cuts = cuts[cuts <= V]
+    src, dst = [], []
+    for a, b in zip(cuts[:-1], cuts[1:]):
+        ring = perm[a:b]
+        if ring.size > 1:
+            src.append(ring)
+            dst.append(np.roll(ring, -1))
+    k = V // 4
+    a, b = rng.integers(0, V, k), rng.integers(0, V, k)
+    island = np.searchsorted(cuts, np.arange(V), side="right")
+    keep = island[a] < island[b]
+    src.append(perm[a[keep]])
+    dst.append(perm[b[keep]])
+    return scc.from_arcs(V, np.concatenate(src), np.concatenate(dst))
+
+
+def _hubs(V, rng):
+    """A third of the arcs leave, and a third enter, one of three vertices."""
+    E = 6 * V
+    src, dst = rng.integers(1, V + 1, E), rng.integers(1, V + 1, E)
+    src[:E // 3] = rng.integers(1, min(V, 3) + 1, E // 3)
+    dst[E // 3:2 * E // 3] = rng.integers(1, min(V, 3) + 1, E // 3)
+    return scc.from_arcs(V, src, dst)
+
+
+@pytest.mark.parametrize("block", [256, 512, 1024])
+@pytest.mark.parametrize("shape", ["islands", "hubs", "sparse", "dense"])
+def test_batch_first_round_and_lists(shape, block):
+    rng = np.random.default_rng([block, len(shape)])
+    make = {"islands": _islands, "hubs": _hubs, "sparse": lambda V, r: random_graph(V, 2 * V, r),
+            "dense": lambda V, r: random_graph(V, 9 * V, r)}[shape]
+    gs = [make(V, rng) for V in EDGES]
+    want = [orc.tarjan(g) for g in gs]
+    with scc.Context(0) as ctx:
+        ctx.batch_upload(scc.batch_from_graphs(gs))
+        for algo, t1, t2 in (("g", True, True), ("g", False, False), ("h", True, False), ("h", False, False)):
+            ctx.batch_run(algo=algo, trim1=t1, trim2=t2, lanes=16, block=block)
+            labs, nscc = ctx.batch_labels()
+            for i, (lab, n) in enumerate(want):
+                what = f"{shape} V={EDGES[i]} -a {algo} trims {t1:d}{t2:d} block {block}"
+                assert_same_labels(labs[i], lab, what)
+                assert nscc[i] == n, what
