@@ -36,6 +36,7 @@ class BatchEngine {
     scc_status launch(const std::vector<uint32_t> &idx, const std::vector<uint32_t> &cfg,
                       const std::vector<int> &block, double *ms, std::vector<double> *lat_ms,
                       uint32_t *launches);
+    bool packed_labels() const;   // the host layout has few words that are not labels
 
     int dev = 0;
     hipStream_t s1 = nullptr, stream2 = nullptr;
@@ -51,7 +52,17 @@ class BatchEngine {
     uint32_t capG = 0;
     uint64_t *m_voff = nullptr, *m_eoff = nullptr;
     uint32_t *m_V = nullptr, *m_Fr = nullptr, *m_Br = nullptr, *m_Fc = nullptr, *m_Bc = nullptr;
-    uint32_t *m_cfg = nullptr, *m_order = nullptr;
+    // launch input, one block (one copy per launch): 64 words of work-queue
+    // heads, then capG configuration words and capG processing-order entries
+    uint32_t *m_meta = nullptr;
+    // per-graph results, one block (one copy per run): start and end ticks
+    // and SCC counts of capG graphs
+    uint64_t *m_res = nullptr;
+    // page-locked host side of both blocks
+    uint32_t *h_meta = nullptr;
+    uint64_t *h_res = nullptr;
+    hipEvent_t ev[3] = {nullptr, nullptr, nullptr};   // start, end of each stream
+    int occ[3] = {0, 0, 0};                           // workgroups per CU at 1,024, 512 and 256 lanes
     std::vector<uint32_t> stage;        // host staging of the row arrays
     uint64_t nverts = 0, narcs = 0;
     double ticks_per_ms = 100000.0;

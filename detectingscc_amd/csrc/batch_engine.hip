@@ -31,6 +31,14 @@ void BatchEngine::release()
     for (void *p : allocs)
         if (p) (void)hipFree(p);
     allocs.clear();
+    if (h_meta) (void)hipHostFree(h_meta);
+    if (h_res) (void)hipHostFree(h_res);
+    h_meta = nullptr;
+    h_res = nullptr;
+    for (auto &e : ev) {
+        if (e) (void)hipEventDestroy(e);
+        e = nullptr;
+    }
     if (stream2) (void)hipStreamDestroy(stream2);
     stream2 = nullptr;
     d = BatchDev();
@@ -45,6 +53,8 @@ template <class T> static hipError_t balloc(std::vector<void *> &allocs, T **p, 
     if (e == hipSuccess) allocs.push_back(*p);
     return e;
 }
+
+constexpr uint32_t kHeads = 64;   // work-queue heads at the front of m_meta, 16 words apart per launch
 
 // Size/degree bucket of a graph (4 size classes x 3 degree classes).
 static int bucket_of(uint32_t V, uint32_t E)
@@ -65,6 +75,8 @@ scc_status BatchEngine::prepare(int device, hipStream_t stream, uint32_t ng, con
     s1 = stream;
     BHIP(hipSetDevice(device));
     if (!stream2) BHIP(hipStreamCreateWithFlags(&stream2, hipStreamNonBlocking));
+    for (auto &e : ev)
+        if (!e) BHIP(hipEventCreate(&e));
     ran = false;
     G = ng;
     V.assign(Vs, Vs + G);
@@ -110,12 +122,15 @@ scc_status BatchEngine::prepare(int device, hipStream_t stream, uint32_t ng, con
         chk(balloc(allocs, &d.piv, 3 * capS));
         chk(balloc(allocs, &d.q, 4 * capS));
         chk(balloc(allocs, &d.pivlist, capS));
-        chk(balloc(allocs, &m_cfg, capG));
-        chk(balloc(allocs, &m_order, capG));
-        chk(balloc(allocs, &d.nscc, capG));
-        chk(balloc(allocs, &d.tstart, capG));
-        chk(balloc(allocs, &d.tend, capG));
-        chk(balloc(allocs, &d.next, 64));
+        chk(balloc(allocs, &m_meta, kHeads + 2 * (size_t)capG));
+        chk(balloc(allocs, &m_res, 2 * (size_t)capG + (capG + 1) / 2));
+        if (h_meta) (void)hipHostFree(h_meta);
+        if (h_res) (void)hipHostFree(h_res);
+        h_meta = nullptr;
+        h_res = nullptr;
+        chk(hipHostMalloc((void **)&h_meta, sizeof(uint32_t) * (kHeads + 2 * (size_t)capG), hipHostMallocDefault));
+        chk(hipHostMalloc((void **)&h_res, sizeof(uint64_t) * (2 * (size_t)capG + (capG + 1) / 2),
+                          hipHostMallocDefault));
         if (e != hipSuccess) {
             (void)hipGetLastError();
             release();
@@ -141,8 +156,12 @@ scc_status BatchEngine::finish_upload()
     d.Br = m_Br;
     d.Fc = m_Fc;
     d.Bc = m_Bc;
-    d.cfg = m_cfg;
-    d.order = m_order;
+    d.next = m_meta;
+    d.cfg = m_meta + kHeads;
+    d.order = m_meta + kHeads + capG;
+    d.tstart = m_res;
+    d.tend = m_res + capG;
+    d.nscc = reinterpret_cast<uint32_t *>(m_res + 2 * (size_t)capG);
     bucket.resize(G);
     for (uint32_t i = 0; i < G; i++) bucket[i] = bucket_of(V[i], E[i]);
     int rate_khz = 0;
@@ -274,44 +293,44 @@ scc_status BatchEngine::launch(const std::vector<uint32_t> &idx, const std::vect
         groups.push_back({bs, {(uint32_t)order.size(), (uint32_t)mine.size()}});
         order.insert(order.end(), mine.begin(), mine.end());
     }
-    std::vector<uint32_t> cfg_all(G, 0);
-    for (uint32_t k = 0; k < idx.size(); k++) cfg_all[idx[k]] = cfg[k];
-    BHIP(hipMemcpyAsync(m_cfg, cfg_all.data(), sizeof(uint32_t) * G, hipMemcpyHostToDevice, s1));
-    BHIP(hipMemcpyAsync(m_order, order.data(), sizeof(uint32_t) * order.size(), hipMemcpyHostToDevice, s1));
-    BHIP(hipMemsetAsync(d.next, 0, 64 * sizeof(uint32_t), s1));
-    hipEvent_t e0, ea, eb;
-    BHIP(hipEventCreate(&e0));
-    BHIP(hipEventCreate(&ea));
-    BHIP(hipEventCreate(&eb));
-    BHIP(hipEventRecord(e0, s1));
-    BHIP(hipStreamWaitEvent(stream2, e0, 0));
+    // work-queue heads, configuration words and order in one copy
+    std::memset(h_meta, 0, sizeof(uint32_t) * (kHeads + (size_t)G));
+    for (uint32_t k = 0; k < idx.size(); k++) h_meta[kHeads + idx[k]] = cfg[k];
+    std::memcpy(h_meta + kHeads + capG, order.data(), sizeof(uint32_t) * order.size());
+    BHIP(hipMemcpyAsync(m_meta, h_meta, sizeof(uint32_t) * (kHeads + (size_t)capG + order.size()),
+                        hipMemcpyHostToDevice, s1));
+    const bool two = groups.size() > 1;
+    BHIP(hipEventRecord(ev[0], s1));
+    if (two) BHIP(hipStreamWaitEvent(stream2, ev[0], 0));
     uint32_t nl = 0;
     for (size_t gidx = 0; gidx < groups.size(); gidx++) {
         const int bs = groups[gidx].first;
         const uint32_t first = groups[gidx].second.first, count = groups[gidx].second.second;
         BatchDev bd = d;
         bd.next = d.next + 16 * gidx;      // own 64-byte-apart counter per group
-        const uint64_t slots = (uint64_t)num_cus * batch_occupancy(bs);
-        const uint32_t grid = (uint32_t)std::min<uint64_t>(count, slots);
+        int &per_cu = occ[bs == 1024 ? 0 : bs == 512 ? 1 : 2];
+        if (!per_cu) per_cu = batch_occupancy(bs);
+        const uint32_t grid = (uint32_t)std::min<uint64_t>(count, (uint64_t)num_cus * per_cu);
         k_batch(gidx % 2 ? stream2 : s1, bd, first, count, bs, grid);
         nl++;
     }
-    BHIP(hipEventRecord(ea, s1));
-    BHIP(hipEventRecord(eb, stream2));
-    BHIP(hipEventSynchronize(ea));
-    BHIP(hipEventSynchronize(eb));
+    BHIP(hipGetLastError());
+    BHIP(hipEventRecord(ev[1], s1));
+    if (two) {
+        BHIP(hipEventRecord(ev[2], stream2));
+        BHIP(hipStreamWaitEvent(s1, ev[2], 0));
+    }
+    if (lat_ms)   // ticks and counts of every graph in one copy
+        BHIP(hipMemcpyAsync(h_res, m_res, sizeof(uint64_t) * (2 * (size_t)capG + (G + 1) / 2), hipMemcpyDeviceToHost,
+                            s1));
+    BHIP(hipStreamSynchronize(s1));
     float ma = 0, mb = 0;
-    BHIP(hipEventElapsedTime(&ma, e0, ea));
-    BHIP(hipEventElapsedTime(&mb, e0, eb));
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(ea);
-    (void)hipEventDestroy(eb);
+    BHIP(hipEventElapsedTime(&ma, ev[0], ev[1]));
+    if (two) BHIP(hipEventElapsedTime(&mb, ev[0], ev[2]));
     if (ms) *ms = std::max(ma, mb);
     if (launches) *launches = nl;
     if (lat_ms) {
-        std::vector<uint64_t> ts(G), te(G);
-        BHIP(hipMemcpy(ts.data(), d.tstart, sizeof(uint64_t) * G, hipMemcpyDeviceToHost));
-        BHIP(hipMemcpy(te.data(), d.tend, sizeof(uint64_t) * G, hipMemcpyDeviceToHost));
+        const uint64_t *ts = h_res, *te = h_res + capG;
         uint64_t t0 = UINT64_MAX;
         for (uint32_t i : idx) t0 = std::min(t0, ts[i]);
         lat_ms->clear();
@@ -363,8 +382,7 @@ scc_status BatchEngine::run(const scc_batch_opts &o, scc_batch_stats *out)
     uint32_t nl = 0;
     scc_status s = launch(idx, cfg, blk, &ms, &lat, &nl);
     if (s != SCC_OK) return s;
-    std::vector<uint32_t> nscc(G);
-    BHIP(hipMemcpy(nscc.data(), d.nscc, sizeof(uint32_t) * G, hipMemcpyDeviceToHost));
+    const uint32_t *nscc = reinterpret_cast<const uint32_t *>(h_res + 2 * (size_t)capG);
     for (uint32_t i = 0; i < G; i++)
         if (nscc[i] == BATCH_ANOMALY)
             return fail(SCC_ERR_DEVICE, "graph %u: a class finished a round without a pivot", i);
@@ -479,11 +497,54 @@ scc_status BatchEngine::autotune(int sample, std::string *report)
     return SCC_OK;
 }
 
+// Labels of graph g (V+1 entries) from slot voff[g] to the host layout's
+// offset: one workgroup per graph.
+__global__ void batch_pack_kernel(const uint32_t *lab, const uint64_t *dvoff, const uint64_t *roff,
+                                  const uint32_t *Vn, uint32_t G, uint32_t *dst)
+{
+    for (uint32_t g = blockIdx.x; g < G; g += gridDim.x) {
+        const uint32_t *src = lab + dvoff[g];
+        uint32_t *to = dst + (roff[g] - roff[0]);
+        for (uint32_t i = threadIdx.x; i <= Vn[g]; i += blockDim.x) to[i] = src[i];
+    }
+}
+
+// Whether the labels leave as one copy: at most as many words between two
+// graphs' labels (one each in the layout of scc_gen_batch_mix) as labels.
+bool BatchEngine::packed_labels() const
+{
+    return row_off[G - 1] + V[G - 1] + 1 - row_off[0] <= 2 * (nverts + G);
+}
+
+// The labels go from the slots into the host layout on the device and leave
+// as one copy straight into the caller's buffer; the few words between two
+// graphs' labels, which are the caller's, are put back after it.  On the
+// 4,096-graph mix (190 MB of labels) 50 ms of a zeroed host vector, a
+// pageable copy into it and a second copy out of it -> 3.6 ms into a
+// page-locked buffer (the link's 56 GB/s and 0.1 ms for the pack).
 scc_status BatchEngine::labels(uint32_t *lab, uint32_t *nscc)
 {
     if (!ran) return fail(SCC_ERR_NOTREADY, "no completed batch run");
     BHIP(hipSetDevice(dev));
-    if (lab) {
+    if (lab && packed_labels()) {
+        // the queues are free between runs: 4 * capS words, of which the
+        // packed labels take at most 2 * (nverts + G) <= 2 * capS, then the offsets
+        uint32_t *packed = d.q;
+        uint64_t *d_roff = reinterpret_cast<uint64_t *>(d.q + 2 * capS);
+        const uint64_t words = row_off[G - 1] + V[G - 1] + 1 - row_off[0];
+        BHIP(hipMemcpyAsync(d_roff, row_off.data(), sizeof(uint64_t) * G, hipMemcpyHostToDevice, s1));
+        batch_pack_kernel<<<std::min<uint32_t>(G, 8192), 256, 0, s1>>>(d.lab, m_voff, d_roff, m_V, G, packed);
+        BHIP(hipGetLastError());
+        std::vector<uint32_t> gaps;
+        gaps.reserve(words - nverts - G);
+        for (uint32_t i = 0; i + 1 < G; i++)
+            gaps.insert(gaps.end(), lab + row_off[i] + V[i] + 1, lab + row_off[i + 1]);
+        BHIP(hipMemcpyAsync(lab + row_off[0], packed, sizeof(uint32_t) * words, hipMemcpyDeviceToHost, s1));
+        BHIP(hipStreamSynchronize(s1));
+        const uint32_t *gap = gaps.data();
+        for (uint32_t i = 0; i + 1 < G; i++)
+            for (uint64_t k = row_off[i] + V[i] + 1; k < row_off[i + 1]; k++) lab[k] = *gap++;
+    } else if (lab) {
         std::vector<uint32_t> all(voff[G]);
         BHIP(hipMemcpy(all.data(), d.lab, sizeof(uint32_t) * voff[G], hipMemcpyDeviceToHost));
         parallel_chunks(G, [&](uint64_t lo, uint64_t hi, int) {

@@ -62,3 +62,32 @@ def test_batch_first_round_and_lists(shape, block):
                 what = f"{shape} V={EDGES[i]} -a {algo} trims {t1:d}{t2:d} block {block}"
                 assert_same_labels(labs[i], lab, what)
                 assert nscc[i] == n, what
+
+
+@pytest.mark.parametrize("slack", [0, 7, 5000])
+def test_batch_labels_layout(slack):
+    """Labels land at the host layout's offsets whatever the distance between
+    two graphs' rows (one copy, or graph by graph where the gaps are wide),
+    and the words between them stay the caller's."""
+    rng = np.random.default_rng(slack)
+    gs = [random_graph(V, 3 * V, rng) for V in (1, 70, 2, 333, 64, 1000, 63)]
+    b = scc.batch_from_graphs(gs)
+    row = np.zeros(len(gs) + 1, np.uint64)
+    row[1:] = np.cumsum([g.V + 2 + slack for g in gs])
+    row += np.uint64(slack)
+    Fr, Br = np.zeros(int(row[-1]), np.uint32), np.zeros(int(row[-1]), np.uint32)
+    for i, g in enumerate(gs):
+        Fr[int(row[i]):int(row[i]) + g.V + 2] = g.Fr
+        Br[int(row[i]):int(row[i]) + g.V + 2] = g.Br
+    b = scc.Batch(b.V, b.E, row, b.col_off, Fr, b.Fc, Br, b.Bc)
+    lab = np.full(int(row[-1]), 0xABCD, np.uint32)
+    own = np.zeros(lab.size, bool)
+    with scc.Context(0) as ctx:
+        ctx.batch_upload(b)
+        ctx.batch_run()
+        assert scc.lib().scc_batch_labels(ctx._ctx, scc._p32(lab), None) == 0
+    for i, g in enumerate(gs):
+        at = int(row[i])
+        own[at:at + g.V + 1] = True
+        assert_same_labels(lab[at:at + g.V + 1], orc.tarjan(g)[0], f"slack {slack} graph {i}")
+    assert (lab[~own] == 0xABCD).all()
