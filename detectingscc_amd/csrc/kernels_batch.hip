@@ -71,6 +71,11 @@ __device__ __forceinline__ bool bbit(const uint32_t *bm, uint32_t v) { return (b
 constexpr uint32_t HUB_DEG = 512;
 constexpr uint32_t HUB_CAP = 128;
 
+// Levels of at most 64 frontier vertices and NARROW_ARCS arcs are run by one
+// wave per direction, without workgroup barriers and with the frontier in
+// LDS (g_narrow).
+constexpr uint32_t NARROW_ARCS = 256;
+
 // per-workgroup scratch in LDS
 struct Lds {
     uint32_t graph;
@@ -82,6 +87,8 @@ struct Lds {
     uint32_t red[2][16];
     unsigned long long key;
     uint32_t hub[HUB_CAP];    // vertex | direction << 31
+    uint32_t near[2][NARROW_ARCS];   // per direction, the frontier of a narrow level
+    uint32_t nlo[2];          // where the frontier begins in the queue after the narrow levels
 };
 
 // one graph's views
@@ -512,6 +519,87 @@ template <int BS, bool SINGLE> __device__ __forceinline__ void g_hubs(Lds &L, co
     }
 }
 
+// Top-down levels of direction d while they are narrow, by the calling wave
+// alone: the frontier is queue entries [lo, hi), hi - lo <= 64.  A level is
+// two dependent loads (rows, columns) and LDS work, about 1.5 us against 3 to
+// 4 us for a level of the whole workgroup with its barriers and queue in
+// global memory; the first and last levels of nearly every search, and all
+// of a long cycle's, are narrow.  Ends when the frontier is empty or no
+// longer narrow: L.tail[d] has then grown by the vertices claimed, and the
+// frontier is queue entries [L.nlo[d], L.tail[d]) (the entries of the levels
+// in between are not written; nothing reads them).
+template <bool SINGLE>
+__device__ __forceinline__ void g_narrow(Lds &L, const G1 &g, uint32_t d, uint32_t lo, uint32_t hi)
+{
+    const uint32_t *R = d ? g.Br : g.Fr, *C = d ? g.Bc : g.Fc;
+    uint32_t *vis = d ? g.bvis : g.fvis, *q = g.queue(2 * d), *near = L.near[d];
+    uint32_t n = hi - lo, tail = hi;
+    uint32_t v = ln() < n ? at(q, lo + ln()) : 0u;   // row 0 is empty
+    for (;;) {
+        const uint32_t b = at(R, v), deg = at(R, v + 1) - b;
+        const uint32_t c = SINGLE ? 0u : g.cls[v];
+        // any degree over the bound ends the loop before sums can wrap
+        uint32_t sum = min(deg, NARROW_ARCS + 1);
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t y = __shfl_up(sum, o);
+            if ((int)ln() >= o) sum += y;
+        }
+        const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)sum, 63);
+        if (total > NARROW_ARCS) break;
+        const uint32_t start = b - (sum - deg);
+        uint32_t m = 0;   // vertices claimed
+        for (uint32_t j0 = 0; j0 < total; j0 += 64) {
+            const uint32_t j = j0 + ln();
+            uint32_t own = 0;
+#pragma unroll
+            for (uint32_t o = 32; o >= 1; o >>= 1) own += (uint32_t)__shfl((int)sum, (int)(own + o - 1)) <= j ? o : 0u;
+            const uint32_t st = __shfl(start, (int)own), cx = SINGLE ? 0u : __shfl(c, (int)own);
+            uint32_t x = 0;
+            if (j < total) x = C[st + j];
+            const bool claimed = j < total && g_claim<SINGLE>(g, vis, x, cx);
+            const uint64_t mask = __ballot(claimed);
+            if (claimed) near[m + (uint32_t)__popcll(mask & ((1ull << ln()) - 1))] = x;
+            m += (uint32_t)__popcll(mask);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        tail += m;
+        n = m;
+        if (m > 64) {
+            for (uint32_t i = ln(); i < m; i += 64) put(q, tail - m + i, near[i]);
+            break;
+        }
+        if (m == 0) break;
+        v = ln() < m ? near[ln()] : 0u;
+        __builtin_amdgcn_wave_barrier();   // every entry is read before the next level's are written
+    }
+    if (n <= 64 && ln() < n) put(q, tail - n + ln(), v);
+    if (ln() == 0) {
+        L.tail[d] = tail;
+        L.nlo[d] = tail - n;
+    }
+}
+
+// The narrow levels of both directions, one wave each; returns false (and
+// does nothing) unless every direction left is narrow.
+template <int BS, bool SINGLE>
+__device__ __forceinline__ bool g_narrow_both(Lds &L, const G1 &g, uint32_t (&lo)[2], uint32_t (&hi)[2])
+{
+    if (hi[0] - lo[0] > 64 || hi[1] - lo[1] > 64) return false;
+    const uint32_t wv = uni(threadIdx.x >> 6);
+    if (wv < 2 && (wv ? hi[1] != lo[1] : hi[0] != lo[0]))
+        g_narrow<SINGLE>(L, g, wv, wv ? lo[1] : lo[0], wv ? hi[1] : hi[0]);
+    __syncthreads();
+    for (uint32_t d = 0; d < 2; d++) {
+        if (lo[d] == hi[d]) continue;
+        lo[d] = uni(L.nlo[d]);
+        hi[d] = uni(L.tail[d]);
+    }
+    __syncthreads();
+    return true;
+}
+
 // A bottom-up level of direction d: a live vertex not yet visited joins if
 // one of its parents is visited: its first parent, if trim-1 has left the
 // array of them (`first`), or one of its row.  A parent that joins in this same level may or may not
@@ -606,6 +694,10 @@ template <int BS> __device__ __forceinline__ void g_first_search(Lds &L, const G
     uint32_t lo[2] = {0, 0}, hi[2] = {1, 1}, prev[2] = {1, 1};
     bool bu[2] = {false, false};
     for (uint32_t level = 0; level <= g.V; level++) {   // each level claims a vertex or ends
+        if (!bu[0] && !bu[1] && g_narrow_both<BS, true>(L, g, lo, hi)) {
+            prev[0] = hi[0] - lo[0];
+            prev[1] = hi[1] - lo[1];
+        }
         if (lo[0] == hi[0] && lo[1] == hi[1]) break;
         g_both<BS>(lo, hi, [&](uint32_t d, uint32_t w, uint32_t nw) {
             if (d ? bu[1] : bu[0]) g_bottom_up(L, g, d, w, nw, first);
@@ -729,6 +821,7 @@ template <int BS> __device__ __forceinline__ void g_reach(Lds &L, const G1 &g, b
     uint32_t hi[2] = {uni(L.tail[0]), do_bw ? uni(L.tail[1]) : 0u};
     __syncthreads();
     for (uint32_t level = 0; level <= g.V; level++) {   // each level claims a vertex or ends
+        g_narrow_both<BS, false>(L, g, lo, hi);
         if (lo[0] == hi[0] && lo[1] == hi[1]) break;
         g_both<BS>(lo, hi, [&](uint32_t d, uint32_t w, uint32_t nw) {
             g_expand<false>(L, g, d, d ? lo[1] : lo[0], d ? hi[1] : hi[0], w, nw);
@@ -1114,8 +1207,11 @@ template <> struct BTier<256> {
     static constexpr uint32_t cls_words = (1u << 11) + 2;
 };
 
+// At least four waves per SIMD (128 vector registers): a second 512-lane
+// workgroup then fits a CU (mix at 512 lanes 2.54 -> 1.67 ms); 1,024 lanes
+// need as many anyway, 256 lanes do not change.
 template <int BS>
-__global__ __launch_bounds__(BS) void batch_scc_kernel(BatchDev B, uint32_t first, uint32_t count)
+__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) void batch_scc_kernel(BatchDev B, uint32_t first, uint32_t count)
 {
     __shared__ Lds L;
     __shared__ uint32_t s_bits[3][BTier<BS>::words];
