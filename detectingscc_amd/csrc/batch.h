@@ -35,4 +35,17 @@ void k_batch(hipStream_t s, const BatchDev &B, uint32_t first, uint32_t count, i
 // workgroups per CU that fit at the given block size
 int batch_occupancy(int block);
 
+// One resident graph in one workgroup (the single-graph engine's path for
+// small graphs).  lab and aux hold V+1 words (lab[0] is written too), piv
+// 3(V+1)+3, pivlist V+1, q 4(V+2); results go to the counter lines of the
+// mapped buffer `pub`, its sequence word (line C_COUNT) last.
+constexpr uint32_t SMALL_V = 16384, SMALL_E = 1u << 18;
+struct SmallArgs {
+    uint32_t V, E, cfg, seq;
+    const uint32_t *Fr, *Fc, *Br, *Bc;
+    uint32_t *lab, *aux, *pivlist, *q, *pub;
+    uint64_t *piv;
+};
+void k_small(hipStream_t s, const SmallArgs &a);
+
 } // namespace sccamd

@@ -91,6 +91,7 @@ class Engine {
                            bool use_live_bits = false, bool lazy = false);
     scc_status min_label();
     scc_status color_loop(int expand, int W, scc_stats *stats);
+    scc_status run_small(char algo, bool trim1, bool trim2, scc_stats *stats);
     scc_status detect_phases(const scc_opts &o, int expand, int W, scc_stats *stats, bool local_only);
     struct DevBuf {
         void *p = nullptr;
@@ -119,6 +120,8 @@ class Engine {
     size_t nmarks = 0;
     int first_reach_marks[2] = {-1, -1};
     uint32_t num_parts = 0;
+    uint32_t *small_q = nullptr;       // the small-graph kernel's queues
+    double ticks_per_ms = 100000.0;    // device wall clock
     DevBuf buf[16];                    // detectSCC scratch (lazily sized)
     std::unique_ptr<Engine> sub;       // engine for the quotient graph
 };

@@ -19,6 +19,7 @@
 
 #include <algorithm>
 
+#include "batch.h"
 #include "engine.h"
 #include "host_util.h"
 #include "merge.h"
@@ -60,6 +61,8 @@ void Engine::release()
         b = DevBuf();
     }
     sub.reset();
+    f(small_q);
+    small_q = nullptr;
     if (h_ctr) (void)hipHostFree(h_ctr);
     if (h_pub) (void)hipHostFree(h_pub);
     h_pub = nullptr;
@@ -109,6 +112,10 @@ scc_status Engine::init(int dev)
         (void)hipGetLastError();
         h_pub = nullptr;
     }
+    HIP_TRY(hipMalloc((void **)&small_q, 4 * (SMALL_V + 2) * sizeof(uint32_t)));
+    int rate_khz = 0;
+    if (hipDeviceGetAttribute(&rate_khz, hipDeviceAttributeWallClockRate, dev) == hipSuccess && rate_khz > 0)
+        ticks_per_ms = (double)rate_khz;
     // diagnostic: SCC_TRACE_LEVELS=1 prints every host decision of a search
     const char *tr = std::getenv("SCC_TRACE_LEVELS");
     trace_levels = tr && tr[0] == '1';
@@ -872,6 +879,17 @@ scc_status Engine::run(const scc_opts &o, scc_stats *out)
 
     scc_stats stats;
     std::memset(&stats, 0, sizeof stats);
+    // A small graph in one launch: where nothing asks for the device-wide
+    // engine's per-phase times, search counts or mappings (batch.h has the
+    // sizes, small_scc_kernel the reason for them).
+    if (A != 'd' && expand == SCC_EXPAND_DO && !o.sizes && !o.phase_times && g.V && g.V <= SMALL_V &&
+        g.E <= SMALL_E && h_pub) {
+        scc_status ss = run_small(A, o.trim1 != 0, o.trim2 != 0, &stats);
+        if (ss != SCC_OK) return ss;
+        ran = true;
+        if (out) *out = stats;
+        return SCC_OK;
+    }
     nmarks = 0;
     first_reach_marks[0] = first_reach_marks[1] = -1;
     mark(-1);
@@ -960,6 +978,44 @@ scc_status Engine::run(const scc_opts &o, scc_stats *out)
     for (int k = 0; k < 8; k++) stats.first_work[k] = u64(C_WORK + k);
     ran = true;
     if (out) *out = stats;
+    return SCC_OK;
+}
+
+// The whole decomposition as one launch of one workgroup; the device times
+// come from the kernel's own clock reads.
+scc_status Engine::run_small(char algo, bool trim1, bool trim2, scc_stats *stats)
+{
+    SmallArgs a;
+    a.V = g.V;
+    a.E = g.E;
+    a.cfg = batch_cfg(trim1, trim2, algo == 'h' || algo == 'y');
+    a.seq = ++pub_seq;
+    a.Fr = g.Fr;
+    a.Fc = g.Fc;
+    a.Br = g.Br;
+    a.Bc = g.Bc;
+    a.lab = st.lab;
+    a.aux = st.aux;
+    a.pivlist = st.pivlist;
+    a.q = small_q;
+    a.pub = d_pub + (a.seq & 1) * kPubBuffer;
+    a.piv = st.piv;
+    k_small(stream, a);
+    scc_status s = wait_ctr(a.seq);
+    if (s != SCC_OK) return s;
+    if (h_ctr[CT(C_ANOM)]) return fail(SCC_ERR_DEVICE, "internal invariant violated: a class without a pivot");
+    auto ms = [&](int i) {
+        return (double)((uint64_t)h_ctr[CT(i)] | ((uint64_t)h_ctr[CT(i) + 1] << 32)) / ticks_per_ms;
+    };
+    stats->num_sccs = h_ctr[CT(C_NSCC)];
+    stats->num_trim1 = h_ctr[CT(C_TRIM1)];
+    stats->num_trim2 = h_ctr[CT(C_TRIM2)];
+    stats->num_pivot = h_ctr[CT(C_PIVOT)];
+    stats->first_pivot = h_ctr[CT(C_PIV0)];
+    stats->rounds = h_ctr[CT(C_NPIV)];
+    stats->levels = h_ctr[CT(C_NLEVELS)];
+    stats->ms_scc = ms(C_FWV);
+    stats->ms_first_reach = ms(C_BWV);
     return SCC_OK;
 }
 

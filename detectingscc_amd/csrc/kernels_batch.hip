@@ -76,6 +76,12 @@ constexpr uint32_t HUB_CAP = 128;
 // LDS (g_narrow).
 constexpr uint32_t NARROW_ARCS = 256;
 
+// what a graph's run counted (scc_stats has the meanings)
+struct GraphStats {
+    uint32_t trim1, trim2, pivots, first_pivot, rounds, levels;
+    uint64_t search_ticks;   // the first search, wall clock
+};
+
 // per-workgroup scratch in LDS
 struct Lds {
     uint32_t graph;
@@ -89,6 +95,8 @@ struct Lds {
     uint32_t hub[HUB_CAP];    // vertex | direction << 31
     uint32_t near[2][NARROW_ARCS];   // per direction, the frontier of a narrow level
     uint32_t nlo[2];          // where the frontier begins in the queue after the narrow levels
+    uint32_t nlev[2];         // and how many there were
+    GraphStats st;            // written by thread 0
 };
 
 // one graph's views
@@ -533,7 +541,7 @@ __device__ __forceinline__ void g_narrow(Lds &L, const G1 &g, uint32_t d, uint32
 {
     const uint32_t *R = d ? g.Br : g.Fr, *C = d ? g.Bc : g.Fc;
     uint32_t *vis = d ? g.bvis : g.fvis, *q = g.queue(2 * d), *near = L.near[d];
-    uint32_t n = hi - lo, tail = hi;
+    uint32_t n = hi - lo, tail = hi, levels = 0;
     uint32_t v = ln() < n ? at(q, lo + ln()) : 0u;   // row 0 is empty
     for (;;) {
         const uint32_t b = at(R, v), deg = at(R, v + 1) - b;
@@ -566,6 +574,7 @@ __device__ __forceinline__ void g_narrow(Lds &L, const G1 &g, uint32_t d, uint32
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         tail += m;
         n = m;
+        levels++;
         if (m > 64) {
             for (uint32_t i = ln(); i < m; i += 64) put(q, tail - m + i, near[i]);
             break;
@@ -578,6 +587,7 @@ __device__ __forceinline__ void g_narrow(Lds &L, const G1 &g, uint32_t d, uint32
     if (ln() == 0) {
         L.tail[d] = tail;
         L.nlo[d] = tail - n;
+        L.nlev[d] = levels;
     }
 }
 
@@ -591,11 +601,14 @@ __device__ __forceinline__ bool g_narrow_both(Lds &L, const G1 &g, uint32_t (&lo
     if (wv < 2 && (wv ? hi[1] != lo[1] : hi[0] != lo[0]))
         g_narrow<SINGLE>(L, g, wv, wv ? lo[1] : lo[0], wv ? hi[1] : hi[0]);
     __syncthreads();
+    uint32_t levels = 0;
     for (uint32_t d = 0; d < 2; d++) {
         if (lo[d] == hi[d]) continue;
         lo[d] = uni(L.nlo[d]);
         hi[d] = uni(L.tail[d]);
+        levels = max(levels, uni(L.nlev[d]));
     }
+    if (threadIdx.x == 0) L.st.levels += levels;
     __syncthreads();
     return true;
 }
@@ -699,6 +712,7 @@ template <int BS> __device__ __forceinline__ void g_first_search(Lds &L, const G
             prev[1] = hi[1] - lo[1];
         }
         if (lo[0] == hi[0] && lo[1] == hi[1]) break;
+        if (threadIdx.x == 0) L.st.levels++;
         g_both<BS>(lo, hi, [&](uint32_t d, uint32_t w, uint32_t nw) {
             if (d ? bu[1] : bu[0]) g_bottom_up(L, g, d, w, nw, first);
             else g_expand<true>(L, g, d, d ? lo[1] : lo[0], d ? hi[1] : hi[0], w, nw);
@@ -751,7 +765,9 @@ template <int BS> __device__ __forceinline__ void g_trim1(Lds &L, const G1 &g, u
                 removed++;
             }
         }
-        if (!wg_sum<BS>(L, removed, pass & 1)) break;
+        const uint32_t n1 = wg_sum<BS>(L, removed, pass & 1);
+        if (!n1) break;
+        if (threadIdx.x == 0) L.st.trim1 += n1;
     }
     __syncthreads();
 }
@@ -777,7 +793,7 @@ __device__ __forceinline__ bool g_arc(const uint32_t *R, const uint32_t *C, uint
 }
 
 // trim-2 (scc_kernels.cu:236-357), claim by CAS on the smaller id
-template <int BS> __device__ __forceinline__ void g_trim2(const G1 &g, uint32_t n)
+template <int BS> __device__ __forceinline__ void g_trim2(Lds &L, const G1 &g, uint32_t n)
 {
     const uint32_t *list = g.list();
     LIST_LOOP(v)
@@ -795,6 +811,7 @@ template <int BS> __device__ __forceinline__ void g_trim2(const G1 &g, uint32_t 
         if (hit) {
             const uint32_t lo = v < k ? v : k, hi = v < k ? k : v;
             if (atomicCAS(&g.cls[lo], c, DEAD) == c) {
+                atomicAdd(&L.st.trim2, 1u);
                 g.lab[lo] = lo | LAB_FINAL;
                 g.lab[hi] = lo | LAB_FINAL;
                 __hip_atomic_store(&g.cls[hi], DEAD, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -823,6 +840,7 @@ template <int BS> __device__ __forceinline__ void g_reach(Lds &L, const G1 &g, b
     for (uint32_t level = 0; level <= g.V; level++) {   // each level claims a vertex or ends
         g_narrow_both<BS, false>(L, g, lo, hi);
         if (lo[0] == hi[0] && lo[1] == hi[1]) break;
+        if (threadIdx.x == 0) L.st.levels++;
         g_both<BS>(lo, hi, [&](uint32_t d, uint32_t w, uint32_t nw) {
             g_expand<false>(L, g, d, d ? lo[1] : lo[0], d ? hi[1] : hi[0], w, nw);
         });
@@ -888,6 +906,7 @@ template <int BS> __device__ __forceinline__ void g_pivots(Lds &L, const G1 &g, 
     if (threadIdx.x == 0) {
         L.tail[0] = np;
         L.tail[1] = np;
+        L.st.pivots += np;   // each finds its SCC
     }
     __syncthreads();
 }
@@ -1013,6 +1032,10 @@ template <int BS> __device__ __forceinline__ void g_color_loop(Lds &L, const G1 
             lpush(root, v, g.queue(0), &L.tail[0]);
         }
         __syncthreads();
+        if (threadIdx.x == 0) {
+            L.st.pivots += L.tail[0];   // each root finds its SCC
+            L.st.rounds++;
+        }
         g_reach<BS>(L, g, false);
         uint32_t lv = 0;
         LIST_LOOP(v)
@@ -1087,6 +1110,7 @@ template <int BS> __device__ __forceinline__ uint32_t g_solve(Lds &L, const G1 &
         L.nhub = 0;
         L.nact = 0;
         L.anom = 0;
+        L.st = GraphStats();
     }
     __syncthreads();
     const uint32_t ndeg = g_degrees<BS>(L, g, cfg_t1(cfg));
@@ -1128,7 +1152,13 @@ template <int BS> __device__ __forceinline__ uint32_t g_solve(Lds &L, const G1 &
             L.tail[1] = 1;
         }
         __syncthreads();
+        const uint64_t t0 = wall_clock64();
         g_first_search<BS>(L, g, nlive, first, g.E >= BU_DEGREE * (uint64_t)g.V);
+        if (threadIdx.x == 0) {
+            L.st.search_ticks = wall_clock64() - t0;
+            L.st.first_pivot = p0;
+            L.st.pivots = 1;
+        }
     }
     // the pivot's SCC: its size, its smallest vertex
     uint32_t members = 0, least = DEAD;
@@ -1139,6 +1169,7 @@ template <int BS> __device__ __forceinline__ uint32_t g_solve(Lds &L, const G1 &
     }
     const uint32_t nmem = wg_sum1<BS>(L, members), root = wg_min1<BS>(L, least);
     const uint32_t singles = g.V - nlive;   // trim-1's
+    if (threadIdx.x == 0) L.st.trim1 = singles;
     if (nmem == nlive) {
         for (uint32_t v = threadIdx.x; v <= g.V; v += BS) g.lab[v] = bbit(g.live, v) ? root : v;
         return singles + (nmem ? 1u : 0u);
@@ -1164,7 +1195,7 @@ template <int BS> __device__ __forceinline__ uint32_t g_solve(Lds &L, const G1 &
     if (!slota) {
         if (cfg_t1(cfg)) g_trim1<BS>(L, g, n);
         if (cfg_t2(cfg)) {
-            g_trim2<BS>(g, n);
+            g_trim2<BS>(L, g, n);
             if (cfg_t1(cfg)) g_trim1<BS>(L, g, n);
         }
         g_minlabel<BS>(L, g, n);
@@ -1174,6 +1205,7 @@ template <int BS> __device__ __forceinline__ uint32_t g_solve(Lds &L, const G1 &
             g_pivots<BS>(L, g, n);
             g_reach<BS>(L, g, true);
             if (!g_update<BS>(L, g, n)) break;
+            if (threadIdx.x == 0) L.st.rounds++;
         }
     } else {
         g_color_loop<BS>(L, g, n);
@@ -1264,6 +1296,89 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) void ba
         }
     }
 }
+
+// ------------------------------------------------ one small graph ---
+// A resident graph of at most SMALL_V vertices and SMALL_E arcs as one
+// launch of one workgroup, instead of the device-wide engine's chain of
+// about 17 launches and two looks at the counters (100 to 150 us on graphs
+// of this size, 300 and more where the first round leaves vertices).  Where
+// the whole CSR and the work arrays fit LDS they are copied there first, so
+// a level's dependent loads are LDS reads.  The counters the host waits for
+// are written to its mapped memory by the kernel itself.
+// Whole calls, one workgroup against the device-wide engine, at 2, 4, 8 and
+// 16 arcs per vertex: 1,000 vertices 57 / 45 / 34 / 31 us against 120 / 112 /
+// 123 / 98, 8,000 vertices 128 / 99 / 83 / 56 against 407 / 134 / 116 / 107,
+// 16,384 vertices 190 / 150 / 103 / 87 against 388 / 149 / 121 / 108; at
+// 32,768 vertices it would be 250 against 148 at 4 arcs.
+constexpr uint32_t SMALL_LDS = 36864;   // words: class words, or everything of a graph that fits
+
+__global__ __launch_bounds__(1024) void small_scc_kernel(SmallArgs a)
+{
+    __shared__ Lds L;
+    __shared__ uint32_t s_bits[3][2 * ((SMALL_V + 64) / 64)];
+    __shared__ uint32_t s_mem[SMALL_LDS];
+    static_assert(SMALL_V + 1 <= SMALL_LDS, "the class words fit");
+    const uint64_t t0 = wall_clock64();
+    G1 g;
+    g.V = a.V;
+    g.E = a.E;
+    g.lab = a.lab;
+    g.piv = a.piv;
+    g.pivlist = a.pivlist;
+    g.live = s_bits[0];
+    g.fvis = s_bits[1];
+    g.bvis = s_bits[2];
+    g.cls = s_mem;
+    uint32_t n;
+    const uint64_t nr = (uint64_t)a.V + 2;
+    if (8 * nr + 2 * (uint64_t)a.E <= SMALL_LDS) {
+        uint32_t *Fr = s_mem + nr, *Br = Fr + nr, *Fc = Br + nr, *Bc = Fc + a.E;
+        g.aux = Bc + a.E;
+        g.q = g.aux + nr;   // 4 * nr words
+        for (uint32_t i = threadIdx.x; i < nr; i += 1024) {
+            Fr[i] = a.Fr[i];
+            Br[i] = a.Br[i];
+        }
+        for (uint32_t i = threadIdx.x; i < a.E; i += 1024) {
+            Fc[i] = a.Fc[i];
+            Bc[i] = a.Bc[i];
+        }
+        g.Fr = Fr;
+        g.Br = Br;
+        g.Fc = Fc;
+        g.Bc = Bc;
+        __syncthreads();
+        n = g_solve<1024>(L, g, a.cfg);
+    } else {
+        g.Fr = a.Fr;
+        g.Br = a.Br;
+        g.Fc = a.Fc;
+        g.Bc = a.Bc;
+        g.aux = a.aux;
+        g.q = a.q;
+        n = g_solve<1024>(L, g, a.cfg);
+    }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    uint32_t *p = a.pub;
+    p[CT(C_NSCC)] = n;
+    p[CT(C_TRIM1)] = L.st.trim1;
+    p[CT(C_TRIM2)] = L.st.trim2;
+    p[CT(C_PIVOT)] = L.st.pivots;
+    p[CT(C_PIV0)] = L.st.first_pivot;
+    p[CT(C_ANOM)] = L.anom;
+    p[CT(C_NPIV)] = L.st.rounds;
+    p[CT(C_NLEVELS)] = L.st.levels;
+    const uint64_t all = wall_clock64() - t0, search = L.st.search_ticks;
+    p[CT(C_FWV)] = (uint32_t)all;
+    p[CT(C_FWV) + 1] = (uint32_t)(all >> 32);
+    p[CT(C_BWV)] = (uint32_t)search;
+    p[CT(C_BWV) + 1] = (uint32_t)(search >> 32);
+    __threadfence_system();
+    __hip_atomic_store(p + CT(C_COUNT), a.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+void k_small(hipStream_t s, const SmallArgs &a) { small_scc_kernel<<<1, 1024, 0, s>>>(a); }
 
 uint32_t batch_cfg(bool trim1, bool trim2, bool slota)
 {
