@@ -67,7 +67,13 @@ class Engine {
     void collect_times(scc_stats *s);
     uint32_t bpd(int W) const;
     scc_status reach(bool fw, bool bw, bool single, int expand, int W, uint32_t *levels_out);
-    scc_status reach_do(bool fw, bool bw, bool single, uint32_t *levels_out);
+    // with `done`: gives up (*done = false) once max_levels levels have run
+    // and the search has not ended
+    scc_status reach_do(bool fw, bool bw, bool single, uint32_t *levels_out, uint32_t max_levels = 0,
+                        bool *done = nullptr);
+    scc_status merge_quotient(const uint32_t *tbits, scc_stats *stats, const uint32_t **qid_out,
+                              const uint32_t **rep_out, const uint32_t **qlab_out);
+    scc_status merge_search(uint32_t *tbits, scc_stats *stats, bool *found, uint32_t *left);
     DirArgs dir_args(int d, uint32_t level) const;
     // single: every live vertex has class 0 (the first trim of a
     // decomposition); none_dead: besides, the state is fresh (no vertex dead,

@@ -556,7 +556,7 @@ static constexpr int kSpecLevels = 16;
 static constexpr int64_t kSpecGrowth = 8;
 static constexpr int64_t kSpecRise = 2;
 
-scc_status Engine::reach_do(bool fw, bool bw, bool single, uint32_t *levels_out)
+scc_status Engine::reach_do(bool fw, bool bw, bool single, uint32_t *levels_out, uint32_t max_levels, bool *done)
 {
     int dirs[2], nd = 0;   // argument position -> direction
     if (fw) dirs[nd++] = 0;
@@ -637,6 +637,13 @@ scc_status Engine::reach_do(bool fw, bool bw, bool single, uint32_t *levels_out)
             // a window queued meanwhile runs as no-ops; its counters are
             // published into the other buffer, which nothing waits for
             if (levels_out) *levels_out += end + h_ctr[CT(C_NLEVELS)] + h_ctr[CT(C_NLEVELS) + 1];
+            if (done) *done = true;
+            return SCC_OK;
+        }
+        if (done && seen >= max_levels) {
+            // levels queued ahead still run, on state that nothing reads
+            if (levels_out) *levels_out += seen;
+            *done = false;
             return SCC_OK;
         }
         // every level claims at least one vertex, so V+1 levels bound a search
@@ -1039,8 +1046,7 @@ scc_status Engine::detect_phases(const scc_opts &o, int expand, int W, scc_stats
     // live bitmap from the class words, and it tests neighbours in the bitmap
     if (o.trim1 && (s = trim1(true, true)) != SCC_OK) return s;
     mark(SCC_PHASE_LOCAL);
-    const size_t nv = (size_t)g.V + 1;
-    uint32_t *tbits, *isrep, *qid, *rep, *cout, *cin, *Qr, *QBr, *tiles;
+    uint32_t *tbits;
     if ((s = scratch(buf[0], st.nwords, &tbits)) != SCC_OK) return s;
     k_local_init(stream, g, st, tbits);
     uint32_t live = 0;
@@ -1053,12 +1059,54 @@ scc_status Engine::detect_phases(const scc_opts &o, int expand, int W, scc_stats
     k_canon(stream, g, st, false);
     if (local_only) return SCC_OK;
     mark(SCC_PHASE_MERGE);
+    // the SCC across most partitions first, then the quotient of what is left
+    bool found = false;
+    uint32_t left = 0;
+    if ((s = merge_search(tbits, stats, &found, &left)) != SCC_OK) return s;
+    const uint32_t *qlab = nullptr, *qid = nullptr, *rep = nullptr;
+    if ((!found || left) && (s = merge_quotient(tbits, stats, &qid, &rep, &qlab)) != SCC_OK) return s;
+    zero_ctr(C_NSCC, 1);
+    k_q_map(stream, g, st, found ? live_bits() : nullptr, tbits, qid, qlab, rep);
+    return SCC_OK;
+}
+
+// FW and BW from one pivot over the vertices of the local phase, classes
+// ignored.  A search that has not ended after kMergeLevels levels is given up
+// (a high-diameter graph, whose quotient graph is the shorter way).
+static constexpr uint32_t kMergeLevels = 16;
+
+scc_status Engine::merge_search(uint32_t *tbits, scc_stats *stats, bool *found, uint32_t *left)
+{
+    k_merge_live(stream, g, tbits, live_bits());
+    init_vis(true, true);
+    const bool counted = search_stats;
+    search_stats = false;   // the work units are those of a first search
+    scc_status s = reach_do(true, true, true, &stats->levels, kMergeLevels, found);
+    search_stats = counted;
+    if (s != SCC_OK || !*found) return s;
+    zero_ctr(C_LIVE, 1);
+    k_merge_giant(stream, g, st, live_bits(), tbits);
+    if ((s = read_ctr()) != SCC_OK) return s;
+    *left = h_ctr[CT(C_LIVE)];
+    return SCC_OK;
+}
+
+// The quotient graph of the local SCCs of the vertices not in tbits and its
+// SCCs: qid (local SCC of each representative), rep (its vertex) and the
+// labels of the quotient vertices (null: no arcs between them).
+scc_status Engine::merge_quotient(const uint32_t *tbits, scc_stats *stats, const uint32_t **qid_out,
+                                  const uint32_t **rep_out, const uint32_t **qlab_out)
+{
+    scc_status s;
+    const size_t nv = (size_t)g.V + 1;
+    uint32_t *isrep, *qid, *rep, *Qr, *QBr, *tiles;
     if ((s = scratch(buf[1], nv, &isrep)) != SCC_OK || (s = scratch(buf[2], nv, &qid)) != SCC_OK ||
-        (s = scratch(buf[3], nv, &rep)) != SCC_OK || (s = scratch(buf[4], nv + 1, &cout)) != SCC_OK ||
-        (s = scratch(buf[5], nv + 1, &cin)) != SCC_OK || (s = scratch(buf[6], nv + 1, &Qr)) != SCC_OK ||
+        (s = scratch(buf[3], nv, &rep)) != SCC_OK || (s = scratch(buf[6], nv + 1, &Qr)) != SCC_OK ||
         (s = scratch(buf[7], nv + 1, &QBr)) != SCC_OK ||
         (s = scratch(buf[8], scan_tile_count(nv + 1), &tiles)) != SCC_OK)
         return s;
+    *qid_out = qid;
+    *rep_out = rep;
     k_q_mark(stream, g, st, tbits, isrep);
     k_exscan(stream, isrep, qid, nv, tiles);
     uint32_t last[2];
@@ -1066,7 +1114,6 @@ scc_status Engine::detect_phases(const scc_opts &o, int expand, int W, scc_stats
     HIP_TRY(hipMemcpyAsync(&last[1], isrep + g.V, 4, hipMemcpyDeviceToHost, stream));
     HIP_TRY(hipStreamSynchronize(stream));
     const uint32_t QV = last[0] + last[1];
-    const uint32_t *qlab = nullptr;
     if (QV) {
         // quotient arcs as sorted 64-bit keys: each vertex's quotient id,
         // the keys of the arcs between different local SCCs, and two radix
@@ -1121,12 +1168,13 @@ scc_status Engine::detect_phases(const scc_opts &o, int expand, int W, scc_stats
             so.sizes = 0;
             scc_stats sst;
             if ((s = sub->run(so, &sst)) != SCC_OK) return s;
-            qlab = sub->st.lab;
+            // its labels are read on this engine's stream: a small graph's
+            // counters arrive before its kernel has ended
+            HIP_TRY(hipStreamSynchronize(sub->stream));
+            *qlab_out = sub->st.lab;
             stats->levels += sst.levels;
         }
     }
-    zero_ctr(C_NSCC, 1);
-    k_q_map(stream, g, st, tbits, qid, qlab, rep);
     return SCC_OK;
 }
 

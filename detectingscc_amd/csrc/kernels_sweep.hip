@@ -1104,6 +1104,66 @@ void k_update_words(hipStream_t s, const DevGraph &g, DevState &st, const uint32
                                                             g.V, st.aux);
 }
 
+// detectSCC's merge: the vertices that took part in the local phase (not in
+// tbits) as a live bitmap.
+__global__ void merge_live_kernel(const uint32_t *__restrict__ tbits, uint32_t *live, uint32_t V)
+{
+    const uint32_t ngroups = (V >> 5) + 1;
+    for (uint32_t gi = blockIdx.x * blockDim.x + threadIdx.x; gi < ngroups; gi += gridDim.x * blockDim.x) {
+        const uint32_t in = gi + 1 < ngroups ? ~0u : ~0u >> (31 - (V & 31));   // vertices past V are none
+        live[gi] = ~tbits[gi] & in;                                             // vertex 0 is in tbits
+    }
+}
+
+void k_merge_live(hipStream_t s, const DevGraph &g, const uint32_t *tbits, uint32_t *live)
+{
+    merge_live_kernel<<<sweep_blocks(g.V >> 5), SWEEP_BLOCK, 0, s>>>(tbits, live, g.V);
+}
+
+// After the merge's search: the pivot's SCC (live, visited both ways) joins
+// tbits, `live` keeps it alone, its smallest vertex goes to scc_min[pivot],
+// and the vertices left are counted in C_LIVE.
+__global__ __launch_bounds__(256) void merge_giant_kernel(const uint32_t *__restrict__ fvis,
+                                                          const uint32_t *__restrict__ bvis, uint32_t *live,
+                                                          uint32_t *tbits, uint32_t *ctr, uint32_t V,
+                                                          uint32_t *scc_min)
+{
+    uint32_t left = 0, mmin = DEAD;
+    const uint32_t ngroups = (V >> 5) + 1;
+    for (uint32_t gi = blockIdx.x * blockDim.x + threadIdx.x; gi < ngroups; gi += gridDim.x * blockDim.x) {
+        const uint32_t lw = live[gi], tb = tbits[gi];
+        const uint32_t f = fvis[2 * gi], b = bvis[2 * gi];
+        const uint32_t member = lw & f & b;
+        left += (uint32_t)__popc(lw & ~member);
+        if (member) {
+            const uint32_t m = (gi << 5) + (uint32_t)(__ffs(member) - 1);
+            mmin = m < mmin ? m : mmin;
+            tbits[gi] = tb | member;
+        }
+        live[gi] = member;
+    }
+    spread_add32(ctr, C_LIVE, left);
+    __shared__ uint32_t s_min[4];
+    for (int o = 32; o > 0; o >>= 1) {
+        const uint32_t x = __shfl_xor(mmin, o);
+        mmin = x < mmin ? x : mmin;
+    }
+    if (lane() == 0) s_min[threadIdx.x >> 6] = mmin;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    for (uint32_t w = 1; w < 4; w++) mmin = s_min[w] < mmin ? s_min[w] : mmin;
+    const uint32_t p0 = ctr[CT(C_PIV0)];
+    if (mmin != DEAD && p0 >= 1 && p0 <= V &&
+        mmin < __hip_atomic_load(&scc_min[p0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMin(&scc_min[p0], mmin);
+}
+
+void k_merge_giant(hipStream_t s, const DevGraph &g, DevState &st, uint32_t *live, uint32_t *tbits)
+{
+    merge_giant_kernel<<<sweep_blocks(g.V >> 5), SWEEP_BLOCK, 0, s>>>(st.fvis, st.bvis, live, tbits, st.ctr, g.V,
+                                                                      st.aux);
+}
+
 // Members of the first pivot's SCC after a lazy first round: visited by
 // both searches and not finished when the bitmaps were initialised (each
 // bitmap's second word per group holds the finished bits).
