@@ -1045,6 +1045,18 @@ scc_status Engine::detect_phases(const scc_opts &o, int expand, int W, scc_stats
     // second fixpoint runs single-class too: its first pass rebuilds the
     // live bitmap from the class words, and it tests neighbours in the bitmap
     if (o.trim1 && (s = trim1(true, true)) != SCC_OK) return s;
+    // Most graphs that are partitioned have one SCC across most partitions:
+    // it is searched for first, over all the vertices, and the local SCCs and
+    // the quotient graph are those of what it leaves, often nothing
+    bool found = false;
+    uint32_t left = 0;
+    if (!local_only) {
+        mark(SCC_PHASE_MERGE);
+        if (!o.trim1) k_live_bits(stream, g, st, live_bits());   // else exact from the second fixpoint
+        if ((s = detect_search(stats, &found, &left)) != SCC_OK) return s;
+        if (found) k_detect_members(stream, g, st, live_bits(), left == 0);
+        if (found && !left) return SCC_OK;
+    }
     mark(SCC_PHASE_LOCAL);
     uint32_t *tbits;
     if ((s = scratch(buf[0], st.nwords, &tbits)) != SCC_OK) return s;
@@ -1059,33 +1071,29 @@ scc_status Engine::detect_phases(const scc_opts &o, int expand, int W, scc_stats
     k_canon(stream, g, st, false);
     if (local_only) return SCC_OK;
     mark(SCC_PHASE_MERGE);
-    // the SCC across most partitions first, then the quotient of what is left
-    bool found = false;
-    uint32_t left = 0;
-    if ((s = merge_search(tbits, stats, &found, &left)) != SCC_OK) return s;
     const uint32_t *qlab = nullptr, *qid = nullptr, *rep = nullptr;
-    if ((!found || left) && (s = merge_quotient(tbits, stats, &qid, &rep, &qlab)) != SCC_OK) return s;
+    if ((s = merge_quotient(tbits, stats, &qid, &rep, &qlab)) != SCC_OK) return s;
     zero_ctr(C_NSCC, 1);
-    k_q_map(stream, g, st, found ? live_bits() : nullptr, tbits, qid, qlab, rep);
+    k_q_map(stream, g, st, tbits, qid, qlab, rep);
     return SCC_OK;
 }
 
-// FW and BW from one pivot over the vertices of the local phase, classes
-// ignored.  A search that has not ended after kMergeLevels levels is given up
-// (a high-diameter graph, whose quotient graph is the shorter way).
-static constexpr uint32_t kMergeLevels = 16;
+// FW and BW from one pivot over every live vertex (classes ignored; they are
+// all still in class 0), in the live bitmap.  A search that has not ended
+// after kDetectLevels levels is given up: on a high-diameter graph the local
+// SCCs and their quotient graph are the shorter way.
+static constexpr uint32_t kDetectLevels = 16;
 
-scc_status Engine::merge_search(uint32_t *tbits, scc_stats *stats, bool *found, uint32_t *left)
+scc_status Engine::detect_search(scc_stats *stats, bool *found, uint32_t *left)
 {
-    k_merge_live(stream, g, tbits, live_bits());
     init_vis(true, true);
     const bool counted = search_stats;
     search_stats = false;   // the work units are those of a first search
-    scc_status s = reach_do(true, true, true, &stats->levels, kMergeLevels, found);
+    scc_status s = reach_do(true, true, true, &stats->levels, kDetectLevels, found);
     search_stats = counted;
     if (s != SCC_OK || !*found) return s;
     zero_ctr(C_LIVE, 1);
-    k_merge_giant(stream, g, st, live_bits(), tbits);
+    k_detect_found(stream, g, st, live_bits());
     if ((s = read_ctr()) != SCC_OK) return s;
     *left = h_ctr[CT(C_LIVE)];
     return SCC_OK;

@@ -10,12 +10,12 @@
 // global SCCs.  This replaces the reference's host set-intersection merge
 // (scc_WCC.cu:1276-1531, defect D7), which is not correct in general.
 //
-// Most graphs that are partitioned have one SCC across most partitions, so
-// the merge first searches for it over the vertices themselves (FW and BW
-// from one pivot, direction-optimised: it reads few of the arcs, while the
-// quotient graph needs the quotient ids at both ends of every arc, one random
-// read each) and builds the quotient of what is left, often nothing.  8.4M
-// vertices, 100M arcs, 200 communities: merge 2.4 -> 0.5 ms.
+// The SCC across most partitions, where there is one, does not come this way:
+// the engine searches for it first (FW and BW from one pivot over all live
+// vertices, direction-optimised: it reads few of the arcs, while the quotient
+// graph needs the quotient ids at both ends of every arc, one random read
+// each), and only what it leaves goes through the local phase and the
+// quotient graph.
 //
 // Quotient vertex ids are assigned in increasing order of the local SCC's
 // minimum vertex id, so the minimum quotient id of a quotient SCC maps back
@@ -306,20 +306,15 @@ __global__ void q_rep_kernel(const uint32_t *__restrict__ isrep, const uint32_t 
         if (isrep[v]) rep[qid[v]] = v;
 }
 
-// global label = minimum vertex of the quotient SCC's minimum local SCC, or
-// the minimum of the merge search's SCC for its members
-__global__ void q_map_kernel(uint32_t *lab, const uint32_t *__restrict__ members, const uint32_t *__restrict__ aux,
-                             const uint32_t *__restrict__ tbits, const uint32_t *__restrict__ qid,
-                             const uint32_t *__restrict__ qlab, const uint32_t *__restrict__ rep, uint32_t *ctr,
-                             uint32_t V)
+// global label = minimum vertex of the quotient SCC's minimum local SCC
+__global__ void q_map_kernel(uint32_t *lab, const uint32_t *__restrict__ tbits,
+                             const uint32_t *__restrict__ qid, const uint32_t *__restrict__ qlab,
+                             const uint32_t *__restrict__ rep, uint32_t *ctr, uint32_t V)
 {
-    const uint32_t p0 = ctr[CT(C_PIV0)];
-    const uint32_t root = members && p0 >= 1 && p0 <= V ? aux[p0] : 0u;
     uint32_t roots = 0;
     for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x + 1; v <= V; v += gridDim.x * blockDim.x) {
         uint32_t l = lab[v];
-        if (members && tbit(members, v)) l = root;
-        else if (qlab && !tbit(tbits, v)) l = rep[qlab[qid[l] + 1] - 1];
+        if (!tbit(tbits, v) && qlab) l = rep[qlab[qid[l] + 1] - 1];
         lab[v] = l;
         roots += l == v;
     }
@@ -371,10 +366,10 @@ void k_q_rep(hipStream_t s, const DevGraph &g, const uint32_t *isrep, const uint
     q_rep_kernel<<<grid_for(g.V), 256, 0, s>>>(isrep, qid, rep, g.V);
 }
 
-void k_q_map(hipStream_t s, const DevGraph &g, DevState &st, const uint32_t *members, const uint32_t *tbits,
-             const uint32_t *qid, const uint32_t *qlab, const uint32_t *rep)
+void k_q_map(hipStream_t s, const DevGraph &g, DevState &st, const uint32_t *tbits, const uint32_t *qid,
+             const uint32_t *qlab, const uint32_t *rep)
 {
-    q_map_kernel<<<grid_for(g.V), 256, 0, s>>>(st.lab, members, st.aux, tbits, qid, qlab, rep, st.ctr, g.V);
+    q_map_kernel<<<grid_for(g.V), 256, 0, s>>>(st.lab, tbits, qid, qlab, rep, st.ctr, g.V);
 }
 
 } // namespace sccamd

@@ -7,6 +7,7 @@
 #include <algorithm>
 
 #include "lds_queue.h"
+#include "merge.h"
 #include "scc_dev.h"
 
 namespace sccamd {
@@ -457,6 +458,11 @@ __global__ void live_bits_kernel(const uint32_t *__restrict__ cls, uint32_t *liv
     }
 }
 
+void k_live_bits(hipStream_t s, const DevGraph &g, const DevState &st, uint32_t *live)
+{
+    live_bits_kernel<<<sweep_blocks(g.V), SWEEP_BLOCK, 0, s>>>(st.cls, live, g.V);
+}
+
 void k_trim1(hipStream_t s, const DevGraph &g, DevState &st, const uint32_t *in, uint32_t *out,
              uint32_t epoch, uint32_t pass, uint32_t sweep_share, uint32_t *live, bool degree_first, bool labels)
 {
@@ -466,8 +472,7 @@ void k_trim1(hipStream_t s, const DevGraph &g, DevState &st, const uint32_t *in,
                                                                       st.cls, st.lab, live, g.V, st.ctr, out,
                                                                       cap, labels ? 1 : 0);
     } else if (live) {
-        if (pass == 0)
-            live_bits_kernel<<<sweep_blocks(g.V), SWEEP_BLOCK, 0, s>>>(st.cls, live, g.V);
+        if (pass == 0) k_live_bits(s, g, st, live);
         trim1_kernel<true><<<sweep_blocks(g.V), SWEEP_BLOCK, 0, s>>>(g.Fr, g.Fc, g.Br, g.Bc, g.F1, g.B1, st.cls,
                                                                      st.lab,
                                                                      live, g.V, st.ctr, in, out, st.stamp,
@@ -1104,41 +1109,22 @@ void k_update_words(hipStream_t s, const DevGraph &g, DevState &st, const uint32
                                                             g.V, st.aux);
 }
 
-// detectSCC's merge: the vertices that took part in the local phase (not in
-// tbits) as a live bitmap.
-__global__ void merge_live_kernel(const uint32_t *__restrict__ tbits, uint32_t *live, uint32_t V)
-{
-    const uint32_t ngroups = (V >> 5) + 1;
-    for (uint32_t gi = blockIdx.x * blockDim.x + threadIdx.x; gi < ngroups; gi += gridDim.x * blockDim.x) {
-        const uint32_t in = gi + 1 < ngroups ? ~0u : ~0u >> (31 - (V & 31));   // vertices past V are none
-        live[gi] = ~tbits[gi] & in;                                             // vertex 0 is in tbits
-    }
-}
-
-void k_merge_live(hipStream_t s, const DevGraph &g, const uint32_t *tbits, uint32_t *live)
-{
-    merge_live_kernel<<<sweep_blocks(g.V >> 5), SWEEP_BLOCK, 0, s>>>(tbits, live, g.V);
-}
-
-// After the merge's search: the pivot's SCC (live, visited both ways) joins
-// tbits, `live` keeps it alone, its smallest vertex goes to scc_min[pivot],
-// and the vertices left are counted in C_LIVE.
-__global__ __launch_bounds__(256) void merge_giant_kernel(const uint32_t *__restrict__ fvis,
-                                                          const uint32_t *__restrict__ bvis, uint32_t *live,
-                                                          uint32_t *tbits, uint32_t *ctr, uint32_t V,
-                                                          uint32_t *scc_min)
+// After detectSCC's search over all live vertices: the pivot's SCC (live,
+// visited both ways) is left alone in `live`, its smallest vertex goes to
+// scc_min[pivot], and the other live vertices are counted in C_LIVE.
+__global__ __launch_bounds__(256) void detect_found_kernel(const uint32_t *__restrict__ fvis,
+                                                           const uint32_t *__restrict__ bvis, uint32_t *live,
+                                                           uint32_t *ctr, uint32_t V, uint32_t *scc_min)
 {
     uint32_t left = 0, mmin = DEAD;
     const uint32_t ngroups = (V >> 5) + 1;
     for (uint32_t gi = blockIdx.x * blockDim.x + threadIdx.x; gi < ngroups; gi += gridDim.x * blockDim.x) {
-        const uint32_t lw = live[gi], tb = tbits[gi];
-        const uint32_t f = fvis[2 * gi], b = bvis[2 * gi];
+        const uint32_t lw = live[gi], f = fvis[2 * gi], b = bvis[2 * gi];
         const uint32_t member = lw & f & b;
         left += (uint32_t)__popc(lw & ~member);
         if (member) {
             const uint32_t m = (gi << 5) + (uint32_t)(__ffs(member) - 1);
             mmin = m < mmin ? m : mmin;
-            tbits[gi] = tb | member;
         }
         live[gi] = member;
     }
@@ -1153,15 +1139,51 @@ __global__ __launch_bounds__(256) void merge_giant_kernel(const uint32_t *__rest
     if (threadIdx.x != 0) return;
     for (uint32_t w = 1; w < 4; w++) mmin = s_min[w] < mmin ? s_min[w] : mmin;
     const uint32_t p0 = ctr[CT(C_PIV0)];
-    if (mmin != DEAD && p0 >= 1 && p0 <= V &&
-        mmin < __hip_atomic_load(&scc_min[p0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+    if (p0 < 1 || p0 > V) return;
+    if (blockIdx.x == 0) atomicAdd(&ctr[CT(C_PIVOT)], 1u);
+    if (mmin != DEAD && mmin < __hip_atomic_load(&scc_min[p0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
         atomicMin(&scc_min[p0], mmin);
 }
 
-void k_merge_giant(hipStream_t s, const DevGraph &g, DevState &st, uint32_t *live, uint32_t *tbits)
+void k_detect_found(hipStream_t s, const DevGraph &g, DevState &st, uint32_t *live)
 {
-    merge_giant_kernel<<<sweep_blocks(g.V >> 5), SWEEP_BLOCK, 0, s>>>(st.fvis, st.bvis, live, tbits, st.ctr, g.V,
-                                                                      st.aux);
+    detect_found_kernel<<<sweep_blocks(g.V >> 5), SWEEP_BLOCK, 0, s>>>(st.fvis, st.bvis, live, st.ctr, g.V, st.aux);
+}
+
+// The labels of that SCC's members.  ALL (nothing else is live): its smallest
+// vertex, every other label (final, from the trims) without its flag, and
+// the SCCs counted; otherwise the pivot, and the members are finished.
+template <bool ALL>
+__global__ __launch_bounds__(256) void detect_members_kernel(uint32_t *lab, uint32_t *cls,
+                                                             const uint32_t *__restrict__ members,
+                                                             const uint32_t *__restrict__ aux, uint32_t *ctr,
+                                                             uint32_t V)
+{
+    const uint32_t p0 = ctr[CT(C_PIV0)];
+    const uint32_t root = p0 >= 1 && p0 <= V ? (ALL ? aux[p0] : p0) : 0u;   // 0: no members
+    uint32_t roots = 0;
+    for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x + 1; v <= V; v += gridDim.x * blockDim.x) {
+        const bool member = (members[v >> 5] >> (v & 31)) & 1u;
+        if (ALL) {
+            const uint32_t r = member ? root : lab[v] & ~LAB_FINAL;
+            lab[v] = r;
+            roots += r == v;
+        } else if (member) {
+            lab[v] = root;
+            cls[v] = DEAD;
+        }
+    }
+    if (ALL) spread_add32(ctr, C_NSCC, roots);
+}
+
+void k_detect_members(hipStream_t s, const DevGraph &g, DevState &st, const uint32_t *members, bool all)
+{
+    if (all)
+        detect_members_kernel<true><<<sweep_blocks(g.V), SWEEP_BLOCK, 0, s>>>(st.lab, st.cls, members, st.aux, st.ctr,
+                                                                              g.V);
+    else
+        detect_members_kernel<false><<<sweep_blocks(g.V), SWEEP_BLOCK, 0, s>>>(st.lab, st.cls, members, st.aux,
+                                                                               st.ctr, g.V);
 }
 
 // Members of the first pivot's SCC after a lazy first round: visited by

@@ -34,15 +34,16 @@ void k_q_keys(hipStream_t s, bool emit, const DevGraph &g, const uint32_t *qv, u
 size_t csr_sort_bytes(uint32_t V, uint64_t n);
 scc_status csr_from_keys(hipStream_t st, uint32_t V, uint64_t n, uint64_t *keys, uint64_t *out, void *tmp,
                          size_t tmp_bytes, uint32_t *R, uint32_t *C, uint32_t *RB, uint32_t *CB);
-// The merge's own search (engine.hip): its live bitmap from tbits, and after
-// it the pivot's SCC into tbits and alone into `live`, its smallest vertex in
-// aux[pivot], the vertices left in C_LIVE (kernels_sweep.hip).
-void k_merge_live(hipStream_t s, const DevGraph &g, const uint32_t *tbits, uint32_t *live);
-void k_merge_giant(hipStream_t s, const DevGraph &g, DevState &st, uint32_t *live, uint32_t *tbits);
-// members (may be null): vertices whose label is the merge search's SCC's
-// smallest vertex; the others are mapped through the quotient labels (qlab
-// null: kept)
-void k_q_map(hipStream_t s, const DevGraph &g, DevState &st, const uint32_t *members, const uint32_t *tbits,
-             const uint32_t *qid, const uint32_t *qlab, const uint32_t *rep);
+// detectSCC's search over every live vertex (engine.hip): after it,
+// k_detect_found leaves the pivot's SCC alone in the live bitmap, its
+// smallest vertex in aux[pivot] and the vertices left in C_LIVE; then
+// k_detect_members labels it.  With `all` nothing else is live: every label
+// is written in its final form and the SCCs are counted; otherwise its
+// members get the pivot as their label and are finished (kernels_sweep.hip).
+void k_live_bits(hipStream_t s, const DevGraph &g, const DevState &st, uint32_t *live);
+void k_detect_found(hipStream_t s, const DevGraph &g, DevState &st, uint32_t *live);
+void k_detect_members(hipStream_t s, const DevGraph &g, DevState &st, const uint32_t *members, bool all);
+void k_q_map(hipStream_t s, const DevGraph &g, DevState &st, const uint32_t *tbits, const uint32_t *qid,
+             const uint32_t *qlab, const uint32_t *rep);
 
 } // namespace sccamd

@@ -1,5 +1,5 @@
-"""detectSCC's merge: its own search for the SCC across the partitions, and
-the quotient graph of what that leaves or of everything."""
+"""detectSCC: its search for the SCC across the partitions, and the local SCCs
+and quotient graph of what that leaves or of everything."""
 import numpy as np
 import pytest
 
@@ -35,8 +35,8 @@ def _rings(k, size, joined, rng):
                                            (4000, 5, 3900)])
 @pytest.mark.parametrize("trims", [True, False])
 def test_merge_shapes(k, size, joined, trims):
-    """All in one SCC, most, none, and a long cycle of rings (a search the
-    merge gives up); partitions that split the rings and that join them."""
+    """All in one SCC, most, none, and a long cycle of rings (a search that
+    is given up); partitions that split the rings and that join them."""
     rng = np.random.default_rng(k + size)
     g = _rings(k, size, joined, rng)
     want, n = orc.tarjan(g)
