@@ -128,6 +128,11 @@ class Engine {
     uint32_t num_parts = 0;
     uint32_t *small_q = nullptr;       // the small-graph kernel's queues
     double ticks_per_ms = 100000.0;    // device wall clock
+    bool deg_known = false;            // this decomposition's degree pass has set C_DEG4 if it is to be set
+    bool low_denied = false;           // no memory for the low-degree rows
+    bool low_rows_ok() const;
+    uint4 *low_rows();
+    DevBuf low_buf;                    // low-degree rows of both directions (lazily sized)
     DevBuf buf[16];                    // detectSCC scratch (lazily sized)
     std::unique_ptr<Engine> sub;       // engine for the quotient graph
 };

@@ -832,6 +832,165 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_sgpr(80))) void expa
 }
 
 // ---------------------------------------------------------------------
+// Low-degree graphs (no vertex of more than LOW_DEG arcs one way: grids,
+// meshes, cycles, chains) with a high-diameter search.  Its thousands of
+// narrow levels are a chain of dependent memory trips, and a hop's time is
+// their latency: the rest of the chip waits.  So a hop is cut to one trip:
+// the rows are copied once into arrays of one 16-byte entry per vertex and
+// direction, and a claimed vertex's arcs load beside its claim, where a
+// top-down level's continuation hop reads columns, then claims and row
+// offsets, between workgroup barriers.  Here each wave goes on alone from
+// the vertices it claims, an arc per lane, its frontier in LDS, for
+// LOW_HOPS hops; what it claims past LOW_KEEP vertices, and after the last
+// hop, goes to the next level's queue.  Every vertex is claimed once, and
+// reachability does not depend on the order.  On MI355X a hop takes 0.5 us
+// on a cycle (both directions; 1.25 before: a 20,000-vertex cycle 25 -> 10
+// ms) and 0.75 us on the 4096^2 grid, whose rows come from HBM (2.1 before;
+// run 21.7 -> 9.4 ms).  64 or 256 hops and 8 or 16 vertices per wave at the
+// start are within 5% of these; keeping 32 to 128 vertices per wave, with
+// two or four steps per hop, made the grid 6% slower.
+constexpr uint32_t LOW_HOPS = 128;
+constexpr uint32_t LOW_PER = 4;                 // frontier vertices per wave, as long as there are waves
+constexpr uint32_t LOW_KEEP = 64 / LOW_DEG;     // frontier entries a wave keeps from hop to hop: an arc per lane
+constexpr uint32_t LOW_WQ = 256;                // entries of a wave's queue for the next level
+
+__global__ void low_rows_kernel(const uint32_t *__restrict__ Fr, const uint32_t *__restrict__ Fc,
+                                const uint32_t *__restrict__ Br, const uint32_t *__restrict__ Bc, uint4 *AF,
+                                uint4 *AB, uint32_t V)
+{
+    for (uint64_t v = 1 + blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v <= V; v += gridDim.x * blockDim.x) {
+        const uint32_t fb = Fr[v], fn = Fr[v + 1] - fb, bb = Br[v], bn = Br[v + 1] - bb;
+        uint32_t f[LOW_DEG] = {}, b[LOW_DEG] = {};
+#pragma unroll
+        for (uint32_t k = 0; k < LOW_DEG; k++) {
+            if (k < fn) f[k] = Fc[fb + k];
+            if (k < bn) b[k] = Bc[bb + k];
+        }
+        AF[v] = make_uint4(f[0], f[1], f[2], f[3]);
+        AB[v] = make_uint4(b[0], b[1], b[2], b[3]);
+    }
+}
+
+void k_low_rows(hipStream_t s, const DevGraph &g, uint4 *AF, uint4 *AB)
+{
+    const uint64_t b = ((uint64_t)g.V + 255) / 256;
+    low_rows_kernel<<<(uint32_t)(b > 8192 ? 8192 : b), 256, 0, s>>>(g.Fr, g.Fc, g.Br, g.Bc, AF, AB, g.V);
+}
+
+// (a native vector: an array of HIP's uint4 structs goes to scratch memory)
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// A value that is the same in every lane of the wave.
+__device__ __forceinline__ uint32_t uniform(uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); }
+
+template <bool COUNT>
+__global__ __launch_bounds__(256) void expand_low_kernel(DoArgs a, uint32_t bpd)
+{
+    __shared__ u32x4 s_arc[4][2][LOW_KEEP];
+    __shared__ uint32_t s_vtx[4][2][LOW_KEEP];
+    __shared__ uint32_t s_q[4][LOW_WQ];
+    __shared__ uint32_t s_pre[kSpread + 2];
+    int dir;
+    uint32_t bid;
+    split_dirs(a.ndirs, bpd, dir, bid);
+    const DirArgs &D = a.d[dir];
+    const int L = a.level;
+    // the level's state and input, as in expand_do_kernel; a direction that
+    // was bottom-up goes on top-down from what its last level visited
+    DirState st = load_dir_state(a.ctr, (L - 1) & 1, dir);
+    const bool slotted = st.mode == DIR_BU;
+    uint32_t n;
+    if (slotted) {
+        seg_prefix(&D.cnt[CT(L % 3)], &D.cslot[CT((L % 3) * kSpread)], a.qcap, s_pre);
+        n = s_pre[kSpread + 1];
+    } else {
+        n = D.cnt[CT(L % 3)];
+    }
+    st = dir_decide(st, n, (uint32_t)(*D.pbigc >> 32), a.ctr[CT(C_NLIVE)], (uint32_t)L, false);
+    if (st.mode == DIR_BU) st.mode = DIR_TD;
+    if (bid == 0) {
+        if (threadIdx.x == 0) store_dir_state(a.ctr, L & 1, dir, st);
+        if (st.mode == DIR_TD) {
+            seg_clear(&D.cnt[CT((L + 2) % 3)], &D.cslot[CT(((L + 2) % 3) * kSpread)]);
+            if (threadIdx.x == 0) *D.bigc_zero = 0ull;
+        }
+    }
+    if (st.mode != DIR_TD || n == 0) return;
+    const u32x4 *__restrict__ A = reinterpret_cast<const u32x4 *>(a.A[dir]);
+    uint32_t *const vis = D.vis;
+    uint32_t *cnt_out = &D.cnt[CT((L + 1) % 3)];
+    const uint32_t wv = uniform(threadIdx.x >> 6), lane = wlane();
+    uint32_t *wq = s_q[wv];
+    uint32_t nq = 0;
+    WorkCount wc;
+    const uint32_t waves = bpd * 4;
+    n = uniform(n);
+    const uint32_t per = min(LOW_KEEP, max(LOW_PER, (n + waves - 1) / waves));
+    for (uint32_t t = (bid * 4 + wv) * per; t < n; t += waves * per) {
+        uint32_t m = min(per, n - t), cur = 0;
+        if (lane < m) {
+            const uint32_t v = D.qin[slotted ? seg_pos(s_pre, t + lane, a.qcap) : t + lane];
+            s_vtx[wv][0][lane] = v;
+            s_arc[wv][0][lane] = A[v];
+        }
+        wave_sync();
+        for (uint32_t hop = 0; hop < LOW_HOPS; hop++) {
+            m = uniform(m);
+            cur = uniform(cur);
+            if (m == 0) break;
+            if (nq + 64 - LOW_KEEP > LOW_WQ) wave_flush(wq, nq, cnt_out, D.qout);
+            const uint32_t x = s_arc[wv][cur][lane / LOW_DEG][lane % LOW_DEG];
+            const uint32_t w = lane < m * LOW_DEG ? x : 0u, bit = w ? 1u << (w & 31) : 0u;
+            uint32_t old = 0;
+            u32x4 row = {0, 0, 0, 0};
+            if (w) {
+                old = atomicOr(&vis[vword(w)], bit);
+                row = A[w];
+            }
+            // what is computed from the claim stays behind the row load (the
+            // compiler otherwise moves it, with its wait, before the load)
+            asm volatile("" : "+v"(old));
+            const bool claimed = bit & ~old;
+            if (COUNT) {
+                wc.n[W_TDV] += lane < m;
+                wc.n[W_TDE] += bit != 0;
+                wc.n[W_CLAIM] += claimed;
+            }
+            const uint64_t mask = __ballot(claimed);
+            if (claimed) {
+                const uint32_t at = (uint32_t)__popcll(mask & ((1ull << lane) - 1));
+                if (at < LOW_KEEP) {
+                    s_vtx[wv][cur ^ 1][at] = w;
+                    s_arc[wv][cur ^ 1][at] = row;
+                } else {
+                    wq[nq + at - LOW_KEEP] = w;
+                }
+            }
+            m = (uint32_t)__popcll(mask);
+            if (m > LOW_KEEP) {
+                nq += m - LOW_KEEP;
+                m = LOW_KEEP;
+            }
+            cur ^= 1;
+            wave_sync();
+        }
+        if (nq + LOW_KEEP > LOW_WQ) wave_flush(wq, nq, cnt_out, D.qout);
+        wave_push(wq, nq, lane < m, lane < m ? s_vtx[wv][cur][lane] : 0u);
+        wave_sync();
+    }
+    wave_flush_block(wq, nq, cnt_out, D.qout);
+    if (COUNT) add_work(a.ctr, wc);
+}
+
+void k_low_level(hipStream_t s, const DoArgs &a, uint32_t bpd)
+{
+    bpd = dir_blocks(bpd, a.ndirs);
+    const uint32_t grid = bpd * (uint32_t)a.ndirs;
+    if (a.count) expand_low_kernel<true><<<grid, 256, 0, s>>>(a, bpd);
+    else expand_low_kernel<false><<<grid, 256, 0, s>>>(a, bpd);
+}
+
+// ---------------------------------------------------------------------
 // Narrow frontiers: many top-down levels inside one workgroup per direction.
 // A high-diameter graph (the 4096 x 4096 grid: 8,193 levels, frontiers of
 // a few thousand vertices) pays a launch and a chain of global round trips

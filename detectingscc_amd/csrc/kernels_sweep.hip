@@ -386,6 +386,7 @@ __global__ __launch_bounds__(256) void trim1_degree_kernel(const uint32_t *__res
     const uint32_t wv = threadIdx.x >> 6;
     uint32_t *wq = s_q[wv];
     uint32_t nq = 0, removed = 0;
+    bool big = false;   // a vertex of more than LOW_DEG arcs one way
     const uint32_t slot = blockIdx.x % kSpread;
     uint32_t *cnt_out = &ctr[CSLOT(C_TLIST + 1, slot)];
     uint32_t *qout = out + (size_t)slot * cap;
@@ -413,6 +414,7 @@ __global__ __launch_bounds__(256) void trim1_degree_kernel(const uint32_t *__res
             // 0: no out-arc or no in-arc (vertex 0, the dummy, has neither)
             const uint64_t p = (uint64_t)(fe[h] - fb[h]) * (uint64_t)(be[h] - bb[h]);
             dp[h] = p > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)p;
+            big |= fe[h] - fb[h] > LOW_DEG || be[h] - bb[h] > LOW_DEG;
             f1[h] = 0;
             b1[h] = 0;
             if (v[h] >= 1 && dp[h]) {
@@ -443,6 +445,7 @@ __global__ __launch_bounds__(256) void trim1_degree_kernel(const uint32_t *__res
         }
     }
     wave_flush_block(wq, nq, cnt_out, qout, cap, anom);
+    if (__syncthreads_or(big) && threadIdx.x == 0) ctr[CT(C_DEG4)] = 1;
     spread_add32(ctr, C_TRIM1, removed);
 }
 

@@ -31,6 +31,7 @@ constexpr uint32_t DEAD = 0xFFFFFFFFu;
 constexpr uint32_t LAB_FINAL = 0x80000000u;
 constexpr int SWEEP_BLOCK = 256;
 constexpr uint32_t LB_BIG = 512;   // degree from which a frontier vertex is a hub (LB mode)
+constexpr uint32_t LOW_DEG = 4;    // most arcs per vertex and direction of a low-degree graph (k_low_rows)
 constexpr uint32_t VIS_BLOCKS = 4096;   // most workgroups of the bitmap initialisation
 
 // Visited bitmaps (fvis, bvis) keep two words per group of 32 vertices: the
@@ -64,6 +65,7 @@ enum : int {
     C_BIGF = 22,     // 3 rotating 64-bit packed (items, chunks) counts of the FW hub lists (22..24)
     C_BIGB = 25,     // same for BW (25..27)
     C_NLEVELS = 28,  // levels run by the narrow-frontier kernel, word 0 FW, word 1 BW
+    C_DEG4 = 29,     // set if a vertex has more than LOW_DEG out- or in-arcs
     C_PIV0 = 30,     // first pivot of the latest election
     C_ANOM = 31,     // invariant violations caught by kernel guards (must stay 0)
     C_NLIVE = 32,    // live vertices when the visited bitmaps were initialised
@@ -207,6 +209,7 @@ struct DoArgs {
     int ndirs;
     int level;
     int bu_ok;                       // 0 on a grid too small for a bottom-up pass: stay top-down
+    const uint4 *A[2];               // low-degree levels: each vertex's arcs in this direction (0: none)
     uint32_t qcap;                   // slot region of a bottom-up level's queue: slot_cap(V, full grid)
     int count;                       // 1: add the level's work units (WorkCount) to C_WORK..C_WORK+7
 };
@@ -434,6 +437,11 @@ void k_do_level(hipStream_t s, const DoArgs &a, bool single_class, uint32_t bloc
 // leaving that level's input rewritten; a no-op unless that level would run
 // top-down from a small frontier with no hubs pending.  narrow_cap(): the
 // largest frontier the host starts it on
+// Rows of a low-degree graph: A[v] = the up to LOW_DEG entries of v's row,
+// zeros after them (V + 1 rows).
+void k_low_rows(hipStream_t s, const DevGraph &g, uint4 *AF, uint4 *AB);
+// A top-down level of a single-class search on a low-degree graph.
+void k_low_level(hipStream_t s, const DoArgs &a, uint32_t blocks_per_dir);
 void k_narrow_levels(hipStream_t s, const DoArgs &a, bool single_class);
 uint32_t narrow_cap();
 uint32_t do_blocks(uint32_t V, int ndirs);
