@@ -20,7 +20,7 @@ class Engine {
     ~Engine();
     scc_status init(int device);
     // `checked`: the caller has already validated the arrays (the server's
-    // submit does), so the host pass over them is skipped
+    // submit does), so they are not checked again
     scc_status upload(uint32_t V, uint32_t E, const uint32_t *Fr, const uint32_t *Fc,
                       const uint32_t *Br, const uint32_t *Bc, bool checked = false);
     scc_status upload_partition(const uint32_t *part);
@@ -56,6 +56,10 @@ class Engine {
   private:
     void release();
     scc_status reserve(uint32_t V, uint32_t E);
+    bool fits(uint32_t V, uint32_t E) const;
+    bool spare_set();
+    void drop_spare();
+    DevGraph spare;                    // a second set of Fr, Fc, Br, Bc (lazily made, see upload)
     scc_status read_ctr();                 // publish_ctr + wait_ctr
     uint32_t publish_ctr();                // queue a publication of the counters, returns its number
     scc_status wait_ctr(uint32_t seq);     // wait for publication `seq`, copy it into h_ctr

@@ -437,6 +437,10 @@ void k_do_level(hipStream_t s, const DoArgs &a, bool single_class, uint32_t bloc
 // leaving that level's input rewritten; a no-op unless that level would run
 // top-down from a small frontier with no hubs pending.  narrow_cap(): the
 // largest frontier the host starts it on
+// Sets *bad (host memory) unless R and C are a reference-layout CSR of V
+// vertices and E arcs: R starts 0,0, does not decrease and ends at E, C
+// holds ids 1..V.  Reads nothing outside the two arrays whatever they hold.
+void k_check_csr(hipStream_t s, const uint32_t *R, const uint32_t *C, uint32_t V, uint32_t E, uint32_t *bad);
 // Rows of a low-degree graph: A[v] = the up to LOW_DEG entries of v's row,
 // zeros after them (V + 1 rows).
 void k_low_rows(hipStream_t s, const DevGraph &g, uint4 *AF, uint4 *AB);
