@@ -676,6 +676,7 @@ scc_status Engine::reach_do(bool fw, bool bw, bool single, uint32_t *levels_out,
     bool low = false;   // queue low-degree levels
     auto queue = [&](int window, uint32_t blocks) {
         a.bu_ok = blocks == full;
+        a.low_next = single && deg_known && !low_denied;
         for (int k = 0; k < window; k++, level++) {
             for (int i = 0; i < nd; i++) a.d[i] = dir_args(dirs[i], level);
             a.level = (int)level;
@@ -792,7 +793,7 @@ scc_status Engine::reach_do(bool fw, bool bw, bool single, uint32_t *levels_out,
         }
         window = spec ? kSpecLevels : kDoWindow;
         blocks = full;
-        if (low) blocks = (uint32_t)std::min<int64_t>(full, std::max<int64_t>(32, (nf_max * 2 + 31) / 32));
+        if (low) blocks = (uint32_t)std::min<int64_t>(full, std::max<int64_t>(128, (nf_max * 2 + 31) / 32));
         else if (spec) blocks = (uint32_t)std::min<int64_t>(full, std::max<int64_t>(32, (nf_max * 4 + 255) / 256));
         if (!ahead) {   // after the first look: queue now, ahead from then on
             queue(window, blocks);
@@ -824,7 +825,7 @@ scc_status Engine::trim1(bool fixpoint, bool single, bool none_dead, bool wait, 
     // during a decomposition; the first pivot round reads it
     uint32_t *live = single ? live_bits() : nullptr;
     const bool degree_first = fixpoint && single && none_dead;
-    deg_known |= degree_first;
+    deg_known |= degree_first && few_arcs(g);
     const bool eager = labels || !degree_first;   // lazy: the live bitmap alone (no class or label writes)
     k_trim1(stream, g, st, st.qf[1], st.qf[0], 0u, 0, kTrimSweepShare, live, degree_first, eager);
     uint32_t pass = 1;
@@ -963,7 +964,6 @@ scc_status Engine::color_loop(int expand, int W, scc_stats *stats)
         zero_ctr(C_LIVE, 1);
         k_color_finish(stream, g, st);
     }
-    return SCC_OK;
 }
 
 scc_status Engine::run(const scc_opts &o, scc_stats *out)

@@ -176,7 +176,7 @@ constexpr uint32_t LB_LDS = QBUF + 2 + (LB_TILE + 1) + 3 * LB_TILE + 4;
 template <bool SINGLE, bool COUNT = false>
 __device__ __forceinline__ void lb_level(const DirArgs &D, const uint32_t *cls, int L, uint32_t bid,
                                          uint32_t bpd, uint32_t *lds, uint32_t n, const uint32_t *pre,
-                                         uint32_t qcap, WorkCount &wc)
+                                         uint32_t qcap, WorkCount &wc, uint32_t hops = LB_HOPS)
 {
     const unsigned long long packed = *D.pbigc;
     const uint32_t items = (uint32_t)(packed >> 32), chunks = (uint32_t)packed;
@@ -293,7 +293,7 @@ __device__ __forceinline__ void lb_level(const DirArgs &D, const uint32_t *cls, 
     }
     // Local continuation.  In a narrow single-class level (a high-diameter
     // graph's search) each workgroup goes on expanding the vertices it has
-    // just claimed, for up to LB_HOPS more hops, while they fit one tile and
+    // just claimed, for up to `hops` more hops, while they fit one tile and
     // carry at most LB_DIRECT_DEG * LB_TILE arcs; what it claims in the last
     // hop, or when it stops early, goes to the next level's queue as usual.
     // Reachability does not depend on the order of expansion, and each
@@ -310,7 +310,7 @@ __device__ __forceinline__ void lb_level(const DirArgs &D, const uint32_t *cls, 
         uint32_t *s_hb = s_off, *s_he = s_beg;   // rows of queue entries < LB_TILE
         uint32_t *const vis = D.vis;
         bool rows = false;                        // entries carry their rows
-        for (uint32_t hop = 0; hop < LB_HOPS; hop++) {
+        for (uint32_t hop = 0; hop < hops; hop++) {
             __syncthreads();
             const uint32_t m = *q.n;
             if (m == 0 || m > LB_TILE) break;
@@ -789,7 +789,7 @@ __device__ __forceinline__ void add_work(uint32_t *ctr, const WorkCount &wc)
 // stores the result in slot L&1 for level L+1.  So the host can queue any
 // number of levels without reading counters in between; a direction that
 // has finished turns its workgroups into no-ops.
-template <bool SINGLE, bool COUNT>
+template <bool SINGLE, bool COUNT, bool LOW>
 // At most 80 scalar registers (the compiler moves the rest to vector lanes):
 // with 86 to 102 (the sparse steps' uniform masks) R-MAT scale 24's dense
 // bottom-up level took 251 us instead of 225, although the compiler
@@ -822,8 +822,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_sgpr(80))) void expa
         if (bid == 0 && threadIdx.x == 0) store_dir_state(a.ctr, L & 1, dir, st);
     }
     WorkCount wc;
+    // LOW: on a low-degree graph the hops are left to the low-degree levels, which
+    // the host queues after its next look and which take a third of the time
+    // per hop: the first window's six launches of 64 hops took 0.8 ms of the
+    // 4096^2 grid's search (run 9.26 -> 8.67 ms without them, 512^2 1.73 ->
+    // 1.31).
     if (st.mode == DIR_TD)
-        lb_level<SINGLE, COUNT>(D, a.cls, L, bid, bpd, s_lds, n, slotted ? s_pre : nullptr, a.qcap, wc);
+        lb_level<SINGLE, COUNT>(D, a.cls, L, bid, bpd, s_lds, n, slotted ? s_pre : nullptr, a.qcap, wc,
+                                LOW && !a.ctr[CT(C_DEG4)] ? 0u : LB_HOPS);
     else if (st.mode == DIR_BU)
         bu_level<SINGLE, COUNT>(D, a.PR[dir], a.PC[dir], a.PF[dir], a.cls, a.V, L, bid, bpd, s_lds, a.qcap,
                                 a.ctr + CT(C_ANOM),
@@ -846,7 +852,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_sgpr(80))) void expa
 // reachability does not depend on the order.  On MI355X a hop takes 0.5 us
 // on a cycle (both directions; 1.25 before: a 20,000-vertex cycle 25 -> 10
 // ms) and 0.75 us on the 4096^2 grid, whose rows come from HBM (2.1 before;
-// run 21.7 -> 9.4 ms).  64 or 256 hops and 8 or 16 vertices per wave at the
+// run 21.7 -> 8.7 ms).  64 or 256 hops and 8 or 16 vertices per wave at the
 // start are within 5% of these; keeping 32 to 128 vertices per wave, with
 // two or four steps per hop, made the grid 6% slower.
 constexpr uint32_t LOW_HOPS = 128;
@@ -1269,11 +1275,13 @@ void k_do_level(hipStream_t s, const DoArgs &a, bool single_class, uint32_t bpd)
     bpd = dir_blocks(bpd, a.ndirs);
     const uint32_t grid = bpd * (uint32_t)a.ndirs;
     if (single_class && a.count)
-        expand_do_kernel<true, true><<<grid, 256, 0, s>>>(a, bpd);
+        (a.low_next ? expand_do_kernel<true, true, true>
+                    : expand_do_kernel<true, true, false>)<<<grid, 256, 0, s>>>(a, bpd);
     else if (single_class)
-        expand_do_kernel<true, false><<<grid, 256, 0, s>>>(a, bpd);
+        (a.low_next ? expand_do_kernel<true, false, true>
+                    : expand_do_kernel<true, false, false>)<<<grid, 256, 0, s>>>(a, bpd);
     else
-        expand_do_kernel<false, false><<<grid, 256, 0, s>>>(a, bpd);
+        expand_do_kernel<false, false, false><<<grid, 256, 0, s>>>(a, bpd);
 }
 
 template <int W>

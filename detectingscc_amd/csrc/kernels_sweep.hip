@@ -373,6 +373,7 @@ __global__ __launch_bounds__(256) void trim1_kernel(const uint32_t *__restrict__
 // lists, with TRIM_DEG_CHUNKS 64-vertex chunks' loads in flight per wave.
 constexpr uint32_t TRIM_DEG_CHUNKS = 4;
 
+template <bool LOW>
 __global__ __launch_bounds__(256) void trim1_degree_kernel(const uint32_t *__restrict__ Fr,
                                                            const uint32_t *__restrict__ Fc,
                                                            const uint32_t *__restrict__ Br,
@@ -414,7 +415,7 @@ __global__ __launch_bounds__(256) void trim1_degree_kernel(const uint32_t *__res
             // 0: no out-arc or no in-arc (vertex 0, the dummy, has neither)
             const uint64_t p = (uint64_t)(fe[h] - fb[h]) * (uint64_t)(be[h] - bb[h]);
             dp[h] = p > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)p;
-            big |= fe[h] - fb[h] > LOW_DEG || be[h] - bb[h] > LOW_DEG;
+            if (LOW) big |= fe[h] - fb[h] > LOW_DEG || be[h] - bb[h] > LOW_DEG;
             f1[h] = 0;
             b1[h] = 0;
             if (v[h] >= 1 && dp[h]) {
@@ -445,7 +446,7 @@ __global__ __launch_bounds__(256) void trim1_degree_kernel(const uint32_t *__res
         }
     }
     wave_flush_block(wq, nq, cnt_out, qout, cap, anom);
-    if (__syncthreads_or(big) && threadIdx.x == 0) ctr[CT(C_DEG4)] = 1;
+    if (LOW && __syncthreads_or(big) && threadIdx.x == 0) ctr[CT(C_DEG4)] = 1;
     spread_add32(ctr, C_TRIM1, removed);
 }
 
@@ -500,9 +501,9 @@ void k_trim1(hipStream_t s, const DevGraph &g, DevState &st, const uint32_t *in,
 {
     const uint32_t cap = trim_slot_cap(g.V);
     if (live && pass == 0 && degree_first) {
-        trim1_degree_kernel<<<sweep_blocks(g.V), SWEEP_BLOCK, 0, s>>>(g.Fr, g.Fc, g.Br, g.Bc, g.F1, g.B1, g.DP,
-                                                                      st.cls, st.lab, live, g.V, st.ctr, out,
-                                                                      cap, labels ? 1 : 0);
+        auto degree = few_arcs(g) ? trim1_degree_kernel<true> : trim1_degree_kernel<false>;
+        degree<<<sweep_blocks(g.V), SWEEP_BLOCK, 0, s>>>(g.Fr, g.Fc, g.Br, g.Bc, g.F1, g.B1, g.DP, st.cls, st.lab,
+                                                         live, g.V, st.ctr, out, cap, labels ? 1 : 0);
     } else if (live) {
         if (pass == 0) k_live_bits(s, g, st, live);
         trim1_kernel<true><<<sweep_blocks(g.V), SWEEP_BLOCK, 0, s>>>(g.Fr, g.Fc, g.Br, g.Bc, g.F1, g.B1, st.cls,

@@ -65,7 +65,7 @@ enum : int {
     C_BIGF = 22,     // 3 rotating 64-bit packed (items, chunks) counts of the FW hub lists (22..24)
     C_BIGB = 25,     // same for BW (25..27)
     C_NLEVELS = 28,  // levels run by the narrow-frontier kernel, word 0 FW, word 1 BW
-    C_DEG4 = 29,     // set if a vertex has more than LOW_DEG out- or in-arcs
+    C_DEG4 = 29,     // set if a vertex has more than LOW_DEG out- or in-arcs (by a degree pass with few_arcs)
     C_PIV0 = 30,     // first pivot of the latest election
     C_ANOM = 31,     // invariant violations caught by kernel guards (must stay 0)
     C_NLIVE = 32,    // live vertices when the visited bitmaps were initialised
@@ -162,6 +162,10 @@ struct DevGraph {
     uint32_t *DP = nullptr;
 };
 
+// Whether every vertex may have at most LOW_DEG arcs each way: the degree
+// pass looks only then (it costs the pass 2 to 5%).
+__host__ __device__ __forceinline__ bool few_arcs(const DevGraph &g) { return g.E <= (uint64_t)LOW_DEG * g.V; }
+
 struct DevState {
     uint32_t *cls = nullptr, *lab = nullptr, *aux = nullptr;
     uint32_t *fvis = nullptr, *bvis = nullptr;
@@ -209,6 +213,7 @@ struct DoArgs {
     int ndirs;
     int level;
     int bu_ok;                       // 0 on a grid too small for a bottom-up pass: stay top-down
+    int low_next;                    // 1: on a low-degree graph (C_DEG4) leave the hops to low-degree levels
     const uint4 *A[2];               // low-degree levels: each vertex's arcs in this direction (0: none)
     uint32_t qcap;                   // slot region of a bottom-up level's queue: slot_cap(V, full grid)
     int count;                       // 1: add the level's work units (WorkCount) to C_WORK..C_WORK+7
