@@ -964,6 +964,7 @@ scc_status Engine::color_loop(int expand, int W, scc_stats *stats)
         zero_ctr(C_LIVE, 1);
         k_color_finish(stream, g, st);
     }
+    return SCC_OK;
 }
 
 scc_status Engine::run(const scc_opts &o, scc_stats *out)
