@@ -1409,10 +1409,11 @@ scc_status Engine::histogram(uint64_t *pairs, uint32_t cap, uint32_t *npairs, do
     HIP_TRY(hipSetDevice(device));
     uint32_t kmax = 1;
     while ((uint64_t)kmax * (kmax + 1) / 2 <= g.V) kmax++;
-    uint64_t *dpairs;
+    // the number of pairs found, a pad word, then the pairs
+    uint64_t *dn;
     scc_status s;
-    if ((s = scratch(buf[11], 2 * (size_t)kmax + 2, &dpairs)) != SCC_OK) return s;
-    uint32_t *dn = reinterpret_cast<uint32_t *>(dpairs + 2 * (size_t)kmax);
+    if ((s = scratch(buf[11], 2 * (size_t)kmax + 2, &dn)) != SCC_OK) return s;
+    uint64_t *const dpairs = dn + 2;
     if (events.size() < 2) {
         for (size_t i = events.size(); i < 2; i++) {
             hipEvent_t e;
@@ -1422,21 +1423,27 @@ scc_status Engine::histogram(uint64_t *pairs, uint32_t cap, uint32_t *npairs, do
     }
     nmarks = 0;   // the run's phase marks are already collected
     HIP_TRY(hipEventRecord(events[0], stream));
-    k_fill_u32(stream, dn, 0u, 1);
-    k_sizes(stream, g, st);
-    k_size_histogram(stream, g, st, st.aux, dpairs, kmax, dn);
+    k_size_histogram(stream, g, st, st.aux, dpairs, kmax, reinterpret_cast<uint32_t *>(dn));
     HIP_TRY(hipEventRecord(events[1], stream));
-    uint32_t n = 0;
-    HIP_TRY(hipMemcpyAsync(&n, dn, sizeof n, hipMemcpyDeviceToHost, stream));
+    // the count and the first pairs in one copy (a power-law graph has a few
+    // dozen sizes), the rest in another
+    const size_t first = std::min<size_t>(kmax, 255);
+    std::vector<uint64_t> h(2 * first + 2);
+    HIP_TRY(hipMemcpyAsync(h.data(), dn, sizeof(uint64_t) * h.size(), hipMemcpyDeviceToHost, stream));
     HIP_TRY(hipStreamSynchronize(stream));
+    const uint32_t n = (uint32_t)h[0];
     if (n > kmax) return fail(SCC_ERR_DEVICE, "%u distinct SCC sizes exceed the bound %u", n, kmax);
-    std::vector<uint64_t> h(2 * (size_t)n);
-    if (n) HIP_TRY(hipMemcpy(h.data(), dpairs, sizeof(uint64_t) * h.size(), hipMemcpyDeviceToHost));
+    if (n > first) {
+        h.resize(2 * (size_t)n + 2);
+        HIP_TRY(hipMemcpyAsync(h.data() + 2 + 2 * first, dpairs + 2 * first, sizeof(uint64_t) * 2 * (n - first),
+                               hipMemcpyDeviceToHost, stream));
+        HIP_TRY(hipStreamSynchronize(stream));
+    }
     float t = 0;
     (void)hipEventElapsedTime(&t, events[0], events[1]);
     if (ms) *ms = t;
     std::vector<std::pair<uint64_t, uint64_t>> v(n);
-    for (uint32_t i = 0; i < n; i++) v[i] = {h[2 * i], h[2 * i + 1]};
+    for (uint32_t i = 0; i < n; i++) v[i] = {h[2 * i + 2], h[2 * i + 3]};
     std::sort(v.begin(), v.end());
     for (uint32_t i = 0; i < n && i < cap; i++) {
         pairs[2 * i] = v[i].first;

@@ -765,6 +765,10 @@ __device__ __forceinline__ void bu_level(const DirArgs &D, const uint32_t *__res
 // scale 20's two widest counted levels took 215 and 205 us; now 28 and 24.
 __device__ __forceinline__ void add_work(uint32_t *ctr, const WorkCount &wc)
 {
+    uint32_t any = 0;
+#pragma unroll
+    for (int k = 0; k < 8; k++) any |= wc.n[k];
+    if (!__syncthreads_or(any != 0)) return;
     __shared__ uint32_t s_w[8][16];
 #pragma unroll
     for (int k = 0; k < 8; k++) {

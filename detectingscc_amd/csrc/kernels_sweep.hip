@@ -1767,8 +1767,9 @@ void k_sizes(hipStream_t s, const DevGraph &g, DevState &st, bool gated)
     size_largest_kernel<<<b, TAB_BLOCK, 0, s>>>(st.lab, st.cls, st.ctr, g.V, gate);
 }
 
-// Size histogram from the sizes pass: hist[k] = number of SCCs of k
-// vertices (hist has V + 1 words, cleared here), counted in the workgroup's
+// Size histogram of the labels: the members of each SCC counted as in the
+// sizes pass, then hist[k] = number of SCCs of k vertices (hist has V + 1
+// words, cleared here with the counts), counted in the workgroup's
 // LDS table like the sizes (a power-law graph has millions of roots of size
 // 1), then the non-zero entries compacted into (size, count) pairs: `pairs`
 // holds up to `cap` of them (64-bit words, size then count), *npairs (a
@@ -1812,12 +1813,20 @@ __global__ void hist_compact_kernel(const uint32_t *__restrict__ hist, uint64_t 
     }
 }
 
+__global__ void hist_reset_kernel(uint32_t *cnt, uint32_t *hist, uint32_t *npairs, uint32_t V)
+{
+    if (blockIdx.x == 0 && threadIdx.x == 0) *npairs = 0;
+    for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v <= V; v += gridDim.x * blockDim.x)
+        cnt[v] = hist[v] = 0;
+}
+
 void k_size_histogram(hipStream_t s, const DevGraph &g, DevState &st, uint32_t *hist, uint64_t *pairs,
                       uint32_t cap, uint32_t *npairs)
 {
-    const uint32_t b = sweep_blocks(g.V);
-    size_reset_kernel<<<b, SWEEP_BLOCK, 0, s>>>(hist, g.V, nullptr);
-    hist_count_kernel<<<tab_blocks(g.V), TAB_BLOCK, 0, s>>>(st.lab, st.cls, hist, g.V);
+    const uint32_t b = sweep_blocks(g.V), t = tab_blocks(g.V);
+    hist_reset_kernel<<<b, SWEEP_BLOCK, 0, s>>>(st.cls, hist, npairs, g.V);
+    size_count_kernel<<<t, TAB_BLOCK, 0, s>>>(st.lab, st.cls, g.V, nullptr);
+    hist_count_kernel<<<t, TAB_BLOCK, 0, s>>>(st.lab, st.cls, hist, g.V);
     hist_compact_kernel<<<b, SWEEP_BLOCK, 0, s>>>(hist, pairs, cap, npairs, g.V);
 }
 
