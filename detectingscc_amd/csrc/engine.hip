@@ -408,13 +408,14 @@ template <class T> scc_status Engine::scratch(DevBuf &b, size_t n, T **out)
 // words 0..1, the search state (DirState) words 0..kDirStateWords-1.
 constexpr int kPubWords = kDirStateWords;
 
-// A spread counter is published as its own word plus its slots.
-__global__ void publish_ctr_kernel(const uint32_t *ctr, uint32_t *pub, uint32_t seq)
+// A spread counter is published as its own word plus its slots (the work
+// units, which only a run with sizes counts, if `wide`).
+__global__ void publish_ctr_kernel(const uint32_t *ctr, uint32_t *pub, uint32_t seq, int wide)
 {
     const uint32_t i = threadIdx.x;
     if (i < C_COUNT) {
         for (int w = 0; w < kPubWords; w++) pub[CT(i) + w] = ctr[CT(i) + w];
-        if (spread_index((int)i) >= 0) {
+        if (spread_index((int)i) >= 0 && (wide || !wide_counter((int)i))) {
             // the second word of a 32-bit counter's lines is 0
             uint64_t t = *reinterpret_cast<const uint64_t *>(ctr + CT(i));
             for (int j = 0; j < kSpread; j++) t += *reinterpret_cast<const uint64_t *>(ctr + CSLOT((int)i, j));
@@ -441,7 +442,8 @@ static constexpr size_t kPubBuffer = CT(C_COUNT + 1);   // words of one buffer, 
 uint32_t Engine::publish_ctr()
 {
     const uint32_t seq = ++pub_seq;
-    if (h_pub) publish_ctr_kernel<<<1, 64, 0, stream>>>(st.ctr, d_pub + (seq & 1) * kPubBuffer, seq);
+    if (h_pub) publish_ctr_kernel<<<1, 64, 0, stream>>>(st.ctr, d_pub + (seq & 1) * kPubBuffer, seq,
+                                                       search_stats ? 1 : 0);
     return seq;
 }
 
@@ -538,7 +540,7 @@ uint32_t Engine::bpd(int W) const
 void Engine::init_vis(bool elect_first, bool use_live_bits)
 {
     k_init_vis(stream, g, st, elect_first, use_live_bits ? live_bits() : nullptr);
-    do_seeded = elect_first;
+    do_seeded = elect_first ? 2 : 0;
 }
 
 // The level-L arguments of direction d (0 = FW, 1 = BW): queues alternate
@@ -572,7 +574,7 @@ scc_status Engine::reach(bool fw, bool bw, bool single, int expand, int W, uint3
 {
     if (!fw && !bw) return SCC_OK;
     if (expand == SCC_EXPAND_DO) return reach_do(fw, bw, single, levels_out);
-    do_seeded = false;   // the seeded state is for a direction-optimised search only
+    do_seeded = 0;   // the seeded state is for a direction-optimised search only
     // levels queued past the end of the search are no-ops, so a look at the
     // counters every 8 levels costs at most 7 empty launches
     const int K = check_every > 0 ? check_every : 8;
@@ -657,8 +659,8 @@ scc_status Engine::reach_do(bool fw, bool bw, bool single, uint32_t *levels_out,
     if (fw) dirs[nd++] = 0;
     if (bw) dirs[nd++] = 1;
     const uint32_t full = do_blocks(g.V, nd);
-    if (!(do_seeded && nd == 2)) k_do_begin(stream, st.ctr, nd);
-    do_seeded = false;
+    if (do_seeded != nd) k_do_begin(stream, st.ctr, nd);
+    do_seeded = 0;
     DoArgs a;
     std::memset(&a, 0, sizeof a);
     a.cls = st.cls;
@@ -880,9 +882,9 @@ scc_status Engine::pivot_round(bool first, int expand, int W, scc_stats *stats, 
     mark(SCC_PHASE_PIVOT);
     init_vis(first, first && use_live_bits);
     if (!first) {
-        zero_ctr(C_NPIV, 1);
         k_elect(stream, g, st);
         k_select(stream, g, st);
+        do_seeded = 2;
     }
     mark(SCC_PHASE_REACH, first);   // the first search is always timed
     const int first_mark = (int)nmarks - 1;
@@ -894,9 +896,8 @@ scc_status Engine::pivot_round(bool first, int expand, int W, scc_stats *stats, 
         first_reach_marks[1] = (int)nmarks - 1;
         if (search_stats) k_reach_stats(stream, g, st);
     }
-    // the first round of a decomposition follows the state initialisation,
-    // which zeroed C_LIVE, and has one pivot at most
-    if (!first) zero_ctr(C_LIVE, 1);
+    // C_LIVE is clear: in the first round (one pivot at most) from the state
+    // initialisation, later from the seeding
     // the first round's update also takes its SCC's minimum (one pivot)
     if (lazy && use_live_bits) k_update_words(stream, g, st, live_bits());
     else k_update(stream, g, st, first, first && use_live_bits ? live_bits() : nullptr, lazy);
@@ -930,7 +931,7 @@ scc_status Engine::min_label()
     scc_status s;
     uint64_t it = 0;
     do {
-        zero_ctr(C_CHANGED, 1);
+        if (it) zero_ctr(C_CHANGED, 1);
         k_minlabel_prop(stream, g, st);
         if ((s = read_ctr()) != SCC_OK) return s;
         if (++it > limit()) return no_convergence("min-label propagation");
@@ -950,18 +951,17 @@ scc_status Engine::color_loop(int expand, int W, scc_stats *stats)
         k_color_init(stream, g, st);
         uint64_t it = 0;
         do {
-            zero_ctr(C_CHANGED, 1);
+            if (it) zero_ctr(C_CHANGED, 1);
             k_color_prop(stream, g, st);
             if ((s = read_ctr()) != SCC_OK) return s;
             if (++it > limit()) return no_convergence("colour propagation");
         } while (h_ctr[CT(C_CHANGED)]);
         init_vis();
-        zero_ctr(C_NPIV, 1);
         k_color_roots(stream, g, st);
+        do_seeded = 1;
         mark(SCC_PHASE_REACH);
         if ((s = reach(true, false, false, expand, W, &stats->levels)) != SCC_OK) return s;
         mark(SCC_PHASE_UPDATE);
-        zero_ctr(C_LIVE, 1);
         k_color_finish(stream, g, st);
     }
     return SCC_OK;
@@ -1578,7 +1578,7 @@ scc_status Engine::phase_min_label(const uint8_t *dead, uint32_t *out)
     k_minlabel_init(stream, g, st);
     uint64_t it = 0;
     do {
-        zero_ctr(C_CHANGED, 1);
+        if (it) zero_ctr(C_CHANGED, 1);
         k_minlabel_prop(stream, g, st);
         if ((s = read_ctr()) != SCC_OK) return s;
         if (++it > limit()) return no_convergence("min-label propagation");
@@ -1596,7 +1596,7 @@ scc_status Engine::phase_max_color(const uint8_t *dead, uint32_t *out)
     k_color_init(stream, g, st);
     uint64_t it = 0;
     do {
-        zero_ctr(C_CHANGED, 1);
+        if (it) zero_ctr(C_CHANGED, 1);
         k_color_prop(stream, g, st);
         if ((s = read_ctr()) != SCC_OK) return s;
         if (++it > limit()) return no_convergence("colour propagation");

@@ -729,7 +729,10 @@ __global__ __launch_bounds__(1024) void vis_finish_kernel(const uint64_t *__rest
     const uint64_t t = block_sum(live);
     if (threadIdx.x != 0) return;
     ctr[CT(C_NLIVE)] = (uint32_t)t;
-    if (!ELECT) return;
+    if (!ELECT) {
+        ctr[CT(C_NPIV)] = 0;   // counted by the kernels that seed this search
+        return;
+    }
     for (uint32_t w = 1; w < (blockDim.x >> 6); w++) best = s_best[w] > best ? s_best[w] : best;
     piv[0] = best;
     const uint32_t n = best ? 1u : 0u;
@@ -944,25 +947,43 @@ __global__ __launch_bounds__(256) void select_kernel(const uint32_t *__restrict_
     wave_flush_block_each(wq, nq, &ctr[CT(C_NPIV)], put);
 }
 
-// Queue counts for level 0 and the two counters after it.
-__global__ void seed_counts_kernel(uint32_t *ctr, const uint32_t *seeds, int seed_bw)
+// Queue counts for level 0 and the two counters after it, the level-0 state
+// of a direction-optimised search in `ndirs` directions (what do_begin_kernel
+// writes) and C_LIVE cleared for the round's update: with the clears of
+// C_NPIV and C_CHANGED in the kernels before, a round of colours takes four
+// launches less, of 4 to 5 us each.
+__global__ __launch_bounds__(64) void seed_counts_kernel(uint32_t *ctr, const uint32_t *seeds, int ndirs)
 {
-    uint32_t n = ctr[CT(C_NPIV)];
-    ctr[CT(C_PIV0)] = n ? seeds[0] : 0u;
-    ctr[CT(C_FWCNT + 0)] = n;
-    ctr[CT(C_FWCNT + 1)] = 0;
-    ctr[CT(C_FWCNT + 2)] = 0;
-    ctr[CT(C_BWCNT + 0)] = seed_bw ? n : 0;
-    ctr[CT(C_BWCNT + 1)] = 0;
-    ctr[CT(C_BWCNT + 2)] = 0;
-    zero_hub_counts(ctr);
+    const int t = (int)threadIdx.x;
+    const uint32_t n = ctr[CT(C_NPIV)];
+    for (int j = t; j < 6 * kSpread; j += 64) ctr[CSLOT(C_FWCNT, j)] = 0;
+    if (t < kSpread) ctr[CSLOT(C_LIVE, t)] = 0;
+    if (t < 3) {
+        ctr[CT(C_FWCNT + t)] = t == 0 ? n : 0u;
+        ctr[CT(C_BWCNT + t)] = t == 0 && ndirs == 2 ? n : 0u;
+        *reinterpret_cast<unsigned long long *>(ctr + CT(C_BIGF + t)) = 0ull;
+        *reinterpret_cast<unsigned long long *>(ctr + CT(C_BIGB + t)) = 0ull;
+    }
+    if (t < 2) {
+        DirState ds;
+        ds.mode = t < ndirs ? DIR_TD : DIR_OFF;
+        ds.end = 0;
+        ds.nf = n;
+        ds.pad = 0;
+        ds.visited = n;
+        store_dir_state(ctr, 0, t, ds);
+    }
+    if (t == 0) {
+        ctr[CT(C_PIV0)] = n ? seeds[0] : 0u;
+        ctr[CT(C_LIVE)] = 0;
+    }
 }
 
 void k_select(hipStream_t s, const DevGraph &g, DevState &st)
 {
     select_kernel<<<sweep_blocks(g.V), SWEEP_BLOCK, 0, s>>>(g.DP, st.cls, st.piv, st.fvis, st.bvis, st.qf[0],
                                                             st.qb[0], st.pivlist, st.ctr, g.V);
-    seed_counts_kernel<<<1, 1, 0, s>>>(st.ctr, st.pivlist, 1);
+    seed_counts_kernel<<<1, 64, 0, s>>>(st.ctr, st.pivlist, 2);
 }
 
 // A single source for the phase entry point: vertex src seeds direction dir.
@@ -1306,15 +1327,23 @@ void k_reach_stats(hipStream_t s, const DevGraph &g, DevState &st)
 // assignUniqueRange + propagateRange1/2 (scc_kernels.cu:477-536): label =
 // min id reachable over live out-arcs; pointer jumping follows label
 // chains.  DEAD is the largest value, so finished vertices never win a min.
-__global__ void minlabel_init_kernel(uint32_t *cls, uint32_t V)
+// Clears C_CHANGED for the first propagation pass (one workgroup calls).
+__device__ __forceinline__ void clear_changed(uint32_t *ctr)
 {
+    if (threadIdx.x < (uint32_t)kSpread) ctr[CSLOT(C_CHANGED, (int)threadIdx.x)] = 0;
+    if (threadIdx.x == 0) ctr[CT(C_CHANGED)] = 0;
+}
+
+__global__ void minlabel_init_kernel(uint32_t *cls, uint32_t *ctr, uint32_t V)
+{
+    if (blockIdx.x == 0) clear_changed(ctr);
     for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x + 1; v <= V; v += gridDim.x * blockDim.x)
         if (cls[v] != DEAD) cls[v] = v;
 }
 
 void k_minlabel_init(hipStream_t s, const DevGraph &g, DevState &st)
 {
-    minlabel_init_kernel<<<sweep_blocks(g.V), SWEEP_BLOCK, 0, s>>>(st.cls, g.V);
+    minlabel_init_kernel<<<sweep_blocks(g.V), SWEEP_BLOCK, 0, s>>>(st.cls, st.ctr, g.V);
 }
 
 // m folded (minimum, or maximum with MAX) with val[w] over the arcs
@@ -1394,15 +1423,16 @@ void k_minlabel_finish(hipStream_t s, const DevGraph &g, DevState &st)
 // ----------------------------------------------------- colouring ---
 // colorPropagation (scc_kernels.cu:539-564): colour = max id reachable over
 // live out-arcs, with pointer jumping added.  aux[v] = 0 for finished v.
-__global__ void color_init_kernel(const uint32_t *__restrict__ cls, uint32_t *aux, uint32_t V)
+__global__ void color_init_kernel(const uint32_t *__restrict__ cls, uint32_t *aux, uint32_t *ctr, uint32_t V)
 {
+    if (blockIdx.x == 0) clear_changed(ctr);
     for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v <= V; v += gridDim.x * blockDim.x)
         aux[v] = (v && cls[v] != DEAD) ? v : 0u;
 }
 
 void k_color_init(hipStream_t s, const DevGraph &g, DevState &st)
 {
-    color_init_kernel<<<sweep_blocks(g.V), SWEEP_BLOCK, 0, s>>>(st.cls, st.aux, g.V);
+    color_init_kernel<<<sweep_blocks(g.V), SWEEP_BLOCK, 0, s>>>(st.cls, st.aux, st.ctr, g.V);
 }
 
 __global__ __attribute__((amdgpu_num_sgpr(80))) void color_prop_kernel(const uint32_t *__restrict__ Fr,
@@ -1472,7 +1502,7 @@ __global__ __launch_bounds__(256) void color_roots_kernel(uint32_t *cls, const u
 void k_color_roots(hipStream_t s, const DevGraph &g, DevState &st)
 {
     color_roots_kernel<<<sweep_blocks(g.V), SWEEP_BLOCK, 0, s>>>(st.cls, st.aux, st.fvis, st.qf[0], st.ctr, g.V);
-    seed_counts_kernel<<<1, 1, 0, s>>>(st.ctr, st.qf[0], 0);
+    seed_counts_kernel<<<1, 64, 0, s>>>(st.ctr, st.qf[0], 1);
 }
 
 // fwdColoring marks each vertex it expands as finished (scc_kernels.cu:607):
