@@ -446,7 +446,7 @@ __global__ __launch_bounds__(256) void trim1_degree_kernel(const uint32_t *__res
         }
     }
     wave_flush_block(wq, nq, cnt_out, qout, cap, anom);
-    if (LOW && __syncthreads_or(big) && threadIdx.x == 0) ctr[CT(C_DEG4)] = 1;
+    if (LOW && big) ctr[CT(C_DEG4)] = 1;   // a plain store: any number of lanes write the same value
     spread_add32(ctr, C_TRIM1, removed);
 }
 
