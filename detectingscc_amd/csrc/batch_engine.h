@@ -13,7 +13,9 @@ class Engine;
 class BatchEngine {
   public:
     ~BatchEngine();
-    scc_status upload(int device, hipStream_t stream, const scc_batch_host *b);
+    // `checked`: the caller has already validated the graphs (the server's
+    // submit does)
+    scc_status upload(int device, hipStream_t stream, const scc_batch_host *b, bool checked = false);
     // a batch in device memory in the host layout (row_off/col_off given on
     // the host, d_roff = row_off on the device), valid by construction
     scc_status upload_device(int device, hipStream_t stream, uint32_t ng, const uint32_t *Vs, const uint32_t *Es,
@@ -32,7 +34,7 @@ class BatchEngine {
     void release();
     scc_status prepare(int device, hipStream_t stream, uint32_t ng, const uint32_t *Vs, const uint32_t *Es,
                        const uint64_t *roff, const uint64_t *coff);
-    scc_status finish_upload();
+    scc_status finish_upload(bool check);
     scc_status launch(const std::vector<uint32_t> &idx, const std::vector<uint32_t> &cfg,
                       const std::vector<int> &block, double *ms, std::vector<double> *lat_ms,
                       uint32_t *launches);

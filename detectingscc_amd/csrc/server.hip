@@ -256,7 +256,7 @@ void Server::worker(int slot)
             h.Fc = Fc.data();
             h.Bc = Bc.data();
             scc_batch_stats bst;
-            st = be->upload(dev, stream, &h);
+            st = be->upload(dev, stream, &h, true);   // checked when they were submitted
             if (st == SCC_OK) st = be->run(opts, &bst);
             if (st == SCC_OK) st = be->labels(lab.data(), nscc.data());
         }

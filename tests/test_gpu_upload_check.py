@@ -47,3 +47,33 @@ def test_faults_are_refused(V, E, held):
             ctx.upload(g)
             assert ctx.run().num_sccs == n
             assert_same_labels(ctx.labels(), want, "after the refusals")
+
+
+@pytest.mark.parametrize("graphs,vmax,degree", [(1, 1, 0), (1, 70000, 3), (9, 600, 4), (300, 200, 5), (9000, 12, 2)])
+def test_batch_faults_are_refused(graphs, vmax, degree):
+    rng = np.random.default_rng(graphs)
+    sizes = [vmax] * graphs if graphs == 1 else rng.integers(1, vmax + 1, graphs)
+    good = scc.batch_from_graphs([random_graph(int(v), int(v) * degree, rng) for v in sizes])
+    wants = [orc.tarjan(good.graph(i)) for i in range(0, graphs, max(1, graphs // 50))]
+    with scc.Context(0) as ctx:
+        for g in sorted({0, graphs // 2, graphs - 1}):
+            V, E = int(good.V[g]), int(good.E[g])
+            faults = [("Fr", "row_off", v, E + 1) for v in {2, V} if V >= 2]
+            faults += [("Br", "row_off", v, E + 1) for v in {2, V} if V >= 2]
+            faults += [(a, "col_off", k, c) for a in ("Fc", "Bc") if E for k in {0, E // 2, E - 1}
+                       for c in (0, V + 1, 0xFFFFFFFF)]
+            for name, off, at, value in faults:
+                arrays = {k: getattr(good, k).copy() for k in ("Fr", "Fc", "Br", "Bc")}
+                arrays[name][int(getattr(good, off)[g]) + at] = value
+                bad = scc.Batch(good.V, good.E, good.row_off, good.col_off, arrays["Fr"], arrays["Fc"],
+                                arrays["Br"], arrays["Bc"])
+                with pytest.raises(scc.SCCError, match="invalid CSR"):
+                    ctx.batch_upload(bad)
+                with pytest.raises(scc.SCCError, match="no batch"):
+                    ctx.batch_run()
+        ctx.batch_upload(good)
+        ctx.batch_run()
+        labels, counts = ctx.batch_labels()
+        for k, i in enumerate(range(0, graphs, max(1, graphs // 50))):
+            assert counts[i] == wants[k][1]
+            assert_same_labels(labels[i], wants[k][0], f"graph {i}")
