@@ -558,19 +558,28 @@ scc_status BatchEngine::labels(uint32_t *lab, uint32_t *nscc)
         uint32_t *packed = d.q;
         uint64_t *d_roff = reinterpret_cast<uint64_t *>(d.q + 2 * capS);
         const uint64_t words = row_off[G - 1] + V[G - 1] + 1 - row_off[0];
-        BHIP(hipMemcpyAsync(d_roff, row_off.data(), sizeof(uint64_t) * G, hipMemcpyHostToDevice, s1));
+        // the offsets go through the page-locked launch block (kHeads words,
+        // then two per graph), the counts through the result block: no copy
+        // but the labels' own waits for the host
+        std::memcpy(h_meta + kHeads, row_off.data(), sizeof(uint64_t) * G);
+        BHIP(hipMemcpyAsync(d_roff, h_meta + kHeads, sizeof(uint64_t) * G, hipMemcpyHostToDevice, s1));
         batch_pack_kernel<<<std::min<uint32_t>(G, 8192), 256, 0, s1>>>(d.lab, m_voff, d_roff, m_V, G, packed);
         BHIP(hipGetLastError());
         std::vector<uint32_t> gaps;
         gaps.reserve(words - nverts - G);
         for (uint32_t i = 0; i + 1 < G; i++)
             gaps.insert(gaps.end(), lab + row_off[i] + V[i] + 1, lab + row_off[i + 1]);
+        uint32_t *const counts = reinterpret_cast<uint32_t *>(h_res + 2 * (size_t)capG);
+        if (nscc) BHIP(hipMemcpyAsync(counts, d.nscc, sizeof(uint32_t) * G, hipMemcpyDeviceToHost, s1));
         BHIP(hipMemcpyAsync(lab + row_off[0], packed, sizeof(uint32_t) * words, hipMemcpyDeviceToHost, s1));
         BHIP(hipStreamSynchronize(s1));
+        if (nscc) std::memcpy(nscc, counts, sizeof(uint32_t) * G);
         const uint32_t *gap = gaps.data();
         for (uint32_t i = 0; i + 1 < G; i++)
             for (uint64_t k = row_off[i] + V[i] + 1; k < row_off[i + 1]; k++) lab[k] = *gap++;
-    } else if (lab) {
+        return SCC_OK;
+    }
+    if (lab) {
         std::vector<uint32_t> all(voff[G]);
         BHIP(hipMemcpy(all.data(), d.lab, sizeof(uint32_t) * voff[G], hipMemcpyDeviceToHost));
         parallel_chunks(G, [&](uint64_t lo, uint64_t hi, int) {
