@@ -627,20 +627,28 @@ __device__ __forceinline__ bool g_narrow_both(Lds &L, const G1 &g, uint32_t (&lo
 // less than two bottom-up sweeps: 63,665 vertices of 2.07 arcs 1.20 -> 0.66
 // ms for the search; from 8 arcs on it costs more (mix 1.91 -> 2.32 ms with
 // BU_DEGREE at 8).
+// 64-vertex chunks a wave takes side by side in a bottom-up level: their
+// lists' loads are in flight together, but a step lasts as long as the
+// longest list of all of them.  A batch, whose workgroups share the memory's
+// latency, takes four (mix 1.84 ms; two 1.88, one 1.99); the small-graph
+// kernel, alone on its CU and with graphs under 15,000 arcs in LDS, one (999
+// vertices 45 us with four, 41 with two, 39 with one; 16,384 and 139,000
+// arcs 101, 98, 95.5).
 constexpr uint32_t BU_CHUNKS = 4;
 constexpr uint64_t BU_SWITCH = 3, BU_BURST = 8, BU_DEGREE = 3;
 
+template <uint32_t BUC>
 __device__ __forceinline__ void g_bottom_up(Lds &L, const G1 &g, uint32_t d, uint32_t w, uint32_t nw,
                                             bool first)
 {
     const uint32_t *R = d ? g.Fr : g.Br, *C = d ? g.Fc : g.Bc, *P = d ? g.f1() : g.b1();
     uint32_t *vis = d ? g.bvis : g.fvis, *q = g.queue(2 * d);
     const uint32_t nch = (g.V + 64) / 64;
-    for (uint32_t c0 = w; c0 < nch; c0 += BU_CHUNKS * nw) {
-        uint32_t word[BU_CHUNKS], cand[BU_CHUNKS], p[BU_CHUNKS];
+    for (uint32_t c0 = w; c0 < nch; c0 += BUC * nw) {
+        uint32_t word[BUC], cand[BUC], p[BUC];
         bool any = false;
 #pragma unroll
-        for (uint32_t h = 0; h < BU_CHUNKS; h++) {
+        for (uint32_t h = 0; h < BUC; h++) {
             const uint32_t ch = c0 + h * nw, i = 2 * ch + (ln() >> 5);
             word[h] = ch < nch ? vis[i] : ~0u;
             cand[h] = ch < nch ? g.live[i] & ~word[h] : 0u;
@@ -649,36 +657,36 @@ __device__ __forceinline__ void g_bottom_up(Lds &L, const G1 &g, uint32_t d, uin
         if (!__ballot(any)) continue;
         if (first) {
 #pragma unroll
-            for (uint32_t h = 0; h < BU_CHUNKS; h++) {
+            for (uint32_t h = 0; h < BUC; h++) {
                 const uint32_t v = (c0 + h * nw) * 64 + ln();
                 p[h] = at(P, v <= g.V ? v : 0u);
             }
         }
-        bool hit[BU_CHUNKS], more[BU_CHUNKS];
+        bool hit[BUC], more[BUC];
         bool anym = false;
 #pragma unroll
-        for (uint32_t h = 0; h < BU_CHUNKS; h++) {
+        for (uint32_t h = 0; h < BUC; h++) {
             const bool is = (cand[h] >> (ln() & 31)) & 1u;
             hit[h] = first && is && bbit(vis, p[h]);   // a live vertex has a first parent
             more[h] = is && !hit[h];
             anym |= more[h];
         }
         if (__ballot(anym)) {
-            const uint32_t *Ck[BU_CHUNKS];
-            uint32_t b[BU_CHUNKS], e[BU_CHUNKS], x[BU_CHUNKS];
+            const uint32_t *Ck[BUC];
+            uint32_t b[BUC], e[BUC], x[BUC];
 #pragma unroll
-            for (uint32_t h = 0; h < BU_CHUNKS; h++) {
+            for (uint32_t h = 0; h < BUC; h++) {
                 const uint32_t r = more[h] ? (c0 + h * nw) * 64 + ln() : 0u;   // row 0 is empty
                 Ck[h] = C;
                 b[h] = at(R, r);
                 e[h] = at(R, r + 1);
             }
-            g_any_bit<BU_CHUNKS>(Ck, b, e, vis, x);
+            g_any_bit<BUC>(Ck, b, e, vis, x);
 #pragma unroll
-            for (uint32_t h = 0; h < BU_CHUNKS; h++) hit[h] |= x[h] != 0;
+            for (uint32_t h = 0; h < BUC; h++) hit[h] |= x[h] != 0;
         }
 #pragma unroll
-        for (uint32_t h = 0; h < BU_CHUNKS; h++) {
+        for (uint32_t h = 0; h < BUC; h++) {
             const uint32_t ch = c0 + h * nw;
             const uint64_t m = __ballot(hit[h]);
             if (!m) continue;
@@ -702,7 +710,8 @@ __device__ __forceinline__ void g_both(const uint32_t *lo, const uint32_t *hi, L
 
 // The first pivot's FW and BW search, each level of a direction top-down or
 // bottom-up (`dense`: the graph has the arcs for it).
-template <int BS> __device__ __forceinline__ void g_first_search(Lds &L, const G1 &g, uint32_t nlive, bool first, bool dense)
+template <int BS, uint32_t BUC>
+__device__ __forceinline__ void g_first_search(Lds &L, const G1 &g, uint32_t nlive, bool first, bool dense)
 {
     uint32_t lo[2] = {0, 0}, hi[2] = {1, 1}, prev[2] = {1, 1};
     bool bu[2] = {false, false};
@@ -714,7 +723,7 @@ template <int BS> __device__ __forceinline__ void g_first_search(Lds &L, const G
         if (lo[0] == hi[0] && lo[1] == hi[1]) break;
         if (threadIdx.x == 0) L.st.levels++;
         g_both<BS>(lo, hi, [&](uint32_t d, uint32_t w, uint32_t nw) {
-            if (d ? bu[1] : bu[0]) g_bottom_up(L, g, d, w, nw, first);
+            if (d ? bu[1] : bu[0]) g_bottom_up<BUC>(L, g, d, w, nw, first);
             else g_expand<true>(L, g, d, d ? lo[1] : lo[0], d ? hi[1] : hi[0], w, nw);
         });
         __syncthreads();
@@ -1102,7 +1111,8 @@ template <int BS> __device__ __forceinline__ uint32_t g_canon(Lds &L, const G1 &
 // The whole pipeline of one graph; returns its number of SCCs.  LDS_BITS /
 // LDS_CLS only say which memory the views point to: the code is the same,
 // and inlined per case so that the accesses are LDS instructions.
-template <int BS> __device__ __forceinline__ uint32_t g_solve(Lds &L, const G1 &g, uint32_t cfg)
+template <int BS, uint32_t BUC = BU_CHUNKS>
+__device__ __forceinline__ uint32_t g_solve(Lds &L, const G1 &g, uint32_t cfg)
 {
     const uint32_t nch = (g.V + 64) / 64, nw = 2 * nch;
     if (threadIdx.x == 0) {
@@ -1153,7 +1163,7 @@ template <int BS> __device__ __forceinline__ uint32_t g_solve(Lds &L, const G1 &
         }
         __syncthreads();
         const uint64_t t0 = wall_clock64();
-        g_first_search<BS>(L, g, nlive, first, g.E >= BU_DEGREE * (uint64_t)g.V);
+        g_first_search<BS, BUC>(L, g, nlive, first, g.E >= BU_DEGREE * (uint64_t)g.V);
         if (threadIdx.x == 0) {
             L.st.search_ticks = wall_clock64() - t0;
             L.st.first_pivot = p0;
@@ -1306,9 +1316,9 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) void ba
 // a level's dependent loads are LDS reads.  The counters the host waits for
 // are written to its mapped memory by the kernel itself.
 // Whole calls, one workgroup against the device-wide engine, at 2, 4, 8 and
-// 16 arcs per vertex: 1,000 vertices 57 / 45 / 34 / 31 us against 120 / 112 /
-// 123 / 98, 8,000 vertices 128 / 99 / 83 / 56 against 407 / 134 / 116 / 107,
-// 16,384 vertices 190 / 150 / 103 / 87 against 388 / 149 / 121 / 108; at
+// 16 arcs per vertex: 1,000 vertices 58 / 39 / 29 / 26 us against 120 / 112 /
+// 123 / 98, 8,000 vertices 125 / 90 / 78 / 56 against 407 / 134 / 116 / 107,
+// 16,384 vertices 193 / 139 / 94 / 87 against 388 / 149 / 121 / 108; at
 // 32,768 vertices it would be 250 against 148 at 4 arcs.
 constexpr uint32_t SMALL_LDS = 36864;   // words: class words, or everything of a graph that fits
 
@@ -1348,7 +1358,7 @@ __global__ __launch_bounds__(1024) void small_scc_kernel(SmallArgs a)
         g.Fc = Fc;
         g.Bc = Bc;
         __syncthreads();
-        n = g_solve<1024>(L, g, a.cfg);
+        n = g_solve<1024, 1>(L, g, a.cfg);
     } else {
         g.Fr = a.Fr;
         g.Br = a.Br;
@@ -1356,7 +1366,7 @@ __global__ __launch_bounds__(1024) void small_scc_kernel(SmallArgs a)
         g.Bc = a.Bc;
         g.aux = a.aux;
         g.q = a.q;
-        n = g_solve<1024>(L, g, a.cfg);
+        n = g_solve<1024, 1>(L, g, a.cfg);
     }
     __syncthreads();
     if (threadIdx.x != 0) return;
