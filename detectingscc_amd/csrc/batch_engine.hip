@@ -535,10 +535,14 @@ __global__ void batch_pack_kernel(const uint32_t *lab, const uint64_t *dvoff, co
     }
 }
 
-// Whether the labels leave as one copy: at most as many words between two
-// graphs' labels (one each in the layout of scc_gen_batch_mix) as labels.
+// Whether the labels leave as one copy: rows in ascending order (prepare()'s
+// check of their distances is modulo 2^64 and lets any order pass), with at
+// most as many words between two graphs' labels (one each in the layout of
+// scc_gen_batch_mix) as labels.
 bool BatchEngine::packed_labels() const
 {
+    for (uint32_t i = 1; i < G; i++)
+        if (row_off[i] < row_off[i - 1]) return false;
     return row_off[G - 1] + V[G - 1] + 1 - row_off[0] <= 2 * (nverts + G);
 }
 

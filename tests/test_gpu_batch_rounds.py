@@ -91,3 +91,30 @@ def test_batch_labels_layout(slack):
         own[at:at + g.V + 1] = True
         assert_same_labels(lab[at:at + g.V + 1], orc.tarjan(g)[0], f"slack {slack} graph {i}")
     assert (lab[~own] == 0xABCD).all()
+
+
+@pytest.mark.parametrize("starts", [(0, 204, 102, 306), (102, 0, 204, 306), (204, 102, 0, 306), (7, 1000, 500, 5000),
+                                    (5000, 0, 9000, 200)])
+def test_batch_labels_row_order(starts):
+    """Rows in any order: graph i's rows, and its labels, are at row_off[i]."""
+    rng = np.random.default_rng(sum(starts))
+    gs = [random_graph(100, 300, rng) for _ in range(len(starts))]
+    n = max(starts) + 102
+    row = np.array(starts + (starts[-1] + 102,), np.uint64)
+    Fr, Br = np.zeros(n, np.uint32), np.zeros(n, np.uint32)
+    for at, g in zip(starts, gs):
+        Fr[at:at + 102], Br[at:at + 102] = g.Fr, g.Br
+    b = scc.batch_from_graphs(gs)
+    b = scc.Batch(b.V, b.E, row, b.col_off, Fr, b.Fc, Br, b.Bc)
+    lab = np.full(n, 0xABCD, np.uint32)
+    nscc = np.zeros(len(gs), np.uint32)
+    with scc.Context(0) as ctx:
+        ctx.batch_upload(b)
+        ctx.batch_run()
+        assert scc.lib().scc_batch_labels(ctx._ctx, scc._p32(lab), scc._p32(nscc)) == 0
+    for i, (at, g) in enumerate(zip(starts, gs)):
+        want, k = orc.tarjan(g)
+        assert_same_labels(lab[at:at + 101], want, f"rows at {starts}, graph {i}")
+        assert nscc[i] == k
+        lab[at:at + 101] = 0xABCD
+    assert (lab == 0xABCD).all()
