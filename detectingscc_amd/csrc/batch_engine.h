@@ -24,7 +24,8 @@ class BatchEngine {
     scc_status run(const scc_batch_opts &o, scc_batch_stats *out);
     scc_status run_serial(Engine &eng, const scc_opts &o, scc_batch_stats *out);
     scc_status autotune(int sample, std::string *report);
-    scc_status labels(uint32_t *lab, uint32_t *nscc);
+    // lab in the host layout, or graph i's V[i]+1 labels to each[i]
+    scc_status labels(uint32_t *lab, uint32_t *nscc, uint32_t *const *each = nullptr);
     // the uploaded batch's sizes and host-layout offsets (arrays may be NULL)
     uint32_t info(uint32_t *Vs, uint32_t *Es, uint64_t *roff, uint64_t *coff) const;
 
@@ -38,7 +39,7 @@ class BatchEngine {
     scc_status launch(const std::vector<uint32_t> &idx, const std::vector<uint32_t> &cfg,
                       const std::vector<int> &block, double *ms, std::vector<double> *lat_ms,
                       uint32_t *launches);
-    bool packed_labels() const;   // the host layout has few words that are not labels
+    scc_status spread_labels(const uint32_t *packed, uint64_t words, uint32_t *lab, uint32_t *const *each);
 
     int dev = 0;
     hipStream_t s1 = nullptr, stream2 = nullptr;
@@ -63,6 +64,13 @@ class BatchEngine {
     // page-locked host side of both blocks
     uint32_t *h_meta = nullptr;
     uint64_t *h_res = nullptr;
+    // two page-locked blocks that labels for pageable memory pass through
+    // (made on first use, at most kLabelBlock words each: a block's wait costs
+    // about 9 us, 190 MB of labels take 14.4 ms in blocks of 2^16 words, 7.9 of
+    // 2^18, 7.4 of 2^20)
+    static constexpr uint64_t kLabelBlock = 1 << 18;
+    uint32_t *h_label = nullptr;
+    uint64_t label_words = 0;
     hipEvent_t ev[3] = {nullptr, nullptr, nullptr};   // start, end of each stream
     int occ[3] = {0, 0, 0};                           // workgroups per CU at 1,024, 512 and 256 lanes
     std::vector<uint32_t> stage;        // host staging of the row arrays

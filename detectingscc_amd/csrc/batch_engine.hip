@@ -32,8 +32,11 @@ void BatchEngine::release()
     allocs.clear();
     if (h_meta) (void)hipHostFree(h_meta);
     if (h_res) (void)hipHostFree(h_res);
+    if (h_label) (void)hipHostFree(h_label);
     h_meta = nullptr;
     h_res = nullptr;
+    h_label = nullptr;
+    label_words = 0;
     for (auto &e : ev) {
         if (e) (void)hipEventDestroy(e);
         e = nullptr;
@@ -523,75 +526,130 @@ scc_status BatchEngine::autotune(int sample, std::string *report)
     return SCC_OK;
 }
 
-// Labels of graph g (V+1 entries) from slot voff[g] to the host layout's
-// offset: one workgroup per graph.
-__global__ void batch_pack_kernel(const uint32_t *lab, const uint64_t *dvoff, const uint64_t *roff,
-                                  const uint32_t *Vn, uint32_t G, uint32_t *dst)
+// Labels of graph g (V+1 entries) from slot dvoff[g] to dst + off[g].
+// Workgroup column y of graph g takes every gridDim.y-th 256 words, so that a
+// few large graphs fill the card too; a wave's 64 words start at a multiple
+// of 256 bytes of the destination, which may be host memory behind the link.
+__global__ __launch_bounds__(256) void batch_pack_kernel(const uint32_t *__restrict__ lab,
+                                                         const uint64_t *__restrict__ dvoff,
+                                                         const uint64_t *__restrict__ off,
+                                                         const uint32_t *__restrict__ Vn, uint32_t G, uint32_t *dst)
 {
     for (uint32_t g = blockIdx.x; g < G; g += gridDim.x) {
         const uint32_t *src = lab + dvoff[g];
-        uint32_t *to = dst + (roff[g] - roff[0]);
-        for (uint32_t i = threadIdx.x; i <= Vn[g]; i += blockDim.x) to[i] = src[i];
+        uint32_t *to = dst + off[g];
+        const uint64_t before = (reinterpret_cast<uint64_t>(to) >> 2) & 63, n = before + Vn[g] + 1;
+        for (uint64_t i = blockIdx.y * 256ull + threadIdx.x; i < n; i += gridDim.y * 256ull)
+            if (i >= before) to[i - before] = src[i - before];
     }
 }
 
-// Whether the labels leave as one copy: rows in ascending order (prepare()'s
-// check of their distances is modulo 2^64 and lets any order pass), with at
-// most as many words between two graphs' labels (one each in the layout of
-// scc_gen_batch_mix) as labels.
-bool BatchEngine::packed_labels() const
+// The device's address of the caller's words p[0..n) if they lie in one
+// page-locked allocation that this device can write, otherwise null.
+static uint32_t *device_view(int dev, uint32_t *p, uint64_t n)
 {
-    for (uint32_t i = 1; i < G; i++)
-        if (row_off[i] < row_off[i - 1]) return false;
-    return row_off[G - 1] + V[G - 1] + 1 - row_off[0] <= 2 * (nverts + G);
+    hipPointerAttribute_t a;
+    hipDeviceptr_t base = nullptr;
+    size_t bytes = 0;
+    if (hipPointerGetAttributes(&a, p) == hipSuccess && a.type == hipMemoryTypeHost && a.device == dev &&
+        a.devicePointer && hipMemGetAddressRange(&base, &bytes, (hipDeviceptr_t)a.devicePointer) == hipSuccess) {
+        const uint64_t at = (uint64_t)(static_cast<char *>(a.devicePointer) - static_cast<char *>(base));
+        if (at <= bytes && sizeof(uint32_t) * n <= bytes - at) return static_cast<uint32_t *>(a.devicePointer);
+        return nullptr;
+    }
+    (void)hipGetLastError();
+    return nullptr;
 }
 
-// The labels go from the slots into the host layout on the device and leave
-// as one copy straight into the caller's buffer; the few words between two
-// graphs' labels, which are the caller's, are put back after it.  On the
-// 4,096-graph mix (190 MB of labels) 50 ms of a zeroed host vector, a
-// pageable copy into it and a second copy out of it -> 3.6 ms into a
-// page-locked buffer (the link's 56 GB/s and 0.1 ms for the pack).
-scc_status BatchEngine::labels(uint32_t *lab, uint32_t *nscc)
+// Every graph's labels go to the host layout's offset, and no other word of
+// the caller's buffer is written.  Into a page-locked buffer the device writes
+// them itself; for any other they are packed on the device and come through
+// two page-locked blocks, one on the link while the host spreads the other.
+// The 4,096-graph mix (190 MB of labels) takes 3.6 ms (the link's rate) into
+// a page-locked buffer and 7.9 ms into pageable memory, where one copy of the
+// whole span, gaps included, took 3.7 and 11.4 and a copy of the slots to a
+// host vector and on to the caller 51; one graph of 2^20 vertices 0.10 and
+// 0.23 ms against 1.53 and 1.70 (one workgroup packed it) and 0.45.
+scc_status BatchEngine::labels(uint32_t *lab, uint32_t *nscc, uint32_t *const *each)
 {
     if (!ran) return fail(SCC_ERR_NOTREADY, "no completed batch run");
     BHIP(hipSetDevice(dev));
-    if (lab && packed_labels()) {
-        // the queues are free between runs: 4 * capS words, of which the
-        // packed labels take at most 2 * (nverts + G) <= 2 * capS, then the offsets
-        uint32_t *packed = d.q;
-        uint64_t *d_roff = reinterpret_cast<uint64_t *>(d.q + 2 * capS);
-        const uint64_t words = row_off[G - 1] + V[G - 1] + 1 - row_off[0];
-        // the offsets go through the page-locked launch block (kHeads words,
-        // then two per graph), the counts through the result block: no copy
-        // but the labels' own waits for the host
-        std::memcpy(h_meta + kHeads, row_off.data(), sizeof(uint64_t) * G);
-        BHIP(hipMemcpyAsync(d_roff, h_meta + kHeads, sizeof(uint64_t) * G, hipMemcpyHostToDevice, s1));
-        batch_pack_kernel<<<std::min<uint32_t>(G, 8192), 256, 0, s1>>>(d.lab, m_voff, d_roff, m_V, G, packed);
+    // counts and offsets go through the page-locked result block (ticks, then
+    // counts) and launch block (kHeads words, then two per graph)
+    uint32_t *const counts = reinterpret_cast<uint32_t *>(h_res + 2 * (size_t)capG);
+    if (nscc) BHIP(hipMemcpyAsync(counts, d.nscc, sizeof(uint32_t) * G, hipMemcpyDeviceToHost, s1));
+    if (lab || each) {
+        uint64_t first = UINT64_MAX, last = 0;
+        for (uint32_t i = 0; i < G; i++) {
+            first = std::min(first, row_off[i]);
+            last = std::max(last, row_off[i] + V[i] + 1);
+        }
+        uint32_t *const view = each ? nullptr : device_view(dev, lab + first, last - first);
+        uint64_t *const off = reinterpret_cast<uint64_t *>(h_meta + kHeads);
+        uint64_t words = 0;
+        for (uint32_t i = 0; i < G; i++) {
+            off[i] = view ? row_off[i] - first : words;
+            words += (uint64_t)V[i] + 1;
+        }
+        // the queues (4 * capS words) are free between runs: the packed labels
+        // (nverts + G <= capS words), then the offsets (2 * G <= capS words)
+        uint32_t *const packed = d.q;
+        uint64_t *const d_off = reinterpret_cast<uint64_t *>(d.q + 2 * capS);
+        BHIP(hipMemcpyAsync(d_off, off, sizeof(uint64_t) * G, hipMemcpyHostToDevice, s1));
+        const uint32_t cols = std::min<uint32_t>(64, std::max<uint32_t>(1, 4096 / G));
+        batch_pack_kernel<<<dim3(std::min<uint32_t>(G, 8192), cols), 256, 0, s1>>>(d.lab, m_voff, d_off, m_V, G,
+                                                                                   view ? view : packed);
         BHIP(hipGetLastError());
-        std::vector<uint32_t> gaps;
-        gaps.reserve(words - nverts - G);
-        for (uint32_t i = 0; i + 1 < G; i++)
-            gaps.insert(gaps.end(), lab + row_off[i] + V[i] + 1, lab + row_off[i + 1]);
-        uint32_t *const counts = reinterpret_cast<uint32_t *>(h_res + 2 * (size_t)capG);
-        if (nscc) BHIP(hipMemcpyAsync(counts, d.nscc, sizeof(uint32_t) * G, hipMemcpyDeviceToHost, s1));
-        BHIP(hipMemcpyAsync(lab + row_off[0], packed, sizeof(uint32_t) * words, hipMemcpyDeviceToHost, s1));
-        BHIP(hipStreamSynchronize(s1));
-        if (nscc) std::memcpy(nscc, counts, sizeof(uint32_t) * G);
-        const uint32_t *gap = gaps.data();
-        for (uint32_t i = 0; i + 1 < G; i++)
-            for (uint64_t k = row_off[i] + V[i] + 1; k < row_off[i + 1]; k++) lab[k] = *gap++;
-        return SCC_OK;
+        if (!view) {
+            scc_status s = spread_labels(packed, words, lab, each);
+            if (s != SCC_OK) return s;
+        }
     }
-    if (lab) {
-        std::vector<uint32_t> all(voff[G]);
-        BHIP(hipMemcpy(all.data(), d.lab, sizeof(uint32_t) * voff[G], hipMemcpyDeviceToHost));
-        parallel_chunks(G, [&](uint64_t lo, uint64_t hi, int) {
-            for (uint64_t i = lo; i < hi; i++)
-                std::memcpy(lab + row_off[i], all.data() + voff[i], sizeof(uint32_t) * ((size_t)V[i] + 1));
-        });
+    BHIP(hipStreamSynchronize(s1));
+    if (nscc) std::memcpy(nscc, counts, sizeof(uint32_t) * G);
+    return SCC_OK;
+}
+
+// The packed labels of all graphs, one graph after another, to their places
+// in the caller's buffer or buffers.
+scc_status BatchEngine::spread_labels(const uint32_t *packed, uint64_t words, uint32_t *lab, uint32_t *const *each)
+{
+    const uint64_t block = std::min(words, kLabelBlock);
+    if (block > label_words) {
+        if (h_label) (void)hipHostFree(h_label);
+        h_label = nullptr;
+        label_words = 0;
+        if (hipHostMalloc((void **)&h_label, sizeof(uint32_t) * 2 * block, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            return fail(SCC_ERR_NOMEM, "no page-locked memory for %llu labels", (unsigned long long)block);
+        }
+        label_words = block;
     }
-    if (nscc) BHIP(hipMemcpy(nscc, d.nscc, sizeof(uint32_t) * G, hipMemcpyDeviceToHost));
+    const uint64_t n = (words + block - 1) / block;
+    uint32_t g = 0;
+    uint64_t done = 0;   // words of graph g already in place
+    for (uint64_t k = 0; k <= n; k++) {
+        if (k < n) {
+            BHIP(hipMemcpyAsync(h_label + (k & 1) * block, packed + k * block,
+                                sizeof(uint32_t) * std::min(block, words - k * block), hipMemcpyDeviceToHost, s1));
+            if (k + 1 < n) BHIP(hipEventRecord(ev[k & 1], s1));
+        }
+        if (k == 0) continue;
+        if (k < n) BHIP(hipEventSynchronize(ev[(k - 1) & 1]));
+        else BHIP(hipStreamSynchronize(s1));
+        const uint32_t *src = h_label + ((k - 1) & 1) * block;
+        for (uint64_t left = std::min(block, words - (k - 1) * block); left;) {
+            const uint64_t take = std::min<uint64_t>(left, (uint64_t)V[g] + 1 - done);
+            std::memcpy((each ? each[g] : lab + row_off[g]) + done, src, sizeof(uint32_t) * take);
+            src += take;
+            left -= take;
+            done += take;
+            if (done == (uint64_t)V[g] + 1) {
+                g++;
+                done = 0;
+            }
+        }
+    }
     return SCC_OK;
 }
 

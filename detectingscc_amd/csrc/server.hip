@@ -191,7 +191,8 @@ void Server::worker(int slot)
         init_err = "cannot create a stream for a server slot";
     std::vector<Req *> batch;
     scc_batch_host h;
-    std::vector<uint32_t> hV, hE, Fr, Br, Fc, Bc, nscc, lab;
+    std::vector<uint32_t> hV, hE, Fr, Br, Fc, Bc, nscc;
+    std::vector<uint32_t *> lab;
     std::vector<uint64_t> ro, co;
     for (;;) {
         uint64_t taken = 0;
@@ -209,7 +210,13 @@ void Server::worker(int slot)
         const uint32_t G = (uint32_t)batch.size();
         ro.assign(G + 1, 0);
         for (uint32_t i = 0; i < G; i++) ro[i + 1] = ro[i] + batch[i]->V + 2;
-        lab.resize(ro[G]);
+        // the labels go straight to their requests (nobody looks at a
+        // request's before it is done)
+        lab.resize(G);
+        for (uint32_t i = 0; i < G; i++) {
+            batch[i]->lab.resize((size_t)batch[i]->V + 1);
+            lab[i] = batch[i]->lab.data();
+        }
         nscc.resize(G);
         scc_status st = init_err.empty() ? SCC_OK : fail(SCC_ERR_DEVICE, "%s", init_err.c_str());
         if (st == SCC_OK && batch[0]->solo) {
@@ -223,7 +230,7 @@ void Server::worker(int slot)
                                       true);   // checked when it was submitted
             scc_stats sst;
             if (st == SCC_OK) st = solo_eng->run(solo_opts, &sst);
-            if (st == SCC_OK) st = solo_eng->labels(lab.data());
+            if (st == SCC_OK) st = solo_eng->labels(lab[0]);
             nscc[0] = sst.num_sccs;
         } else if (st == SCC_OK) {
             // pack the batch in the reference layout, one graph after another
@@ -258,7 +265,7 @@ void Server::worker(int slot)
             scc_batch_stats bst;
             st = be->upload(dev, stream, &h, true);   // checked when they were submitted
             if (st == SCC_OK) st = be->run(opts, &bst);
-            if (st == SCC_OK) st = be->labels(lab.data(), nscc.data());
+            if (st == SCC_OK) st = be->labels(nullptr, nscc.data(), lab.data());
         }
         const std::string err = st == SCC_OK ? std::string() : std::string(scc_last_error());
         const auto now = clock::now();
@@ -274,7 +281,6 @@ void Server::worker(int slot)
                 std::vector<uint32_t>().swap(r->Fc);
                 std::vector<uint32_t>().swap(r->Bc);
                 if (st == SCC_OK) {
-                    r->lab.assign(lab.begin() + ro[i], lab.begin() + ro[i] + r->V + 1);
                     r->nscc = nscc[i];
                     latencies.push_back(std::chrono::duration<double, std::milli>(now - r->arrival).count());
                     completed++;

@@ -322,7 +322,8 @@ scc_status scc_batch_run_serial(scc_ctx *ctx, const scc_opts *opts, scc_batch_st
  * bucket in one launch; a text report of the choices goes to `report`
  * (may be NULL).  Labels of the uploaded batch are overwritten. */
 scc_status scc_batch_autotune(scc_ctx *ctx, int sample, char *report, size_t report_len);
-/* Labels (row_off layout: V[i]+1 entries at row_off[i]) and SCC counts. */
+/* Labels (row_off layout: V[i]+1 entries at row_off[i]; no other word of
+ * lab is written) and SCC counts. */
 scc_status scc_batch_labels(scc_ctx *ctx, uint32_t *lab, uint32_t *nscc);
 
 /* ----------------------------------------------------------- serving --- */

@@ -3,8 +3,11 @@ where they change path: graphs at the edges of a chunk (64 vertices) and of
 the LDS tiers, with hubs walked by the whole workgroup, sparse enough to be
 trimmed and searched top-down only, dense enough for bottom-up levels, and
 with thousands of SCCs that the first round leaves to the list phases."""
+import threading
+
 import numpy as np
 import pytest
+import torch
 
 import detectingscc_amd as scc
 from oracle import pyoracle as orc
@@ -117,4 +120,46 @@ def test_batch_labels_row_order(starts):
         assert_same_labels(lab[at:at + 101], want, f"rows at {starts}, graph {i}")
         assert nscc[i] == k
         lab[at:at + 101] = 0xABCD
+    assert (lab == 0xABCD).all()
+
+
+@pytest.mark.parametrize("pinned", [False, True])
+@pytest.mark.parametrize("spacing", [0, 61])
+def test_batch_labels_gaps_stay_the_callers(pinned, spacing):
+    """A word between two graphs' labels that another thread counts in while
+    the labels are copied loses no count, in pageable and page-locked memory."""
+    rng = np.random.default_rng(spacing)
+    gs = [random_graph(V, 2 * V, rng) for V in rng.integers(1, 6000, 700)]
+    b = scc.batch_from_graphs(gs)
+    row = np.zeros(len(gs) + 1, np.uint64)
+    row[1:] = np.cumsum([g.V + 2 + spacing for g in gs])
+    Fr, Br = np.zeros(int(row[-1]), np.uint32), np.zeros(int(row[-1]), np.uint32)
+    for at, g in zip(row.astype(int), gs):
+        Fr[at:at + g.V + 2], Br[at:at + g.V + 2] = g.Fr, g.Br
+    b = scc.Batch(b.V, b.E, row, b.col_off, Fr, b.Fc, Br, b.Bc)
+    lab = torch.full((int(row[-1]),), 0xABCD, dtype=torch.int32, pin_memory=pinned).numpy().view(np.uint32)
+    mine = int(row[len(gs) // 2]) + gs[len(gs) // 2].V + 1
+    lab[mine] = 0
+    counted, stop = 0, threading.Event()
+
+    def count():
+        nonlocal counted
+        while not stop.is_set():
+            lab[mine] += 1
+            counted += 1
+
+    with scc.Context(0) as ctx:
+        ctx.batch_upload(b)
+        ctx.batch_run()
+        t = threading.Thread(target=count)
+        t.start()
+        status = [scc.lib().scc_batch_labels(ctx._ctx, scc._p32(lab), None) for _ in range(20)]
+        stop.set()
+        t.join()
+    assert status == [0] * 20 and counted > 0
+    assert int(lab[mine]) == counted & 0xFFFFFFFF
+    lab[mine] = 0xABCD
+    for i, (at, g) in enumerate(zip(row.astype(int), gs)):
+        assert_same_labels(lab[at:at + g.V + 1], orc.tarjan(g)[0], f"graph {i}")
+        lab[at:at + g.V + 1] = 0xABCD
     assert (lab == 0xABCD).all()
