@@ -177,6 +177,7 @@ scc_status BatchEngine::finish_upload(bool check)
     BHIP(hipMemcpyAsync(m_eoff, eoff.data(), sizeof(uint64_t) * (G + 1), hipMemcpyHostToDevice, s1));
     BHIP(hipMemcpyAsync(m_V, V.data(), sizeof(uint32_t) * G, hipMemcpyHostToDevice, s1));
     if (check) {
+        (void)hipGetLastError();   // an earlier call's error is not this launch's
         k_fill_u32(s1, m_meta, 0u, 1);
         const uint32_t cols = std::min<uint32_t>(64, std::max<uint32_t>(1, 4096 / G));
         batch_check_kernel<<<dim3(std::min<uint32_t>(G, 8192), cols), 256, 0, s1>>>(m_voff, m_eoff, m_V, m_Fr, m_Br,
@@ -332,6 +333,7 @@ scc_status BatchEngine::launch(const std::vector<uint32_t> &idx, const std::vect
     BHIP(hipEventRecord(ev[0], s1));
     if (two) BHIP(hipStreamWaitEvent(stream2, ev[0], 0));
     uint32_t nl = 0;
+    (void)hipGetLastError();   // an earlier call's error is not these launches'
     for (size_t gidx = 0; gidx < groups.size(); gidx++) {
         const int bs = groups[gidx].first;
         const uint32_t first = groups[gidx].second.first, count = groups[gidx].second.second;
@@ -597,6 +599,7 @@ scc_status BatchEngine::labels(uint32_t *lab, uint32_t *nscc, uint32_t *const *e
         uint64_t *const d_off = reinterpret_cast<uint64_t *>(d.q + 2 * capS);
         BHIP(hipMemcpyAsync(d_off, off, sizeof(uint64_t) * G, hipMemcpyHostToDevice, s1));
         const uint32_t cols = std::min<uint32_t>(64, std::max<uint32_t>(1, 4096 / G));
+        (void)hipGetLastError();   // an earlier call's error is not this launch's
         batch_pack_kernel<<<dim3(std::min<uint32_t>(G, 8192), cols), 256, 0, s1>>>(d.lab, m_voff, d_off, m_V, G,
                                                                                    view ? view : packed);
         BHIP(hipGetLastError());

@@ -97,6 +97,7 @@ scc_status Engine::init(int dev)
     // on the engine's stream: it does not wait for the null stream, where a
     // memset may still be queued (behind another engine's kernels, say) when
     // this call returns, and would then clear the counters of a later run
+    (void)hipGetLastError();   // an earlier call's error, the caller's own perhaps, is not this launch's
     k_fill_u32(stream, st.ctr, 0u, CT(kCtrLines));
     HIP_TRY(hipGetLastError());
     // counters published into mapped, coherent host memory: C_COUNT lines
@@ -291,13 +292,19 @@ scc_status Engine::upload(uint32_t V, uint32_t E, const uint32_t *Fr, const uint
     }
     DevGraph &to = on_device && keep ? spare : g;
     uint32_t *const flag = h_pub ? h_pub + CT(C_COUNT) + kCheckWord : nullptr;
-    if (on_device) flag[0] = flag[1] = 0;
+    if (on_device) {
+        flag[0] = flag[1] = 0;
+        (void)hipGetLastError();   // an earlier call's
+    }
     const uint32_t *const rows[2] = {Fr, Br}, *const cols[2] = {Fc, Bc};
     uint32_t *const drows[2] = {to.Fr, to.Br}, *const dcols[2] = {to.Fc, to.Bc};
     for (int d = 0; d < 2; d++) {
         HIP_TRY(hipMemcpyAsync(drows[d], rows[d], sizeof(uint32_t) * ((size_t)V + 2), hipMemcpyHostToDevice, stream));
         if (E) HIP_TRY(hipMemcpyAsync(dcols[d], cols[d], sizeof(uint32_t) * E, hipMemcpyHostToDevice, stream));
-        if (on_device) k_check_csr(stream, drows[d], dcols[d], V, E, d_pub + CT(C_COUNT) + kCheckWord + d);
+        if (on_device) {
+            k_check_csr(stream, drows[d], dcols[d], V, E, d_pub + CT(C_COUNT) + kCheckWord + d);
+            HIP_TRY(hipGetLastError());   // a check that did not run finds nothing wrong
+        }
     }
     HIP_TRY(hipStreamSynchronize(stream));
     if (on_device && (flag[0] || flag[1])) {
