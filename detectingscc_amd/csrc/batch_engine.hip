@@ -453,7 +453,9 @@ scc_status BatchEngine::run_serial(Engine &eng, const scc_opts &o, scc_batch_sta
         lat[i] = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     }
     const double ms = lat.empty() ? 0 : lat.back();
-    BHIP(hipMemcpy(d.nscc, nscc.data(), sizeof(uint32_t) * G, hipMemcpyHostToDevice));
+    // on the stream that labels() reads the counts on
+    BHIP(hipMemcpyAsync(d.nscc, nscc.data(), sizeof(uint32_t) * G, hipMemcpyHostToDevice, s1));
+    BHIP(hipStreamSynchronize(s1));
     if (out) {
         std::memset(out, 0, sizeof *out);
         out->graphs = G;
