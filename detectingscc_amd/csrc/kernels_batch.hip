@@ -109,14 +109,14 @@ struct G1 {
     uint64_t *piv;
     // four arrays of V+2 words: 0 and 2 are the FW and BW queues (each
     // vertex enters a search's queue once, so a queue is never reused within
-    // a search), 1 holds the first out-neighbours and then the list of the
-    // vertices the first round left, 3 the live bitmap of a graph too large
-    // for LDS
+    // a search), 1 holds the first out-neighbours and then (batch) the list
+    // of the vertices the first round left, 3 the live bitmap of a graph too
+    // large for LDS
     uint32_t *q;
     __device__ __forceinline__ uint32_t *queue(uint32_t k) const { return q + (size_t)k * (V + 2); }
     __device__ __forceinline__ uint32_t *f1() const { return queue(1); }
     __device__ __forceinline__ uint32_t *b1() const { return aux; }   // first in-neighbours (first round only)
-    __device__ __forceinline__ uint32_t *list() const { return queue(1); }
+    uint32_t *list;   // the vertices the first round left, V+2 words
     uint32_t *pivlist;
 };
 
@@ -784,7 +784,7 @@ __device__ __forceinline__ void g_first_search(Lds &L, const G1 &g, uint32_t nli
 }
 
 // ----------------------------------------------- the later phases ---
-// Over the `n` vertices the first round left (g.list()), in classes.
+// Over the `n` vertices the first round left (g.list), in classes.
 
 #define LIST_LOOP(v)                                                                        \
     for (uint32_t _i = threadIdx.x, v; _i < n && (v = at(list, _i), true); _i += BS)
@@ -795,7 +795,7 @@ __device__ __forceinline__ void g_first_search(Lds &L, const G1 &g, uint32_t nli
 
 template <int BS> __device__ __forceinline__ void g_trim1(Lds &L, const G1 &g, uint32_t n)
 {
-    const uint32_t *list = g.list();
+    const uint32_t *list = g.list;
     for (uint32_t pass = 0; pass <= g.V; pass++) {   // each pass removes a vertex or ends
         uint32_t removed = 0;
         WAVE_LIST_LOOP(v)
@@ -843,7 +843,7 @@ __device__ __forceinline__ bool g_arc(const uint32_t *R, const uint32_t *C, uint
 // trim-2 (scc_kernels.cu:236-357), claim by CAS on the smaller id
 template <int BS> __device__ __forceinline__ void g_trim2(Lds &L, const G1 &g, uint32_t n)
 {
-    const uint32_t *list = g.list();
+    const uint32_t *list = g.list;
     LIST_LOOP(v)
     {
         const uint32_t c = g.cls[v];
@@ -910,7 +910,7 @@ template <int BS> __device__ __forceinline__ void g_reach(Lds &L, const G1 &g, b
 // One pivot per live class, seeded in both directions.
 template <int BS> __device__ __forceinline__ void g_pivots(Lds &L, const G1 &g, uint32_t n)
 {
-    const uint32_t *list = g.list();
+    const uint32_t *list = g.list;
     // a wave whose live lanes share a class does one atomic
     unsigned long long *piv = reinterpret_cast<unsigned long long *>(g.piv);
     for (uint32_t i0 = threadIdx.x & ~63u; i0 < n; i0 += BS) {
@@ -959,10 +959,11 @@ template <int BS> __device__ __forceinline__ void g_pivots(Lds &L, const G1 &g, 
     __syncthreads();
 }
 
-// update (scc_kernels.cu:124-142) + clear the next round's pivot slots
+// update (scc_kernels.cu:124-142) + clear the next round's pivot slots, if
+// there is one
 template <int BS> __device__ __forceinline__ uint32_t g_update(Lds &L, const G1 &g, uint32_t n)
 {
-    const uint32_t *list = g.list();
+    const uint32_t *list = g.list;
     uint32_t live = 0;
     LIST_LOOP(v)
     {
@@ -983,6 +984,7 @@ template <int BS> __device__ __forceinline__ uint32_t g_update(Lds &L, const G1 
         }
     }
     const uint32_t left = wg_sum1<BS>(L, live);
+    if (!left) return 0;   // nothing reads the keys of a graph that is done
     for (uint32_t i = threadIdx.x; i < L.npiv; i += BS) {
         const uint32_t p = g.pivlist[i];
         g.piv[3ull * p] = 0;
@@ -996,7 +998,7 @@ template <int BS> __device__ __forceinline__ uint32_t g_update(Lds &L, const G1 
 // "WCC" min reachable label with pointer jumping (scc_kernels.cu:477-536)
 template <int BS> __device__ __forceinline__ void g_minlabel(Lds &L, const G1 &g, uint32_t n)
 {
-    const uint32_t *list = g.list();
+    const uint32_t *list = g.list;
     LIST_LOOP(v)
         if (g.cls[v] != DEAD) g.cls[v] = v;
     __syncthreads();
@@ -1037,7 +1039,7 @@ template <int BS> __device__ __forceinline__ void g_minlabel(Lds &L, const G1 &g
 // vertex outside the list
 template <int BS> __device__ __forceinline__ void g_color_loop(Lds &L, const G1 &g, uint32_t n)
 {
-    const uint32_t *list = g.list();
+    const uint32_t *list = g.list;
     uint32_t live = n;
     for (uint32_t round = 0; live && round <= g.V; round++) {   // a round finishes >= 1 SCC
         LIST_LOOP(v)
@@ -1102,13 +1104,15 @@ template <int BS> __device__ __forceinline__ void g_color_loop(Lds &L, const G1 
 }
 
 // Canonical labels of the listed vertices; returns their number of SCCs.
-// The minimum per label: lanes of a wave that share a label combine first
-// (up to four labels per wave step, then lane by lane), and the guard reads
-// the current minimum at agent scope (the CU's L1 may hold a stale copy),
-// so a large SCC costs about one atomic per wave instead of one per vertex.
+// The minimum per label: the lanes of a wave that share its first label
+// combine, the others go lane by lane, and the guard reads the current
+// minimum at agent scope (the CU's L1 may hold a stale copy), so a large SCC
+// costs about one atomic per wave instead of one per vertex.  Combining up to
+// four labels per step made the pass 70 us on 16,384 vertices in 5,466 SCCs,
+// so 55.
 template <int BS> __device__ __forceinline__ uint32_t g_canon(Lds &L, const G1 &g, uint32_t n)
 {
-    const uint32_t *list = g.list();
+    const uint32_t *list = g.list;
     LIST_LOOP(v)
         g.aux[v] = DEAD;
     __syncthreads();
@@ -1116,22 +1120,19 @@ template <int BS> __device__ __forceinline__ uint32_t g_canon(Lds &L, const G1 &
         const uint32_t v = i0 + ln() < n ? at(list, i0 + ln()) : 0u;
         const uint32_t l = v ? g.lab[v] : LAB_FINAL;
         bool pending = !(l & LAB_FINAL);
-        for (int it = 0; it < 4; it++) {
-            const uint64_t pm = __ballot(pending);
-            if (!pm) break;
-            const int lead = __ffsll((unsigned long long)pm) - 1;
-            const uint32_t rl = __shfl(l, lead);
-            const bool mine = pending && l == rl;
-            uint32_t m = mine ? v : DEAD;
-            for (int o = 32; o > 0; o >>= 1) {
-                const uint32_t x = __shfl_xor(m, o);
-                m = x < m ? x : m;
-            }
-            if ((int)ln() == lead &&
-                m < __hip_atomic_load(&g.aux[rl], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-                atomicMin(&g.aux[rl], m);
-            pending = pending && !mine;
+        const uint64_t pm = __ballot(pending);
+        if (!pm) continue;
+        const int lead = __ffsll((unsigned long long)pm) - 1;
+        const uint32_t rl = (uint32_t)__builtin_amdgcn_readlane((int)l, lead);
+        const bool mine = pending && l == rl;
+        uint32_t m = mine ? v : DEAD;
+        for (int o = 32; o > 0; o >>= 1) {
+            const uint32_t x = __shfl_xor(m, o);
+            m = x < m ? x : m;
         }
+        if ((int)ln() == lead && m < __hip_atomic_load(&g.aux[rl], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+            atomicMin(&g.aux[rl], m);
+        pending = pending && !mine;
         if (pending && v < __hip_atomic_load(&g.aux[l], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
             atomicMin(&g.aux[l], v);
     }
@@ -1226,7 +1227,7 @@ __device__ __forceinline__ uint32_t g_solve(Lds &L, const G1 &g, uint32_t cfg)
     // Vertices are left: their classes and the list of them.  Every other
     // label is final.  Class 3 p0 + k needs its pivot key cleared.
     const bool slota = cfg_slota(cfg);
-    uint32_t *list = g.list();   // the first out-neighbours are not needed any more
+    uint32_t *list = g.list;   // the first out-neighbours are not needed any more
     for (uint32_t c0 = uni(threadIdx.x >> 6); c0 < nch; c0 += BS / 64) {
         const uint32_t v = c0 * 64 + ln(), i = 2 * c0 + (ln() >> 5), sh = ln() & 31;
         const uint32_t lw = g.live[i], f = (g.fvis[i] >> sh) & 1u, b = (g.bvis[i] >> sh) & 1u;
@@ -1318,6 +1319,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) void ba
         g.aux = B.aux + vo;
         g.piv = B.piv + 3 * vo;
         g.q = B.q + 4 * vo;
+        g.list = g.queue(1);
         g.pivlist = B.pivlist + vo;
         uint32_t n;
         if (2 * ((g.V + 64) / 64) > BTier<BS>::words) {
@@ -1358,15 +1360,24 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) void ba
 // 16 arcs per vertex: 1,000 vertices 58 / 39 / 29 / 26 us against 120 / 112 /
 // 123 / 98, 8,000 vertices 125 / 90 / 78 / 56 against 407 / 134 / 116 / 107,
 // 16,384 vertices 193 / 139 / 94 / 87 against 388 / 149 / 121 / 108; at
-// 32,768 vertices it would be 250 against 148 at 4 arcs.
-constexpr uint32_t SMALL_LDS = 36864;   // words: class words, or everything of a graph that fits
+// 32,768 vertices it would be 250 against 148 at 4 arcs.  Structured graphs
+// of 16,384 vertices: a 0.7 grid 524 against 734, islands of up to nine 713
+// against 2,140, rings of 16 1,230 against 6,660, a path 54,000 against
+// 74,000, a chain of 2-cycles 62,000 against 207,000.  Slower here are a
+// cycle (14.7 against 9.7 ms, 4,096 vertices 3.6 against 2.1: a hop of the
+// device-wide engine's low-degree levels is one memory trip, a narrow level
+// two; nothing known before the launch tells it from a path) and, with the
+// trims off, a star without a cycle (207 against 186): one CU does all its
+// scattered key accesses.  What is left after the first round is listed in
+// LDS beside the class words (16,384 vertices in 5,466 SCCs 358 -> 344).
+constexpr uint32_t SMALL_LDS = 36864;   // words: class words and list, or everything of a graph that fits
 
 __global__ __launch_bounds__(1024) void small_scc_kernel(SmallArgs a)
 {
     __shared__ Lds L;
     __shared__ uint32_t s_bits[3][2 * ((SMALL_V + 64) / 64)];
     __shared__ uint32_t s_mem[SMALL_LDS];
-    static_assert(SMALL_V + 1 <= SMALL_LDS, "the class words fit");
+    static_assert(2 * SMALL_V + 3 <= SMALL_LDS, "the class words and the list of vertices left fit");
     const uint64_t t0 = wall_clock64();
     G1 g;
     g.V = a.V;
@@ -1384,6 +1395,7 @@ __global__ __launch_bounds__(1024) void small_scc_kernel(SmallArgs a)
         uint32_t *Fr = s_mem + nr, *Br = Fr + nr, *Fc = Br + nr, *Bc = Fc + a.E;
         g.aux = Bc + a.E;
         g.q = g.aux + nr;   // 4 * nr words
+        g.list = g.queue(1);
         for (uint32_t i = threadIdx.x; i < nr; i += 1024) {
             Fr[i] = a.Fr[i];
             Br[i] = a.Br[i];
@@ -1405,6 +1417,7 @@ __global__ __launch_bounds__(1024) void small_scc_kernel(SmallArgs a)
         g.Bc = a.Bc;
         g.aux = a.aux;
         g.q = a.q;
+        g.list = s_mem + SMALL_V + 1;
         n = g_solve<1024, 1>(L, g, a.cfg);
     }
     __syncthreads();
