@@ -320,10 +320,11 @@ __device__ __forceinline__ uint32_t g_fold(const uint32_t *C, uint32_t i, uint32
 
 // Degrees: the live bitmap (vertices with an in- and an out-arc; all of them
 // with the trims off) and the best pivot key among them, which goes to
-// L.key.  Returns the number of vertices that are not live.
+// L.key.  Returns the number of vertices that are not live.  FULL: they are
+// listed in queue 0 for g_trim_listed.
 constexpr uint32_t DEG_CHUNKS = 4;
 
-template <int BS> __device__ __forceinline__ uint32_t g_degrees(Lds &L, const G1 &g, bool trim)
+template <int BS, bool FULL> __device__ __forceinline__ uint32_t g_degrees(Lds &L, const G1 &g, bool trim)
 {
     const uint32_t nch = (g.V + 64) / 64;
     unsigned long long best = 0;
@@ -346,6 +347,7 @@ template <int BS> __device__ __forceinline__ uint32_t g_degrees(Lds &L, const G1
             gone += in && !alive;
             const uint64_t m = __ballot(alive);
             if (ch < nch && ln() < 2) g.live[2 * ch + ln()] = ln() ? (uint32_t)(m >> 32) : (uint32_t)m;
+            if (FULL) lpush(in && !alive && (fe[h] > fb[h] || be[h] > bb[h]), v, g.queue(0), &L.tail[0]);
             if (alive) {
                 const unsigned long long k = bkey_deg(fe[h] - fb[h], be[h] - bb[h], v);
                 best = k > best ? k : best;
@@ -375,13 +377,19 @@ template <int BS> __device__ __forceinline__ uint32_t g_degrees(Lds &L, const G1
 // direction, costs more than what it would remove (mix 3.05 -> 2.69 ms).
 constexpr uint32_t TRIM_CHUNKS = 4;
 constexpr uint32_t TRIM_STOP = 32;
+// FULL: queue 0 lists what the last pass removed, for g_trim_listed.
 constexpr uint32_t TRIM_MIN = 8;
 
-template <int BS> __device__ __forceinline__ void g_trim_bits(Lds &L, const G1 &g)
+template <int BS, bool FULL> __device__ __forceinline__ void g_trim_bits(Lds &L, const G1 &g)
 {
     const uint32_t nch = (g.V + 64) / 64;
     uint32_t *F1 = g.f1(), *B1 = g.b1();
     for (uint32_t pass = 0; pass <= g.V; pass++) {   // each pass removes a vertex or ends
+        if (FULL) {
+            __syncthreads();
+            if (threadIdx.x == 0) L.tail[0] = 0;
+            __syncthreads();
+        }
         uint32_t removed = 0;                        // wave-uniform
         for (uint32_t c0 = uni(threadIdx.x >> 6); c0 < nch; c0 += TRIM_CHUNKS * (BS / 64)) {
             uint32_t word[TRIM_CHUNKS], pin[TRIM_CHUNKS], pout[TRIM_CHUNKS];
@@ -463,7 +471,9 @@ template <int BS> __device__ __forceinline__ void g_trim_bits(Lds &L, const G1 &
 #pragma unroll
                 for (uint32_t h = 0; h < TRIM_CHUNKS; h++) {
                     const uint32_t ch = c0 + h * (BS / 64);
-                    const uint64_t m = __ballot(!x[2 * h] || !x[2 * h + 1]);
+                    const bool out = !x[2 * h] || !x[2 * h + 1];
+                    const uint64_t m = __ballot(out);
+                    if (FULL) lpush(out, ch * 64 + ln(), g.queue(0), &L.tail[0]);
                     const uint32_t mw = ln() < 32 ? (uint32_t)m : (uint32_t)(m >> 32);
                     if ((ln() & 31) == 0 && mw) g.live[2 * ch + (ln() >> 5)] = word[h] & ~mw;
                     removed += (uint32_t)__popcll(m);
@@ -471,6 +481,76 @@ template <int BS> __device__ __forceinline__ void g_trim_bits(Lds &L, const G1 &
             }
         }
         if ((uint64_t)wg_sum<BS>(L, ln() == 0 ? removed : 0u, pass & 1) * TRIM_STOP <= g.V) break;
+    }
+    __syncthreads();
+}
+
+// A live neighbour w (0: none) that lost an out-arc (d = 1) or in-arc (d = 0)
+// goes too, and is listed in queue 0, unless another live arc that way is
+// left.  All 64 lanes of the wave call.
+__device__ __forceinline__ void g_recheck(Lds &L, const G1 &g, uint32_t d, uint32_t w)
+{
+    const uint32_t *R = d ? g.Fr : g.Br, *const C[1] = {d ? g.Fc : g.Bc};
+    const uint32_t r = bbit(g.live, w) ? w : 0u;   // row 0 is empty
+    if (!__ballot(r != 0)) return;
+    uint32_t i[1] = {at(R, r)}, x[1];
+    const uint32_t e[1] = {at(R, r + 1)};
+    g_any_bit<1>(C, i, e, g.live, x);
+    const uint32_t bit = 1u << (w & 31);
+    const bool gone = r && !x[0] && (atomicAnd(&g.live[w >> 5], ~bit) & bit);
+    lpush(gone, w, g.queue(0), &L.tail[0]);
+}
+
+// trim-1 on to its fixpoint, from the removed vertices in queue 0 that no
+// pass has followed up yet.  For the small-graph kernel under Hong's order,
+// whose pivot and counts then are those of trim-1's fixpoint, as the
+// device-wide engine reports them.  The arcs of many vertices are balanced
+// over their wave, as in g_expand; few vertices get several waves each.
+// 16,384 vertices and 139,000 arcs 123 -> 125 us, 999 vertices 50.5 -> 46.7,
+// a path of 16,384 54 -> 10.8 ms (its trims left to g_trim1 before), a star
+// without a cycle 89 -> 97 us.
+template <int BS> __device__ __forceinline__ void g_trim_listed(Lds &L, const G1 &g)
+{
+    const uint32_t *q = g.queue(0);
+    const uint32_t wv = uni(threadIdx.x >> 6), nwv = BS / 64, d = wv & 1, w = wv >> 1, nw = nwv / 2;
+    const uint32_t *R = d ? g.Br : g.Fr, *C = d ? g.Bc : g.Fc;
+    __syncthreads();
+    for (uint32_t lo = 0, hi = uni(L.tail[0]); lo != hi;) {   // each pass but the last lists a vertex
+        __syncthreads();   // every lane has read the tail
+        const uint32_t n = hi - lo;
+        if (n < nw) {
+            const uint32_t each = nw / n;   // waves per vertex and side
+            if (w / each < n) {
+                const uint32_t u = at(q, lo + w / each);
+                for (uint32_t j = at(R, u) + 64 * (w % each), end = at(R, u + 1); j < end; j += 64 * each)
+                    g_recheck(L, g, d, j + ln() < end ? C[j + ln()] : 0u);
+            }
+        } else {
+            const uint32_t per = min(64u, (n + nw - 1) / nw);
+            for (uint32_t t = lo + per * w; t < hi; t += per * nw) {
+                const uint32_t u = ln() < per && t + ln() < hi ? at(q, t + ln()) : 0u;   // row 0 is empty
+                const uint32_t b = at(R, u), deg = at(R, u + 1) - b;
+                uint32_t sum = deg;   // inclusive
+                for (int o = 1; o < 64; o <<= 1) {
+                    const uint32_t y = __shfl_up(sum, o);
+                    if ((int)ln() >= o) sum += y;
+                }
+                const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)sum, 63);
+                const uint32_t start = b - (sum - deg);   // arc j of the tile is C[start + j], modulo 2^32
+                for (uint32_t j0 = 0; j0 < total; j0 += 64) {
+                    const uint32_t j = j0 + ln();
+                    uint32_t own = 0;
+#pragma unroll
+                    for (uint32_t o = 32; o >= 1; o >>= 1)
+                        own += (uint32_t)__shfl((int)sum, (int)(own + o - 1)) <= j ? o : 0u;
+                    const uint32_t st = __shfl(start, (int)own);   // past the end `own` is 63, and the load is skipped
+                    g_recheck(L, g, d, j < total ? C[st + j] : 0u);
+                }
+            }
+        }
+        __syncthreads();
+        lo = hi;
+        hi = uni(L.tail[0]);
     }
     __syncthreads();
 }
@@ -1151,7 +1231,7 @@ template <int BS> __device__ __forceinline__ uint32_t g_canon(Lds &L, const G1 &
 // The whole pipeline of one graph; returns its number of SCCs.  LDS_BITS /
 // LDS_CLS only say which memory the views point to: the code is the same,
 // and inlined per case so that the accesses are LDS instructions.
-template <int BS, uint32_t BUC = BU_CHUNKS>
+template <int BS, uint32_t BUC = BU_CHUNKS, bool FULL = false>
 __device__ __forceinline__ uint32_t g_solve(Lds &L, const G1 &g, uint32_t cfg)
 {
     const uint32_t nch = (g.V + 64) / 64, nw = 2 * nch;
@@ -1160,12 +1240,15 @@ __device__ __forceinline__ uint32_t g_solve(Lds &L, const G1 &g, uint32_t cfg)
         L.nhub = 0;
         L.nact = 0;
         L.anom = 0;
+        L.tail[0] = 0;
         L.st = GraphStats();
     }
     __syncthreads();
-    const uint32_t ndeg = g_degrees<BS>(L, g, cfg_t1(cfg));
-    const bool first = (uint64_t)ndeg * TRIM_MIN > g.V;   // never with the trims off
-    if (first) g_trim_bits<BS>(L, g);
+    const uint32_t ndeg = g_degrees<BS, FULL>(L, g, cfg_t1(cfg));
+    // (never with the trims off; FULL: colouring trims once, as in the device-wide engine)
+    const bool first = (uint64_t)ndeg * TRIM_MIN > g.V && !(FULL && cfg_slota(cfg));
+    if (first) g_trim_bits<BS, FULL>(L, g);
+    if (FULL && cfg_t1(cfg) && !cfg_slota(cfg)) g_trim_listed<BS>(L, g);
     uint32_t nl = 0;
     for (uint32_t i = threadIdx.x; i < nw; i += BS) {
         nl += (uint32_t)__popc(g.live[i]);
@@ -1409,7 +1492,7 @@ __global__ __launch_bounds__(1024) void small_scc_kernel(SmallArgs a)
         g.Fc = Fc;
         g.Bc = Bc;
         __syncthreads();
-        n = g_solve<1024, 1>(L, g, a.cfg);
+        n = g_solve<1024, 1, true>(L, g, a.cfg);
     } else {
         g.Fr = a.Fr;
         g.Br = a.Br;
@@ -1418,7 +1501,7 @@ __global__ __launch_bounds__(1024) void small_scc_kernel(SmallArgs a)
         g.aux = a.aux;
         g.q = a.q;
         g.list = s_mem + SMALL_V + 1;
-        n = g_solve<1024, 1>(L, g, a.cfg);
+        n = g_solve<1024, 1, true>(L, g, a.cfg);
     }
     __syncthreads();
     if (threadIdx.x != 0) return;

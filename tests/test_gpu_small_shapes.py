@@ -109,3 +109,51 @@ def test_long_rows_do_not_hold_a_lane():
                 best = min(best, time.perf_counter() - t0)
             ms[wide] = best * 1e3
     assert ms[False] * 3 < ms[True], ms
+
+
+def _trimmed(g, once):
+    """Live vertices after trim-1: one pass, or the fixpoint."""
+    src = np.repeat(np.arange(g.V + 1), np.diff(g.Fr.astype(np.int64)))
+    dst = g.Fc.astype(np.int64)
+    live = np.arange(g.V + 1) > 0
+    while True:
+        ok = live[src] & live[dst]
+        keep = live & (np.bincount(src[ok], minlength=g.V + 1) > 0) & (np.bincount(dst[ok], minlength=g.V + 1) > 0)
+        if once or (keep == live).all():
+            return keep
+        live = keep
+
+
+def _hub_dag(V, rng):
+    """A random SCC and a vertex of many arcs that only trim-1's second pass
+    removes: sources to it, it to sinks."""
+    k = V // 20
+    body = V - 2 * k - 1
+    hub = body + 1
+    ring = np.arange(1, body + 1)
+    return V, [ring, rng.integers(1, body + 1, 4 * body), np.arange(hub + 1, hub + 1 + k), np.full(k, hub), [hub]], [
+        np.roll(ring, -1), rng.integers(1, body + 1, 4 * body), np.full(k, hub), np.arange(hub + 1 + k, V + 1), [1]]
+
+
+@pytest.mark.parametrize("V", [900, 1700, 4000, 16384])
+@pytest.mark.parametrize("arcs", ["hub", 2, 4, 8])
+def test_small_counts(V, arcs):
+    """What is trimmed, and the pivot elected from the rest: trim-1 to its
+    fixpoint under Hong's order, one pass of it before colouring."""
+    g = _graph(_hub_dag, V) if arcs == "hub" else scc.gen_er(V, arcs * V, 4, 2, 64, seed=V)
+    _, n = orc.tarjan(g)
+    Fr, Br = g.Fr.astype(np.int64), g.Br.astype(np.int64)
+    product = np.minimum(np.diff(Fr) * np.diff(Br), 0xFFFFFFFF)
+    with scc.Context(0) as ctx:
+        ctx.upload(g)
+        for algo in "gxhy":
+            st = ctx.run(algo=algo, trim1=True, trim2=False, sizes=False)
+            live = _trimmed(g, once=algo in "hy")
+            first = int(np.argmax(np.where(live, product, -1)))
+            assert st.first_pivot == first, f"-a {algo}"
+            if algo in "hy":
+                assert st.num_trim1 == g.V - live.sum()
+            elif arcs == "hub":
+                assert (st.num_trim1, st.num_pivot) == (n - 1, 1)
+            else:
+                assert st.num_trim1 >= g.V - live.sum()
