@@ -106,6 +106,7 @@ struct G1 {
     const uint32_t *Fr, *Fc, *Br, *Bc;
     uint32_t *cls, *lab, *aux;
     uint32_t *live, *fvis, *bvis;   // one bit per vertex
+    uint32_t *seen;                 // two such bitmaps (g_trim_listed), one after the other
     uint64_t *piv;
     // four arrays of V+2 words: 0 and 2 are the FW and BW queues (each
     // vertex enters a search's queue once, so a queue is never reused within
@@ -320,11 +321,10 @@ __device__ __forceinline__ uint32_t g_fold(const uint32_t *C, uint32_t i, uint32
 
 // Degrees: the live bitmap (vertices with an in- and an out-arc; all of them
 // with the trims off) and the best pivot key among them, which goes to
-// L.key.  Returns the number of vertices that are not live.  FULL: they are
-// listed in queue 0 for g_trim_listed.
+// L.key.  Returns the number of vertices that are not live.
 constexpr uint32_t DEG_CHUNKS = 4;
 
-template <int BS, bool FULL> __device__ __forceinline__ uint32_t g_degrees(Lds &L, const G1 &g, bool trim)
+template <int BS> __device__ __forceinline__ uint32_t g_degrees(Lds &L, const G1 &g, bool trim)
 {
     const uint32_t nch = (g.V + 64) / 64;
     unsigned long long best = 0;
@@ -347,7 +347,6 @@ template <int BS, bool FULL> __device__ __forceinline__ uint32_t g_degrees(Lds &
             gone += in && !alive;
             const uint64_t m = __ballot(alive);
             if (ch < nch && ln() < 2) g.live[2 * ch + ln()] = ln() ? (uint32_t)(m >> 32) : (uint32_t)m;
-            if (FULL) lpush(in && !alive && (fe[h] > fb[h] || be[h] > bb[h]), v, g.queue(0), &L.tail[0]);
             if (alive) {
                 const unsigned long long k = bkey_deg(fe[h] - fb[h], be[h] - bb[h], v);
                 best = k > best ? k : best;
@@ -377,15 +376,15 @@ template <int BS, bool FULL> __device__ __forceinline__ uint32_t g_degrees(Lds &
 // direction, costs more than what it would remove (mix 3.05 -> 2.69 ms).
 constexpr uint32_t TRIM_CHUNKS = 4;
 constexpr uint32_t TRIM_STOP = 32;
-// FULL: queue 0 lists what the last pass removed, for g_trim_listed.
+// LISTED: queue 0 lists what the last pass removed, for g_trim_listed.
 constexpr uint32_t TRIM_MIN = 8;
 
-template <int BS, bool FULL> __device__ __forceinline__ void g_trim_bits(Lds &L, const G1 &g)
+template <int BS, bool LISTED> __device__ __forceinline__ void g_trim_bits(Lds &L, const G1 &g)
 {
     const uint32_t nch = (g.V + 64) / 64;
     uint32_t *F1 = g.f1(), *B1 = g.b1();
     for (uint32_t pass = 0; pass <= g.V; pass++) {   // each pass removes a vertex or ends
-        if (FULL) {
+        if (LISTED) {
             __syncthreads();
             if (threadIdx.x == 0) L.tail[0] = 0;
             __syncthreads();
@@ -473,7 +472,7 @@ template <int BS, bool FULL> __device__ __forceinline__ void g_trim_bits(Lds &L,
                     const uint32_t ch = c0 + h * (BS / 64);
                     const bool out = !x[2 * h] || !x[2 * h + 1];
                     const uint64_t m = __ballot(out);
-                    if (FULL) lpush(out, ch * 64 + ln(), g.queue(0), &L.tail[0]);
+                    if (LISTED) lpush(out, ch * 64 + ln(), g.queue(0), &L.tail[0]);
                     const uint32_t mw = ln() < 32 ? (uint32_t)m : (uint32_t)(m >> 32);
                     if ((ln() & 31) == 0 && mw) g.live[2 * ch + (ln() >> 5)] = word[h] & ~mw;
                     removed += (uint32_t)__popcll(m);
@@ -485,45 +484,67 @@ template <int BS, bool FULL> __device__ __forceinline__ void g_trim_bits(Lds &L,
     __syncthreads();
 }
 
+// no vertex visited (finished ones are told apart by their class)
+template <int BS> __device__ __forceinline__ void g_clear_vis(const G1 &g)
+{
+    const uint32_t nw = 2 * ((g.V + 64) / 64);
+    for (uint32_t i = threadIdx.x; i < nw; i += BS) {
+        g.fvis[i] = 0;
+        g.bvis[i] = 0;
+    }
+}
+
 // A live neighbour w (0: none) that lost an out-arc (d = 1) or in-arc (d = 0)
 // goes too, and is listed in queue 0, unless another live arc that way is
-// left.  All 64 lanes of the wave call.
-__device__ __forceinline__ void g_recheck(Lds &L, const G1 &g, uint32_t d, uint32_t w)
+// left.  The first lane to mark w in `seen` looks: whatever else w lost, it
+// lost before this pass.  (Without the marks every one of a thousand parallel
+// arcs walked the row.)  All 64 lanes of the wave call.
+__device__ __forceinline__ void g_recheck(Lds &L, const G1 &g, uint32_t d, uint32_t w, uint32_t *seen)
 {
     const uint32_t *R = d ? g.Fr : g.Br, *const C[1] = {d ? g.Fc : g.Bc};
-    const uint32_t r = bbit(g.live, w) ? w : 0u;   // row 0 is empty
-    if (!__ballot(r != 0)) return;
+    const uint32_t bit = 1u << (w & 31);
+    const bool look = bbit(g.live, w) && !bbit(seen, w) && !(atomicOr(&seen[w >> 5], bit) & bit);
+    if (!__ballot(look)) return;
+    const uint32_t r = look ? w : 0u;   // row 0 is empty
     uint32_t i[1] = {at(R, r)}, x[1];
     const uint32_t e[1] = {at(R, r + 1)};
     g_any_bit<1>(C, i, e, g.live, x);
-    const uint32_t bit = 1u << (w & 31);
-    const bool gone = r && !x[0] && (atomicAnd(&g.live[w >> 5], ~bit) & bit);
+    const bool gone = look && !x[0] && (atomicAnd(&g.live[w >> 5], ~bit) & bit);
     lpush(gone, w, g.queue(0), &L.tail[0]);
 }
 
+// Every vertex that is not live and has arcs, in queue 0.
+template <int BS> __device__ __forceinline__ void g_list_gone(Lds &L, const G1 &g)
+{
+    __syncthreads();
+    if (threadIdx.x == 0) L.tail[0] = 0;
+    __syncthreads();
+    for (uint32_t v = threadIdx.x; v <= g.V; v += BS)
+        lpush(!bbit(g.live, v) && (at(g.Fr, v + 1) > at(g.Fr, v) || at(g.Br, v + 1) > at(g.Br, v)), v, g.queue(0),
+              &L.tail[0]);
+}
+
 // trim-1 on to its fixpoint, from the removed vertices in queue 0 that no
-// pass has followed up yet.  For the small-graph kernel under Hong's order,
-// whose pivot and counts then are those of trim-1's fixpoint, as the
-// device-wide engine reports them.  The arcs of many vertices are balanced
-// over their wave, as in g_expand; few vertices get several waves each.
-// 16,384 vertices and 139,000 arcs 123 -> 125 us, 999 vertices 50.5 -> 46.7,
-// a path of 16,384 54 -> 10.8 ms (its trims left to g_trim1 before), a star
-// without a cycle 89 -> 97 us.
+// pass has followed up yet.  The arcs of many vertices are balanced over
+// their wave, as in g_expand; few vertices get several waves each.
 template <int BS> __device__ __forceinline__ void g_trim_listed(Lds &L, const G1 &g)
 {
     const uint32_t *q = g.queue(0);
     const uint32_t wv = uni(threadIdx.x >> 6), nwv = BS / 64, d = wv & 1, w = wv >> 1, nw = nwv / 2;
     const uint32_t *R = d ? g.Br : g.Fr, *C = d ? g.Bc : g.Fc;
+    const uint32_t nb = 2 * ((g.V + 64) / 64);
+    uint32_t *seen = g.seen + d * nb;
     __syncthreads();
     for (uint32_t lo = 0, hi = uni(L.tail[0]); lo != hi;) {   // each pass but the last lists a vertex
-        __syncthreads();   // every lane has read the tail
+        for (uint32_t i = threadIdx.x; i < 2 * nb; i += BS) g.seen[i] = 0;
+        __syncthreads();   // and every lane has read the tail
         const uint32_t n = hi - lo;
         if (n < nw) {
             const uint32_t each = nw / n;   // waves per vertex and side
             if (w / each < n) {
                 const uint32_t u = at(q, lo + w / each);
                 for (uint32_t j = at(R, u) + 64 * (w % each), end = at(R, u + 1); j < end; j += 64 * each)
-                    g_recheck(L, g, d, j + ln() < end ? C[j + ln()] : 0u);
+                    g_recheck(L, g, d, j + ln() < end ? C[j + ln()] : 0u, seen);
             }
         } else {
             const uint32_t per = min(64u, (n + nw - 1) / nw);
@@ -544,7 +565,7 @@ template <int BS> __device__ __forceinline__ void g_trim_listed(Lds &L, const G1
                     for (uint32_t o = 32; o >= 1; o >>= 1)
                         own += (uint32_t)__shfl((int)sum, (int)(own + o - 1)) <= j ? o : 0u;
                     const uint32_t st = __shfl(start, (int)own);   // past the end `own` is 63, and the load is skipped
-                    g_recheck(L, g, d, j < total ? C[st + j] : 0u);
+                    g_recheck(L, g, d, j < total ? C[st + j] : 0u, seen);
                 }
             }
         }
@@ -949,16 +970,6 @@ template <int BS> __device__ __forceinline__ void g_trim2(Lds &L, const G1 &g, u
     __syncthreads();
 }
 
-// no vertex visited (finished ones are told apart by their class)
-template <int BS> __device__ __forceinline__ void g_clear_vis(const G1 &g)
-{
-    const uint32_t nw = 2 * ((g.V + 64) / 64);
-    for (uint32_t i = threadIdx.x; i < nw; i += BS) {
-        g.fvis[i] = 0;
-        g.bvis[i] = 0;
-    }
-}
-
 // FW and, with do_bw, BW top-down levels from the seeded queues
 template <int BS> __device__ __forceinline__ void g_reach(Lds &L, const G1 &g, bool do_bw)
 {
@@ -1231,7 +1242,18 @@ template <int BS> __device__ __forceinline__ uint32_t g_canon(Lds &L, const G1 &
 // The whole pipeline of one graph; returns its number of SCCs.  LDS_BITS /
 // LDS_CLS only say which memory the views point to: the code is the same,
 // and inlined per case so that the accesses are LDS instructions.
-template <int BS, uint32_t BUC = BU_CHUNKS, bool FULL = false>
+//
+// Under Hong's order the small-graph kernel reports the pivot and the counts
+// of trim-1's fixpoint, as the device-wide engine does.  FULL 2 trims that
+// far before the first search, and so does FULL 1 where it sweeps anyway.
+// Otherwise FULL 1 searches first: a pivot on a cycle is none that trim-1
+// would have removed, and the list phases then remove and count the same
+// vertices (none of them lies on a path between two that stay, so the search
+// puts those into the same classes).  After an SCC of one vertex it trims, and
+// searches again if the pivot went.  Trimming first where the graph is in LDS
+// takes 999 vertices from 50.5 to 46.5 us; outside it 16,384 vertices and
+// 139,000 arcs take 126 us so and 122 searched first.
+template <int BS, uint32_t BUC = BU_CHUNKS, int FULL = 0>
 __device__ __forceinline__ uint32_t g_solve(Lds &L, const G1 &g, uint32_t cfg)
 {
     const uint32_t nch = (g.V + 64) / 64, nw = 2 * nch;
@@ -1240,67 +1262,86 @@ __device__ __forceinline__ uint32_t g_solve(Lds &L, const G1 &g, uint32_t cfg)
         L.nhub = 0;
         L.nact = 0;
         L.anom = 0;
-        L.tail[0] = 0;
         L.st = GraphStats();
     }
     __syncthreads();
-    const uint32_t ndeg = g_degrees<BS, FULL>(L, g, cfg_t1(cfg));
+    const uint32_t ndeg = g_degrees<BS>(L, g, cfg_t1(cfg));
     // (never with the trims off; FULL: colouring trims once, as in the device-wide engine)
     const bool first = (uint64_t)ndeg * TRIM_MIN > g.V && !(FULL && cfg_slota(cfg));
-    if (first) g_trim_bits<BS, FULL>(L, g);
-    if (FULL && cfg_t1(cfg) && !cfg_slota(cfg)) g_trim_listed<BS>(L, g);
-    uint32_t nl = 0;
-    for (uint32_t i = threadIdx.x; i < nw; i += BS) {
-        nl += (uint32_t)__popc(g.live[i]);
-        g.fvis[i] = 0;
-        g.bvis[i] = 0;
+    if (first) g_trim_bits<BS, FULL != 0>(L, g);
+    const bool full = FULL && cfg_t1(cfg) && !cfg_slota(cfg);
+    bool trim = full && (FULL == 2 || first);
+    if (trim) {
+        if (!first) g_list_gone<BS>(L, g);   // else queue 0 holds what the last sweep removed
+        g_trim_listed<BS>(L, g);
     }
-    const uint32_t nlive = wg_sum1<BS>(L, nl);
-    // the best key of the degree pass may name a vertex the trim removed
-    if (nlive && !bbit(g.live, bkey_vertex(L.key))) {
-        __syncthreads();
-        if (threadIdx.x == 0) L.key = 0;
-        __syncthreads();
-        unsigned long long best = 0;
-        for (uint32_t v = threadIdx.x; v <= g.V; v += BS)
-            if (bbit(g.live, v)) {
-                const unsigned long long k = bkey(g.Fr, g.Br, v);
-                best = k > best ? k : best;
+    uint32_t nlive, p0, nmem, root;
+    for (;;) {
+        uint32_t nl = 0;
+        for (uint32_t i = threadIdx.x; i < nw; i += BS) {
+            nl += (uint32_t)__popc(g.live[i]);
+            g.fvis[i] = 0;
+            g.bvis[i] = 0;
+        }
+        nlive = wg_sum1<BS>(L, nl);
+        // the best key of the degree pass may name a vertex the trim removed
+        if (nlive && !bbit(g.live, bkey_vertex(L.key))) {
+            __syncthreads();
+            if (threadIdx.x == 0) L.key = 0;
+            __syncthreads();
+            unsigned long long best = 0;
+            for (uint32_t v = threadIdx.x; v <= g.V; v += BS)
+                if (bbit(g.live, v)) {
+                    const unsigned long long k = bkey(g.Fr, g.Br, v);
+                    best = k > best ? k : best;
+                }
+            for (int o = 32; o > 0; o >>= 1) {
+                const unsigned long long x = __shfl_xor(best, o);
+                best = x > best ? x : best;
             }
-        for (int o = 32; o > 0; o >>= 1) {
-            const unsigned long long x = __shfl_xor(best, o);
-            best = x > best ? x : best;
+            if (ln() == 0 && best) atomicMax(&L.key, best);
+            __syncthreads();
         }
-        if (ln() == 0 && best) atomicMax(&L.key, best);
-        __syncthreads();
-    }
-    const uint32_t p0 = nlive ? uni(bkey_vertex(L.key)) : 0u;
-    if (nlive) {
-        if (threadIdx.x == 0) {
-            g.fvis[p0 >> 5] |= 1u << (p0 & 31);
-            g.bvis[p0 >> 5] |= 1u << (p0 & 31);
-            g.queue(0)[0] = p0;
-            g.queue(2)[0] = p0;
-            L.tail[0] = 1;
-            L.tail[1] = 1;
+        p0 = nlive ? uni(bkey_vertex(L.key)) : 0u;
+        if (nlive) {
+            if (threadIdx.x == 0) {
+                g.fvis[p0 >> 5] |= 1u << (p0 & 31);
+                g.bvis[p0 >> 5] |= 1u << (p0 & 31);
+                g.queue(0)[0] = p0;
+                g.queue(2)[0] = p0;
+                L.tail[0] = 1;
+                L.tail[1] = 1;
+            }
+            __syncthreads();
+            const uint64_t t0 = wall_clock64();
+            g_first_search<BS, BUC>(L, g, nlive, first, g.E >= BU_DEGREE * (uint64_t)g.V);
+            if (threadIdx.x == 0) {
+                L.st.search_ticks = wall_clock64() - t0;
+                L.st.first_pivot = p0;
+                L.st.pivots = 1;
+            }
         }
-        __syncthreads();
-        const uint64_t t0 = wall_clock64();
-        g_first_search<BS, BUC>(L, g, nlive, first, g.E >= BU_DEGREE * (uint64_t)g.V);
-        if (threadIdx.x == 0) {
-            L.st.search_ticks = wall_clock64() - t0;
-            L.st.first_pivot = p0;
-            L.st.pivots = 1;
+        // the pivot's SCC: its size, its smallest vertex
+        uint32_t members = 0, least = DEAD;
+        for (uint32_t i = threadIdx.x; i < nw; i += BS) {
+            const uint32_t m = g.live[i] & g.fvis[i] & g.bvis[i];
+            members += (uint32_t)__popc(m);
+            if (m && least == DEAD) least = 32 * i + (uint32_t)(__ffs(m) - 1);
         }
+        nmem = wg_sum1<BS>(L, members);
+        root = wg_min1<BS>(L, least);
+        if (!full || trim || nmem != 1) break;
+        g_list_gone<BS>(L, g);
+        g_trim_listed<BS>(L, g);
+        trim = true;
+        if (bbit(g.live, p0)) {   // what the trim removed had no part in the search
+            nl = 0;
+            for (uint32_t i = threadIdx.x; i < nw; i += BS) nl += (uint32_t)__popc(g.live[i]);
+            nlive = wg_sum1<BS>(L, nl);
+            break;
+        }
+        if (threadIdx.x == 0) L.st = GraphStats();
     }
-    // the pivot's SCC: its size, its smallest vertex
-    uint32_t members = 0, least = DEAD;
-    for (uint32_t i = threadIdx.x; i < nw; i += BS) {
-        const uint32_t m = g.live[i] & g.fvis[i] & g.bvis[i];
-        members += (uint32_t)__popc(m);
-        if (m && least == DEAD) least = 32 * i + (uint32_t)(__ffs(m) - 1);
-    }
-    const uint32_t nmem = wg_sum1<BS>(L, members), root = wg_min1<BS>(L, least);
     const uint32_t singles = g.V - nlive;   // trim-1's
     if (threadIdx.x == 0) L.st.trim1 = singles;
     if (nmem == nlive) {
@@ -1453,14 +1494,15 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) void ba
 // trims off, a star without a cycle (207 against 186): one CU does all its
 // scattered key accesses.  What is left after the first round is listed in
 // LDS beside the class words (16,384 vertices in 5,466 SCCs 358 -> 344).
-constexpr uint32_t SMALL_LDS = 36864;   // words: class words and list, or everything of a graph that fits
+constexpr uint32_t SMALL_LDS = 36864;   // words: class words, list and marks, or all of a graph that fits
 
 __global__ __launch_bounds__(1024) void small_scc_kernel(SmallArgs a)
 {
     __shared__ Lds L;
-    __shared__ uint32_t s_bits[3][2 * ((SMALL_V + 64) / 64)];
+    constexpr uint32_t words = 2 * ((SMALL_V + 64) / 64);
+    __shared__ uint32_t s_bits[3 * words];
     __shared__ uint32_t s_mem[SMALL_LDS];
-    static_assert(2 * SMALL_V + 3 <= SMALL_LDS, "the class words and the list of vertices left fit");
+    static_assert(2 * SMALL_V + 3 + 2 * words <= SMALL_LDS, "class words, list of vertices left and marks fit");
     const uint64_t t0 = wall_clock64();
     G1 g;
     g.V = a.V;
@@ -1468,9 +1510,9 @@ __global__ __launch_bounds__(1024) void small_scc_kernel(SmallArgs a)
     g.lab = a.lab;
     g.piv = a.piv;
     g.pivlist = a.pivlist;
-    g.live = s_bits[0];
-    g.fvis = s_bits[1];
-    g.bvis = s_bits[2];
+    g.live = s_bits;
+    g.fvis = s_bits + words;
+    g.bvis = s_bits + 2 * words;
     g.cls = s_mem;
     uint32_t n;
     const uint64_t nr = (uint64_t)a.V + 2;
@@ -1479,6 +1521,7 @@ __global__ __launch_bounds__(1024) void small_scc_kernel(SmallArgs a)
         g.aux = Bc + a.E;
         g.q = g.aux + nr;   // 4 * nr words
         g.list = g.queue(1);
+        g.seen = s_bits + words;   // the visited bitmaps, free until the search
         for (uint32_t i = threadIdx.x; i < nr; i += 1024) {
             Fr[i] = a.Fr[i];
             Br[i] = a.Br[i];
@@ -1492,7 +1535,7 @@ __global__ __launch_bounds__(1024) void small_scc_kernel(SmallArgs a)
         g.Fc = Fc;
         g.Bc = Bc;
         __syncthreads();
-        n = g_solve<1024, 1, true>(L, g, a.cfg);
+        n = g_solve<1024, 1, 2>(L, g, a.cfg);
     } else {
         g.Fr = a.Fr;
         g.Br = a.Br;
@@ -1501,7 +1544,8 @@ __global__ __launch_bounds__(1024) void small_scc_kernel(SmallArgs a)
         g.aux = a.aux;
         g.q = a.q;
         g.list = s_mem + SMALL_V + 1;
-        n = g_solve<1024, 1, true>(L, g, a.cfg);
+        g.seen = s_mem + 2 * SMALL_V + 3;
+        n = g_solve<1024, 1, 1>(L, g, a.cfg);
     }
     __syncthreads();
     if (threadIdx.x != 0) return;
