@@ -749,7 +749,6 @@ scc_status Engine::reach_do(bool fw, bool bw, bool single, uint32_t *levels_out,
             return SCC_OK;
         }
         if (done && seen >= max_levels) {
-            // levels queued ahead still run, on state that nothing reads
             if (levels_out) *levels_out += seen;
             *done = false;
             return SCC_OK;
@@ -802,6 +801,8 @@ scc_status Engine::reach_do(bool fw, bool bw, bool single, uint32_t *levels_out,
             low = rows != nullptr;
         }
         window = spec ? kSpecLevels : kDoWindow;
+        // no level is queued past the bound (level <= max_levels: the first window fits it)
+        if (done) window = (int)std::min<uint32_t>((uint32_t)window, max_levels - level);
         blocks = full;
         if (low) blocks = (uint32_t)std::min<int64_t>(full, std::max<int64_t>(128, (nf_max * 2 + 31) / 32));
         else if (spec) blocks = (uint32_t)std::min<int64_t>(full, std::max<int64_t>(32, (nf_max * 4 + 255) / 256));
@@ -1209,7 +1210,9 @@ scc_status Engine::detect_phases(const scc_opts &o, int expand, int W, scc_stats
 // FW and BW from one pivot over every live vertex (classes ignored; they are
 // all still in class 0), in the live bitmap.  A search that has not ended
 // after kDetectLevels levels is given up: on a high-diameter graph the local
-// SCCs and their quotient graph are the shorter way.
+// SCCs and their quotient graph are the shorter way.  A level is one launch;
+// narrow ones go on for up to 64 hops each, low-degree ones for 128, so a
+// search that is given up has cost at most about 1,300 hops.
 static constexpr uint32_t kDetectLevels = 16;
 
 scc_status Engine::detect_search(scc_stats *stats, bool *found, uint32_t *left)

@@ -1,0 +1,67 @@
+"""detectSCC's search across the partitions: where it is given up, and the
+labels in each case."""
+import re
+
+import numpy as np
+import pytest
+
+import detectingscc_amd as scc
+from oracle import pyoracle as orc
+from helpers import assert_same_labels
+
+pytestmark = pytest.mark.gpu
+
+
+def _grid(side, rng, p=0.8):
+    x = np.arange(side * side).reshape(side, side) + 1
+    s, d = [], []
+    for a, b in ((x[:, :-1], x[:, 1:]), (x[:, 1:], x[:, :-1]), (x[:-1], x[1:]), (x[1:], x[:-1])):
+        keep = rng.random(a.shape) < p
+        s.append(a[keep])
+        d.append(b[keep])
+    return scc.from_arcs(side * side, np.concatenate(s), np.concatenate(d))
+
+
+def _part(V, p):
+    part = np.zeros(V + 2, np.uint32)
+    part[1:V + 1] = p
+    return part
+
+
+def _run(g, parts, **kw):
+    want, n = orc.tarjan(g)
+    with scc.Context(0) as ctx:
+        ctx.upload(g)
+        for part in parts:
+            ctx.upload_partition(_part(g.V, part))
+            for trims in (True, False):
+                for sizes in (False, True):
+                    st = ctx.run(algo="d", trim1=trims, trim2=trims, sizes=sizes)
+                    assert_same_labels(ctx.labels(), want, f"trims {trims} sizes {sizes}")
+                    assert st.num_sccs == n
+
+
+@pytest.mark.parametrize("side", [150, 700])
+def test_high_diameter(side):
+    """Low-degree graphs whose search ends within the bound or is given up."""
+    rng = np.random.default_rng(side)
+    g = _grid(side, rng)
+    _run(g, [np.arange(g.V) * 16 // g.V, rng.integers(0, 16, g.V)])
+
+
+def test_search_keeps_its_bound(monkeypatch, capfd):
+    """On a grid in blocks of rows no level past the sixteenth is run."""
+    g = _grid(1000, np.random.default_rng(1), p=0.7)
+    monkeypatch.setenv("SCC_TRACE_LEVELS", "1")
+    with scc.Context(0) as ctx:
+        ctx.upload(g)
+        ctx.upload_partition(_part(g.V, np.arange(g.V) * 16 // g.V))
+        capfd.readouterr()
+        ctx.run(algo="d", sizes=False)
+    looks = [int(x) for x in re.findall(r"\[scc reach\] after level (\d+):", capfd.readouterr().err)]
+    first = [looks[0]]
+    for x in looks[1:]:
+        if x < first[-1]:
+            break
+        first.append(x)
+    assert first[-1] == 15, first
