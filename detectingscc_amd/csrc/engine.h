@@ -77,7 +77,7 @@ class Engine {
                         bool *done = nullptr);
     scc_status merge_quotient(const uint32_t *tbits, scc_stats *stats, const uint32_t **qid_out,
                               const uint32_t **rep_out, const uint32_t **qlab_out);
-    scc_status detect_search(scc_stats *stats, bool *found, uint32_t *left);
+    scc_status detect_search(uint32_t max_levels, scc_stats *stats, bool *found, uint32_t *left);
     DirArgs dir_args(int d, uint32_t level) const;
     // single: every live vertex has class 0 (the first trim of a
     // decomposition); none_dead: besides, the state is fresh (no vertex dead,

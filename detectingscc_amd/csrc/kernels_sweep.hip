@@ -1163,6 +1163,31 @@ void k_update_words(hipStream_t s, const DevGraph &g, DevState &st, const uint32
                                                             g.V, st.aux);
 }
 
+constexpr uint32_t CROSS_SAMPLE = 1u << 16;
+
+__global__ __launch_bounds__(256) void cross_sample_kernel(const uint32_t *__restrict__ Fr,
+                                                           const uint32_t *__restrict__ Fc,
+                                                           const uint32_t *__restrict__ part, uint32_t *ctr,
+                                                           uint32_t V, uint32_t n)
+{
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    bool arc = false, cross = false;
+    if (i < n) {
+        const uint32_t v = 1 + (uint32_t)((uint64_t)i * V / n), b = Fr[v], deg = Fr[v + 1] - b;
+        arc = deg != 0;
+        if (arc) cross = part[Fc[b + (i * 2654435761u >> 8) % deg]] != part[v];
+    }
+    const uint32_t arcs = (uint32_t)__syncthreads_count(arc), crossing = (uint32_t)__syncthreads_count(cross);
+    if (threadIdx.x == 0 && arcs)
+        atomicAdd(reinterpret_cast<unsigned long long *>(ctr + CT(C_CROSS)), ((unsigned long long)arcs << 32) | crossing);
+}
+
+void k_cross_sample(hipStream_t s, const DevGraph &g, DevState &st)
+{
+    const uint32_t n = std::min(g.V, CROSS_SAMPLE);
+    cross_sample_kernel<<<n / 256 + 1, 256, 0, s>>>(g.Fr, g.Fc, st.part, st.ctr, g.V, n);
+}
+
 // After detectSCC's search over all live vertices: the pivot's SCC (live,
 // visited both ways) is left alone in `live`, its smallest vertex goes to
 // scc_min[pivot], and the other live vertices are counted in C_LIVE.

@@ -34,6 +34,9 @@ void k_q_keys(hipStream_t s, bool emit, const DevGraph &g, const uint32_t *qv, u
 size_t csr_sort_bytes(uint32_t V, uint64_t n);
 scc_status csr_from_keys(hipStream_t st, uint32_t V, uint64_t n, uint64_t *keys, uint64_t *out, void *tmp,
                          size_t tmp_bytes, uint32_t *R, uint32_t *C, uint32_t *RB, uint32_t *CB);
+// Counts in C_CROSS, of up to 2^16 vertices spread over the graph, one arc
+// each: how many arcs there are and how many lead to another partition.
+void k_cross_sample(hipStream_t s, const DevGraph &g, DevState &st);
 // detectSCC's search over every live vertex (engine.hip): after it,
 // k_detect_found leaves the pivot's SCC alone in the live bitmap, its
 // smallest vertex in aux[pivot] and the vertices left in C_LIVE; then

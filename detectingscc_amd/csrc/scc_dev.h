@@ -59,6 +59,7 @@ enum : int {
     C_NSCC = 12,     // canonical roots
     C_LARGEST = 13,  // largest SCC size
     C_FWV = 14,      // first-search statistics: |R| and |E_R| (64-bit pairs)
+    C_CROSS = 15,    // sampled arcs that lead to another partition (word 0) of all sampled (word 1)
     C_FWE = 16,
     C_BWV = 18,
     C_BWE = 20,

@@ -1,5 +1,5 @@
-"""detectSCC's search across the partitions: where it is given up, and the
-labels in each case."""
+"""detectSCC's search across the partitions: when it runs, where it is given
+up, and the labels in each case."""
 import re
 
 import numpy as np
@@ -22,6 +22,18 @@ def _grid(side, rng, p=0.8):
     return scc.from_arcs(side * side, np.concatenate(s), np.concatenate(d))
 
 
+def _communities(k, size, between, rng):
+    """k random graphs of `size` vertices and 6 arcs each, and `between` arcs
+    from each to the next (the last to the first)."""
+    V = k * size
+    s = rng.integers(0, V, 6 * V)
+    d = s // size * size + rng.integers(0, size, s.size)
+    c = np.repeat(np.arange(k), between)
+    s = np.concatenate([s, c * size + rng.integers(0, size, c.size)])
+    d = np.concatenate([d, (c + 1) % k * size + rng.integers(0, size, c.size)])
+    return scc.from_arcs(V, s + 1, d + 1)
+
+
 def _part(V, p):
     part = np.zeros(V + 2, np.uint32)
     part[1:V + 1] = p
@@ -41,9 +53,18 @@ def _run(g, parts, **kw):
                     assert st.num_sccs == n
 
 
+@pytest.mark.parametrize("between", [0, 1, 40, 2000])
+@pytest.mark.parametrize("k,size", [(2, 40), (12, 3000), (60, 1500)])
+def test_communities(k, size, between):
+    """Partitions without, with few and with many arcs between them."""
+    g = _communities(k, size, between, np.random.default_rng(between + k))
+    _run(g, [np.arange(g.V) // size])
+
+
 @pytest.mark.parametrize("side", [150, 700])
 def test_high_diameter(side):
-    """Low-degree graphs whose search ends within the bound or is given up."""
+    """Low-degree graphs whose search ends within the bound, is given up, or
+    is given the longer one."""
     rng = np.random.default_rng(side)
     g = _grid(side, rng)
     _run(g, [np.arange(g.V) * 16 // g.V, rng.integers(0, 16, g.V)])
