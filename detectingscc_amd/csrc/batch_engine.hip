@@ -679,7 +679,9 @@ scc_status scc_batch_upload(scc_ctx *ctx, const scc_batch_host *b)
     clear_error();
     if (!ctx) return fail(SCC_ERR_INVALID, "null context");
     if (!ctx->batch) ctx->batch.reset(new BatchEngine());
-    return ctx->batch->upload(ctx->eng.device, ctx->eng.stream, b);
+    scc_status s = ctx->batch->upload(ctx->eng.device, ctx->eng.stream, b);
+    if (s == SCC_ERR_NOMEM && ctx->eng.give_back()) s = ctx->batch->upload(ctx->eng.device, ctx->eng.stream, b);
+    return s;
 }
 
 scc_status scc_batch_run(scc_ctx *ctx, const scc_batch_opts *opts, scc_batch_stats *stats)
@@ -703,7 +705,9 @@ scc_status scc_batch_run_serial(scc_ctx *ctx, const scc_opts *opts, scc_batch_st
         scc_status s = ctx->serial->init(ctx->eng.device);
         if (s != SCC_OK) return s;
     }
-    return ctx->batch->run_serial(*ctx->serial, o, stats);
+    scc_status s = ctx->batch->run_serial(*ctx->serial, o, stats);
+    if (s == SCC_ERR_NOMEM && ctx->eng.give_back()) s = ctx->batch->run_serial(*ctx->serial, o, stats);
+    return s;
 }
 
 scc_status scc_batch_autotune(scc_ctx *ctx, int sample, char *report, size_t report_len)

@@ -19,6 +19,10 @@ class Engine {
   public:
     ~Engine();
     scc_status init(int device);
+    // Frees what the engine can do without (the second set of graph arrays,
+    // the low-degree rows) for an allocation that has failed; false if there
+    // was nothing.  Not during a search.
+    bool give_back();
     // `checked`: the caller has already validated the arrays (the server's
     // submit does), so they are not checked again
     scc_status upload(uint32_t V, uint32_t E, const uint32_t *Fr, const uint32_t *Fc,
@@ -59,6 +63,8 @@ class Engine {
     bool fits(uint32_t V, uint32_t E) const;
     bool spare_set();
     void drop_spare();
+    uint64_t extra_bytes() const;
+    uint64_t extra_limit = UINT64_MAX;   // most bytes of scratch and optional arrays (SCC_SCRATCH_LIMIT)
     DevGraph spare;                    // a second set of Fr, Fc, Br, Bc (lazily made, see upload)
     scc_status read_ctr();                 // publish_ctr + wait_ctr
     uint32_t publish_ctr();                // queue a publication of the counters, returns its number

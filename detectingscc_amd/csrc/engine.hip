@@ -123,6 +123,10 @@ scc_status Engine::init(int dev)
     // diagnostic: SCC_TRACE_LEVELS=1 prints every host decision of a search
     const char *tr = std::getenv("SCC_TRACE_LEVELS");
     trace_levels = tr && tr[0] == '1';
+    // a bound on the scratch and optional arrays, past which the engine acts
+    // as where the device has no more memory
+    const char *limit = std::getenv("SCC_SCRATCH_LIMIT");
+    if (limit && limit[0]) extra_limit = std::strtoull(limit, nullptr, 10);
     return SCC_OK;
 }
 
@@ -160,7 +164,7 @@ scc_status Engine::reserve(uint32_t V, uint32_t E)
         f(st.bigf[i]); f(st.bigb[i]); f(st.bigoff_f[i]); f(st.bigoff_b[i]);
     }
     f(st.pivlist); f(st.stamp); f(st.part); f(st.bred); f(d_tmp8);
-    drop_spare();
+    (void)give_back();
     uint32_t *ctr = st.ctr;
     g = DevGraph();
     st = DevState();
@@ -242,7 +246,8 @@ bool Engine::spare_set()
 {
     if (spare.Fr) return true;
     const size_t rows = (size_t)capV + 2;
-    if (8 * ((uint64_t)rows + capE) > kSpareMax) return false;
+    const uint64_t bytes = 8 * ((uint64_t)rows + capE);
+    if (bytes > kSpareMax || extra_bytes() + bytes > extra_limit) return false;
     hipError_t e[4] = {dalloc(&spare.Fr, rows), dalloc(&spare.Br, rows), dalloc(&spare.Fc, capE),
                        dalloc(&spare.Bc, capE)};
     for (hipError_t r : e)
@@ -251,6 +256,24 @@ bool Engine::spare_set()
             drop_spare();
             return false;
         }
+    return true;
+}
+
+uint64_t Engine::extra_bytes() const
+{
+    uint64_t n = low_buf.cap + (spare.Fr ? 8 * ((uint64_t)capV + 2 + capE) : 0);
+    for (const auto &b : buf) n += b.cap;
+    return n;
+}
+
+bool Engine::give_back()
+{
+    if (!spare.Fr && !low_buf.p) return false;
+    (void)hipSetDevice(device);
+    (void)hipStreamSynchronize(stream);
+    drop_spare();
+    if (low_buf.p) (void)hipFree(low_buf.p);
+    low_buf = DevBuf();
     return true;
 }
 
@@ -398,9 +421,11 @@ template <class T> scc_status Engine::scratch(DevBuf &b, size_t n, T **out)
         if (b.p) (void)hipFree(b.p);
         b.p = nullptr;
         b.cap = 0;
-        hipError_t e = hipMalloc(&b.p, bytes);
-        if (e != hipSuccess) {
+        auto get = [&] { return extra_bytes() + bytes > extra_limit ? hipErrorOutOfMemory : hipMalloc(&b.p, bytes); };
+        // an allocation that fails is tried again without the optional arrays
+        if (get() != hipSuccess && (!give_back() || get() != hipSuccess)) {
             (void)hipGetLastError();
+            b.p = nullptr;
             return fail(SCC_ERR_NOMEM, "Error: Not enough memory on GPU (%zu scratch bytes)", bytes);
         }
         b.cap = bytes;
@@ -1317,7 +1342,9 @@ scc_status Engine::merge_quotient(const uint32_t *tbits, scc_stats *stats, const
                 sub.reset(new Engine());
                 if ((s = sub->init(device)) != SCC_OK) return s;
             }
-            if ((s = sub->upload_device(QV, QE, Qr, Qc, QBr, QBc, stream)) != SCC_OK) return s;
+            s = sub->upload_device(QV, QE, Qr, Qc, QBr, QBc, stream);
+            if (s == SCC_ERR_NOMEM && give_back()) s = sub->upload_device(QV, QE, Qr, Qc, QBr, QBc, stream);
+            if (s != SCC_OK) return s;
             scc_opts so;
             scc_opts_default(&so);
             so.algo = 'g';

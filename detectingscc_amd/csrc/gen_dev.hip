@@ -494,6 +494,7 @@ scc_status scc_gen_er_dev(scc_ctx *ctx, uint32_t V, uint64_t draws, uint32_t cyc
                           uint64_t seed)
 {
     CTX_DEV(ctx);
+    (void)ctx->eng.give_back();   // the memory may be short
     if (V < 1 || V >= (1u << 30)) return fail(SCC_ERR_INVALID, "bad ER arguments");
     Engine &e = ctx->eng;
     hipStream_t st = e.stream;
@@ -542,6 +543,7 @@ scc_status scc_gen_er_dev(scc_ctx *ctx, uint32_t V, uint64_t draws, uint32_t cyc
 scc_status scc_gen_rmat_dev(scc_ctx *ctx, uint32_t scale, uint64_t E, double a, double b, double c, uint64_t seed)
 {
     CTX_DEV(ctx);
+    (void)ctx->eng.give_back();   // the memory may be short
     if (scale < 1 || scale > 29 || a < 0 || b < 0 || c < 0 || a + b + c > 1.0)
         return fail(SCC_ERR_INVALID, "bad R-MAT arguments");
     const uint32_t V = 1u << scale;
@@ -563,6 +565,7 @@ scc_status scc_gen_rmat_dev(scc_ctx *ctx, uint32_t scale, uint64_t E, double a, 
 scc_status scc_gen_grid_dev(scc_ctx *ctx, uint32_t side, double p, uint64_t seed)
 {
     CTX_DEV(ctx);
+    (void)ctx->eng.give_back();   // the memory may be short
     if (side < 1 || (uint64_t)side * side >= (1u << 30) || p < 0 || p > 1)
         return fail(SCC_ERR_INVALID, "bad grid arguments");
     const uint64_t V = (uint64_t)side * side;
@@ -579,6 +582,7 @@ scc_status scc_gen_communities_dev(scc_ctx *ctx, uint32_t V, uint32_t K, double 
                                    uint32_t *part)
 {
     CTX_DEV(ctx);
+    (void)ctx->eng.give_back();   // the memory may be short
     if (V < 1 || K < 1 || K > V || V >= (1u << 30) || deg < 0 || inter < 0 || inter > 1)
         return fail(SCC_ERR_INVALID, "bad community arguments");
     const uint64_t E = (uint64_t)std::llround(deg * V);
@@ -607,6 +611,7 @@ scc_status scc_gen_batch_mix_dev(scc_ctx *ctx, uint32_t num_graphs, uint32_t lgm
                                  double dmax, uint64_t seed, scc_batch_host *copy)
 {
     CTX_DEV(ctx);
+    (void)ctx->eng.give_back();   // the memory may be short
     if (!num_graphs || lgmin < 1 || lgmax < lgmin || lgmax > 24 || dmin < 0 || dmax < dmin)
         return fail(SCC_ERR_INVALID, "bad batch-mix arguments");
     const uint32_t G = num_graphs;

@@ -390,6 +390,7 @@ scc_status scc_server_start(scc_ctx *ctx, uint64_t hbm_budget, uint32_t max_batc
     clear_error();
     if (!ctx || !opts) return fail(SCC_ERR_INVALID, "null argument");
     if (!ctx->server) ctx->server.reset(new Server(ctx->eng.device));
+    (void)ctx->eng.give_back();   // the slots' memory may be short
     return ctx->server->start(hbm_budget, max_batch, slots, solo_vertices, *opts);
 }
 
