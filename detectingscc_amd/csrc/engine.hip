@@ -170,6 +170,7 @@ scc_status Engine::reserve(uint32_t V, uint32_t E)
     st = DevState();
     st.ctr = ctr;
     capV = capE = 0;
+    has_graph = has_part = ran = false;   // the caller sets them again, unless the allocation fails
     const size_t nv = (size_t)nV + 1;
     const size_t nwords = 2 * ((nv + 63) / 64);
     hipError_t e = hipSuccess;
