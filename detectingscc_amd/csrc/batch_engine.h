@@ -35,6 +35,10 @@ class BatchEngine {
     void release();
     scc_status prepare(int device, hipStream_t stream, uint32_t ng, const uint32_t *Vs, const uint32_t *Es,
                        const uint64_t *roff, const uint64_t *coff);
+    scc_status upload_host(int device, hipStream_t stream, const scc_batch_host *b, bool checked);
+    scc_status install_device(int device, hipStream_t stream, uint32_t ng, const uint32_t *Vs, const uint32_t *Es,
+                              const uint64_t *roff, const uint64_t *coff, const uint64_t *d_roff,
+                              const uint32_t *dFr, const uint32_t *dBr, const uint32_t *dFc, const uint32_t *dBc);
     scc_status finish_upload(bool check);
     scc_status launch(const std::vector<uint32_t> &idx, const std::vector<uint32_t> &cfg,
                       const std::vector<int> &block, double *ms, std::vector<double> *lat_ms,

@@ -170,7 +170,7 @@ __global__ __launch_bounds__(256) void batch_check_kernel(const uint64_t *__rest
 }
 
 // Metadata to the device, the upload check, and the per-graph tables of the
-// launches.  A batch that is refused leaves none.
+// launches.
 scc_status BatchEngine::finish_upload(bool check)
 {
     BHIP(hipMemcpyAsync(m_voff, voff.data(), sizeof(uint64_t) * (G + 1), hipMemcpyHostToDevice, s1));
@@ -186,10 +186,7 @@ scc_status BatchEngine::finish_upload(bool check)
         BHIP(hipMemcpyAsync(h_meta, m_meta, sizeof(uint32_t), hipMemcpyDeviceToHost, s1));
     }
     BHIP(hipStreamSynchronize(s1));
-    if (check && h_meta[0]) {
-        G = 0;
-        return fail(SCC_ERR_INVALID, "a batch graph has an invalid CSR");
-    }
+    if (check && h_meta[0]) return fail(SCC_ERR_INVALID, "a batch graph has an invalid CSR");
     d.G = G;
     d.voff = m_voff;
     d.eoff = m_eoff;
@@ -218,6 +215,8 @@ scc_status BatchEngine::finish_upload(bool check)
     return SCC_OK;
 }
 
+// An upload that fails once the sizes are taken over leaves no batch: the
+// buffers and tables are those of the batch before, or none.
 scc_status BatchEngine::upload(int device, hipStream_t stream, const scc_batch_host *b, bool checked)
 {
     if (!b || !b->num_graphs || !b->V || !b->E || !b->row_off || !b->col_off || !b->Fr || !b->Br ||
@@ -230,6 +229,13 @@ scc_status BatchEngine::upload(int device, hipStream_t stream, const scc_batch_h
         if (Fr[0] || Fr[1] || Br[0] || Br[1] || Fr[b->V[i] + 1] != b->E[i] || Br[b->V[i] + 1] != b->E[i])
             return fail(SCC_ERR_INVALID, "graph %u: row arrays are not in the reference layout", i);
     }
+    scc_status s = upload_host(device, stream, b, checked);
+    if (s != SCC_OK) G = 0;
+    return s;
+}
+
+scc_status BatchEngine::upload_host(int device, hipStream_t stream, const scc_batch_host *b, bool checked)
+{
     scc_status st = prepare(device, stream, b->num_graphs, b->V, b->E, b->row_off, b->col_off);
     if (st != SCC_OK) return st;
     const uint64_t S = voff[G], A = eoff[G];
@@ -281,6 +287,16 @@ scc_status BatchEngine::upload_device(int device, hipStream_t stream, uint32_t n
                                       const uint32_t *Es, const uint64_t *roff, const uint64_t *coff,
                                       const uint64_t *d_roff, const uint32_t *dFr, const uint32_t *dBr,
                                       const uint32_t *dFc, const uint32_t *dBc)
+{
+    scc_status s = install_device(device, stream, ng, Vs, Es, roff, coff, d_roff, dFr, dBr, dFc, dBc);
+    if (s != SCC_OK) G = 0;
+    return s;
+}
+
+scc_status BatchEngine::install_device(int device, hipStream_t stream, uint32_t ng, const uint32_t *Vs,
+                                       const uint32_t *Es, const uint64_t *roff, const uint64_t *coff,
+                                       const uint64_t *d_roff, const uint32_t *dFr, const uint32_t *dBr,
+                                       const uint32_t *dFc, const uint32_t *dBc)
 {
     scc_status st = prepare(device, stream, ng, Vs, Es, roff, coff);
     if (st != SCC_OK) return st;

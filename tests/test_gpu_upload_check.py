@@ -77,3 +77,25 @@ def test_batch_faults_are_refused(graphs, vmax, degree):
         for k, i in enumerate(range(0, graphs, max(1, graphs // 50))):
             assert counts[i] == wants[k][1]
             assert_same_labels(labels[i], wants[k][0], f"graph {i}")
+
+
+def test_batch_of_wrong_offsets_is_none():
+    """A larger batch whose offsets are refused does not run in the buffers of
+    the batch before."""
+    rng = np.random.default_rng(8)
+    good = scc.batch_from_graphs([random_graph(9, 20, rng) for _ in range(3)])
+    more = scc.batch_from_graphs([random_graph(50, 200, rng) for _ in range(500)])
+    col = more.col_off.copy()
+    col[-1] += 1
+    wrong = scc.Batch(more.V, more.E, more.row_off, col, more.Fr, more.Fc, more.Br, more.Bc)
+    with scc.Context(0) as ctx:
+        ctx.batch_upload(good)
+        ctx.batch_run()
+        with pytest.raises(scc.SCCError, match="offsets do not match"):
+            ctx.batch_upload(wrong)
+        for call in (ctx.batch_run, ctx.batch_run_serial, ctx.batch_autotune):
+            with pytest.raises(scc.SCCError, match="no batch uploaded"):
+                call()
+        ctx.batch_upload(more)
+        ctx.batch_run()
+        assert_same_labels(ctx.batch_labels()[0][499], orc.tarjan(more.graph(499))[0])
