@@ -36,7 +36,8 @@ class Server {
     struct Req {
         uint64_t id = 0;
         uint32_t V = 0, E = 0;
-        std::vector<uint32_t> Fr, Fc, Br, Bc, lab;
+        std::vector<uint32_t> Fr, Fc, Br, Bc;
+        std::unique_ptr<uint32_t[]> lab;   // V + 1 labels, made when a slot takes the request
         uint64_t bytes = 0;
         clock::time_point arrival, done_at;
         uint32_t nscc = 0;

@@ -214,8 +214,8 @@ void Server::worker(int slot)
         // request's before it is done)
         lab.resize(G);
         for (uint32_t i = 0; i < G; i++) {
-            batch[i]->lab.resize((size_t)batch[i]->V + 1);
-            lab[i] = batch[i]->lab.data();
+            batch[i]->lab.reset(new uint32_t[(size_t)batch[i]->V + 1]);   // not cleared: every word is written
+            lab[i] = batch[i]->lab.get();
         }
         nscc.resize(G);
         scc_status st = init_err.empty() ? SCC_OK : fail(SCC_ERR_DEVICE, "%s", init_err.c_str());
@@ -314,7 +314,7 @@ scc_status Server::poll(uint64_t id, uint32_t *lab, uint32_t *nscc, double *late
     if (!r->done) return fail(SCC_ERR_NOTREADY, "request %llu not done", (unsigned long long)id);
     scc_status st = r->status;
     if (st == SCC_OK) {
-        if (lab) std::memcpy(lab, r->lab.data(), sizeof(uint32_t) * r->lab.size());
+        if (lab) std::memcpy(lab, r->lab.get(), sizeof(uint32_t) * ((size_t)r->V + 1));
         if (nscc) *nscc = r->nscc;
         if (latency_ms) *latency_ms = std::chrono::duration<double, std::milli>(r->done_at - r->arrival).count();
     } else {
