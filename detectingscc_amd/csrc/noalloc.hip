@@ -121,8 +121,6 @@ extern "C" scc_status scc_histogram_noalloc(scc_ctx *ctx, uint64_t *pairs, uint3
     if (!d) return fail(SCC_ERR_NOTREADY, "scratch address of device %d not set up", E.device);
     HIP_TRY(hipSetDevice(E.device));
     uint32_t *dn = reinterpret_cast<uint32_t *>(d + 2 * (size_t)kNoAllocPairs);
-    k_fill_u32(E.stream, dn, 0u, 1);   // a fill kernel, not a memset node
-    k_sizes(E.stream, E.g, E.st);
     k_size_histogram(E.stream, E.g, E.st, E.st.aux, d, kNoAllocPairs, dn);
     pairs_sort_kernel<<<1, kSortThreads, 0, E.stream>>>(d, dn, kNoAllocPairs);
     uint32_t n = 0;
