@@ -429,6 +429,8 @@ def _batch_stats(s: _BatchStats) -> BatchStats:
 
 def make_batch_opts(algo: str = "g", trim1: bool = True, trim2: bool = True, lanes: int = 4,
                     block: int = 256, autotuned: bool = False) -> _BatchOpts:
+    """Options of scc_batch_run and the server; `lanes` (a power of two up to
+    64) is checked and otherwise unused."""
     o = _BatchOpts()
     o.algo = algo.encode()[:1]
     o.trim1, o.trim2, o.lanes, o.block, o.autotuned = int(trim1), int(trim2), int(lanes), int(block), int(autotuned)

@@ -1456,11 +1456,10 @@ scc_status Engine::labels(uint32_t *lab)
     return SCC_OK;
 }
 
-// The size histogram of the last run, on the device: sizes from the
-// canonical labels (k_sizes), then the per-size counts and their non-zero
-// entries (at most floor(sqrt(2V)) + 1 distinct sizes: the sizes of
-// distinct SCCs sum to at most V).  *ms is the device time of the three
-// passes plus the compaction.
+// The size histogram of the last run, on the device (k_size_histogram): sizes
+// from the canonical labels, then the per-size counts and their non-zero
+// entries (at most floor(sqrt(2V)) + 1 distinct sizes: the sizes of distinct
+// SCCs sum to at most V).  *ms is the device time of its four passes.
 scc_status Engine::histogram(uint64_t *pairs, uint32_t cap, uint32_t *npairs, double *ms)
 {
     if (!ran) return fail(SCC_ERR_NOTREADY, "no completed run");

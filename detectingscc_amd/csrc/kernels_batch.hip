@@ -25,8 +25,8 @@
 // balanced over its wave, hubs over the workgroup, bottom-up levels where
 // the degree pays for them, no gather of first neighbours where trim-1 would
 // remove little, and nothing run for vertices that are finished.  The mix
-// (47.6M vertices, 434M arcs, 1,024 lanes) 11.1 -> 1.9 ms; 700 graphs of 2^8
-// to 2^12 vertices with 256 lanes 1.31 -> 0.19 ms.
+// (47.6M vertices, 434M arcs, 1,024 lanes) 11.1 -> 1.8 ms; 700 graphs of 2^8
+// to 2^12 vertices with 256 lanes 1.31 -> 0.17 ms.
 //
 // Layout: graph i's per-vertex arrays start at slot voff[i] (a multiple of
 // 64, so bitmap words never straddle two graphs) and span V_i+2 slots; its
@@ -1239,9 +1239,8 @@ template <int BS> __device__ __forceinline__ uint32_t g_canon(Lds &L, const G1 &
     return wg_sum1<BS>(L, roots);
 }
 
-// The whole pipeline of one graph; returns its number of SCCs.  LDS_BITS /
-// LDS_CLS only say which memory the views point to: the code is the same,
-// and inlined per case so that the accesses are LDS instructions.
+// The whole pipeline of one graph; returns its number of SCCs.  Inlined once
+// per place the views may be in, so that accesses to LDS are LDS instructions.
 //
 // Under Hong's order the small-graph kernel reports the pivot and the counts
 // of trim-1's fixpoint, as the device-wide engine does.  FULL 2 trims that
@@ -1475,7 +1474,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) void ba
 // ------------------------------------------------ one small graph ---
 // A resident graph of at most SMALL_V vertices and SMALL_E arcs as one
 // launch of one workgroup, instead of the device-wide engine's chain of
-// about 17 launches and two looks at the counters (100 to 150 us on graphs
+// about 19 launches and two looks at the counters (100 to 150 us on graphs
 // of this size, 300 and more where the first round leaves vertices).  Where
 // the whole CSR and the work arrays fit LDS they are copied there first, so
 // a level's dependent loads are LDS reads.  The counters the host waits for

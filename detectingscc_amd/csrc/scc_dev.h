@@ -443,6 +443,8 @@ void k_do_level(hipStream_t s, const DoArgs &a, bool single_class, uint32_t bloc
 // leaving that level's input rewritten; a no-op unless that level would run
 // top-down from a small frontier with no hubs pending.  narrow_cap(): the
 // largest frontier the host starts it on
+void k_narrow_levels(hipStream_t s, const DoArgs &a, bool single_class);
+uint32_t narrow_cap();
 // Sets *bad (host memory) unless R and C are a reference-layout CSR of V
 // vertices and E arcs: R starts 0,0, does not decrease and ends at E, C
 // holds ids 1..V.  Reads nothing outside the two arrays whatever they hold.
@@ -452,8 +454,6 @@ void k_check_csr(hipStream_t s, const uint32_t *R, const uint32_t *C, uint32_t V
 void k_low_rows(hipStream_t s, const DevGraph &g, uint4 *AF, uint4 *AB);
 // A top-down level of a single-class search on a low-degree graph.
 void k_low_level(hipStream_t s, const DoArgs &a, uint32_t blocks_per_dir);
-void k_narrow_levels(hipStream_t s, const DoArgs &a, bool single_class);
-uint32_t narrow_cap();
 uint32_t do_blocks(uint32_t V, int ndirs);
 // Words of a search queue: bottom-up levels write kSpread slot regions.
 size_t queue_words(uint32_t V);

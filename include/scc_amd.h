@@ -167,7 +167,9 @@ typedef struct {
     uint32_t num_sccs;       /* "Number Of Sccs" (scc_WCC.cu:966) */
     uint32_t num_trim1;      /* "numberOf1Sccs" (scc_WCC.cu:948) */
     uint32_t num_trim2;      /* 2-SCCs removed by trim-2 */
-    uint32_t num_pivot;      /* SCCs found by a pivot / colour-root search */
+    uint32_t num_pivot;      /* SCCs found by a pivot / colour-root search.  SCC_ALGO_DETECT:
+                                if its search across the partitions found an SCC, that one
+                                counts here, and trims and local SCCs are those of the rest */
     uint32_t largest;        /* size of the largest SCC (0 unless opts.sizes) */
     uint32_t rounds;         /* outer rounds of the main loop */
     uint32_t levels;         /* BFS levels launched, both directions */
@@ -176,7 +178,8 @@ typedef struct {
     uint64_t first_bw_vertices, first_bw_arcs; /* |R|, |E_R| of the first BW (opts.sizes) */
     double ms_scc;           /* CSR resident -> labels resident (device clock) */
     double ms_first_reach;   /* first-pivot FW||BW (device clock) */
-    double ms_phase[SCC_PHASE_COUNT];   /* with opts.phase_times, else 0 */
+    double ms_phase[SCC_PHASE_COUNT];   /* with opts.phase_times, else 0; the search across
+                                           the partitions counts as SCC_PHASE_MERGE */
     /* Work units of the first search when it is direction-optimised and
      * opts.sizes is set (else 0), both directions: [0] vertices expanded
      * top-down, [1] arcs scanned top-down, [2] vertices claimed, [3]
