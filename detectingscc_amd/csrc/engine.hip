@@ -422,9 +422,15 @@ template <class T> scc_status Engine::scratch(DevBuf &b, size_t n, T **out)
         if (b.p) (void)hipFree(b.p);
         b.p = nullptr;
         b.cap = 0;
-        auto get = [&] { return extra_bytes() + bytes > extra_limit ? hipErrorOutOfMemory : hipMalloc(&b.p, bytes); };
+        // past the bound it asks for more than any device has, which the runtime refuses
+        auto get = [&] { return hipMalloc(&b.p, extra_bytes() + bytes > extra_limit ? SIZE_MAX / 4 : bytes); };
         // an allocation that fails is tried again without the optional arrays
-        if (get() != hipSuccess && (!give_back() || get() != hipSuccess)) {
+        hipError_t e = get();
+        if (e != hipSuccess) {
+            (void)hipGetLastError();   // not to be taken for a launch's
+            if (give_back()) e = get();
+        }
+        if (e != hipSuccess) {
             (void)hipGetLastError();
             b.p = nullptr;
             return fail(SCC_ERR_NOMEM, "Error: Not enough memory on GPU (%zu scratch bytes)", bytes);
