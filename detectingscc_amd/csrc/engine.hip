@@ -454,12 +454,15 @@ __global__ void publish_ctr_kernel(const uint32_t *ctr, uint32_t *pub, uint32_t 
     const uint32_t i = threadIdx.x;
     if (i < C_COUNT) {
         for (int w = 0; w < kPubWords; w++) pub[CT(i) + w] = ctr[CT(i) + w];
-        if (spread_index((int)i) >= 0 && (wide || !wide_counter((int)i))) {
-            // the second word of a 32-bit counter's lines is 0
+        if (spread_index((int)i) >= 0 && !wide_counter((int)i)) {
+            uint32_t t = ctr[CT(i)];
+            for (int j = 0; j < kSpread; j++) t += ctr[CSLOT((int)i, j)];
+            pub[CT(i)] = t;
+        } else if (wide && wide_counter((int)i)) {
             uint64_t t = *reinterpret_cast<const uint64_t *>(ctr + CT(i));
             for (int j = 0; j < kSpread; j++) t += *reinterpret_cast<const uint64_t *>(ctr + CSLOT((int)i, j));
             pub[CT(i)] = (uint32_t)t;
-            if (wide_counter((int)i)) pub[CT(i) + 1] = (uint32_t)(t >> 32);
+            pub[CT(i) + 1] = (uint32_t)(t >> 32);
         }
     }
     __threadfence_system();
