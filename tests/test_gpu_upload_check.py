@@ -79,6 +79,31 @@ def test_batch_faults_are_refused(graphs, vmax, degree):
             assert_same_labels(labels[i], wants[k][0], f"graph {i}")
 
 
+@pytest.mark.parametrize("graphs", [1, 3, 12])
+def test_faults_in_small_batches(graphs):
+    """Batches small enough for the host's check, on both sides of its limit."""
+    rng = np.random.default_rng(graphs)
+    for degree in (3, 40):   # up to 12 graphs of 38 to 60 vertices, then more than 2^15 words
+        good = scc.batch_from_graphs([random_graph(int(v), int(v) * degree, rng) for v in rng.integers(38, 61, graphs)])
+        with scc.Context(0) as ctx:
+            for g in (0, graphs - 1):
+                V, E = int(good.V[g]), int(good.E[g])
+                for name, off, at, value in (("Fr", "row_off", 2, E + 1), ("Br", "row_off", V, E + 1),
+                                             ("Fc", "col_off", 0, 0), ("Fc", "col_off", E - 1, V + 1),
+                                             ("Bc", "col_off", 0, V + 1), ("Bc", "col_off", E - 1, 0xFFFFFFFF)):
+                    arrays = {k: getattr(good, k).copy() for k in ("Fr", "Fc", "Br", "Bc")}
+                    arrays[name][int(getattr(good, off)[g]) + at] = value
+                    with pytest.raises(scc.SCCError, match="invalid CSR"):
+                        ctx.batch_upload(scc.Batch(good.V, good.E, good.row_off, good.col_off, arrays["Fr"],
+                                                   arrays["Fc"], arrays["Br"], arrays["Bc"]))
+                    with pytest.raises(scc.SCCError, match="no batch"):
+                        ctx.batch_run()
+            ctx.batch_upload(good)
+            ctx.batch_run()
+            for i, lab in enumerate(ctx.batch_labels()[0]):
+                assert_same_labels(lab, orc.tarjan(good.graph(i))[0], f"graph {i}")
+
+
 def test_batch_of_wrong_offsets_is_none():
     """A larger batch whose offsets are refused does not run in the buffers of
     the batch before."""
