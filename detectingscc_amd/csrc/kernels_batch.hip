@@ -1244,14 +1244,14 @@ template <int BS> __device__ __forceinline__ uint32_t g_canon(Lds &L, const G1 &
 //
 // Under Hong's order the small-graph kernel reports the pivot and the counts
 // of trim-1's fixpoint, as the device-wide engine does.  FULL 2 trims that
-// far before the first search.  FULL 1 searches first: a pivot on a cycle is
-// none that trim-1 would have removed, and the list phases then remove and count the same
+// far before the first search, and so does FULL 1 where it sweeps anyway.
+// Otherwise FULL 1 searches first: a pivot on a cycle is none that trim-1
+// would have removed, and the list phases then remove and count the same
 // vertices (none of them lies on a path between two that stay, so the search
 // puts those into the same classes).  After an SCC of one vertex it trims, and
 // searches again if the pivot went.  Trimming first where the graph is in LDS
 // takes 999 vertices from 50.5 to 46.5 us; outside it 16,384 vertices and
-// 139,000 arcs take 126 us so and 122 searched first, 5,000 and 7,500 160 and
-// 144.
+// 139,000 arcs take 126 us so and 122 searched first.
 template <int BS, uint32_t BUC = BU_CHUNKS, int FULL = 0>
 __device__ __forceinline__ uint32_t g_solve(Lds &L, const G1 &g, uint32_t cfg)
 {
@@ -1267,9 +1267,9 @@ __device__ __forceinline__ uint32_t g_solve(Lds &L, const G1 &g, uint32_t cfg)
     const uint32_t ndeg = g_degrees<BS>(L, g, cfg_t1(cfg));
     // (never with the trims off; FULL: colouring trims once, as in the device-wide engine)
     const bool first = (uint64_t)ndeg * TRIM_MIN > g.V && !(FULL && cfg_slota(cfg));
-    if (first) g_trim_bits<BS, FULL == 2>(L, g);
+    if (first) g_trim_bits<BS, FULL != 0>(L, g);
     const bool full = FULL && cfg_t1(cfg) && !cfg_slota(cfg);
-    bool trim = full && FULL == 2;
+    bool trim = full && (FULL == 2 || first);
     if (trim) {
         if (!first) g_list_gone<BS>(L, g);   // else queue 0 holds what the last sweep removed
         g_trim_listed<BS>(L, g);
