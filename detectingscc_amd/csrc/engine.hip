@@ -718,6 +718,7 @@ scc_status Engine::reach_do(bool fw, bool bw, bool single, uint32_t *levels_out,
     }
     uint32_t level = 0;
     bool low = false;   // queue low-degree levels
+    bool thorough = false;   // max_levels does not hold: there have been low-degree levels
     auto queue = [&](int window, uint32_t blocks) {
         a.bu_ok = blocks == full;
         a.low_next = single && deg_known && !low_denied;
@@ -783,7 +784,7 @@ scc_status Engine::reach_do(bool fw, bool bw, bool single, uint32_t *levels_out,
             if (done) *done = true;
             return SCC_OK;
         }
-        if (done && seen >= max_levels) {
+        if (done && !thorough && seen >= max_levels) {
             if (levels_out) *levels_out += seen;
             *done = false;
             return SCC_OK;
@@ -836,8 +837,9 @@ scc_status Engine::reach_do(bool fw, bool bw, bool single, uint32_t *levels_out,
             low = rows != nullptr;
         }
         window = spec ? kSpecLevels : kDoWindow;
+        thorough |= low;
         // no level is queued past the bound (level <= max_levels: the first window fits it)
-        if (done) window = (int)std::min<uint32_t>((uint32_t)window, max_levels - level);
+        if (done && !thorough) window = (int)std::min<uint32_t>((uint32_t)window, max_levels - level);
         blocks = full;
         if (low) blocks = (uint32_t)std::min<int64_t>(full, std::max<int64_t>(128, (nf_max * 2 + 31) / 32));
         else if (spec) blocks = (uint32_t)std::min<int64_t>(full, std::max<int64_t>(32, (nf_max * 4 + 255) / 256));
@@ -1190,16 +1192,17 @@ scc_status Engine::run_small(char algo, bool trim1, bool trim2, scc_stats *stats
 // communities with no arc between them 822 us with the search and 690
 // without, with 1 arc in 10,000 between them 1,855 and 840; with 1 in 1,000
 // it is 587 with it and 1,018 without.
-// It is given up if it has not ended after kDetectLevels levels: on a
-// high-diameter graph the local SCCs and their quotient graph may be the
-// shorter way.  Where most arcs cross, the local SCCs are small and the
-// quotient graph nearly as deep, and it gets kDetectDeep.  A level is one
-// launch; narrow ones go on for up to 64 hops each, low-degree ones for 128,
-// so a search that is given up has cost at most about 1,300 hops, or 5,400.
-// The 1024^2 grid of 0.7 in 16 blocks of rows, which is given up, takes 18.2
-// to 18.8 ms (18.4 without a search, 19.3 with 46 levels, half of them queued
-// past the bound); in random partitions, which are searched to the end, 11 ms
-// against 9.7 s, and a cycle of 2,000 in five 1.3 against 27.6.
+// On a low-degree graph it runs to its end: a hop takes 0.5 to 0.75 us there
+// (expand_low_kernel), and the local SCCs and the quotient graph of such a
+// graph are as deep in sum (the 1024^2 grid of 0.7 in 16 blocks of rows 5.6
+// ms against 18.4, in random partitions 11 ms against 9.7 s, a cycle of 20,000
+// in 50 parts 9.8 against 55).  Otherwise it is given up if it has not ended
+// after kDetectLevels levels: on a high-diameter graph the local SCCs and
+// their quotient graph may be the shorter way.  Where most arcs cross, the
+// local SCCs are small and the quotient graph nearly as deep, and it gets
+// kDetectDeep.  A level is one launch, and narrow ones go on for up to 64 hops
+// each, so a search that is given up has cost at most about 1,000 hops of 1.3
+// to 2.1 us, or 3,000.
 static constexpr uint32_t kCrossShare = 2048;
 static constexpr uint32_t kDetectLevels = 16, kDetectDeep = 48;
 

@@ -12,10 +12,13 @@ from helpers import assert_same_labels
 pytestmark = pytest.mark.gpu
 
 
-def _grid(side, rng, p=0.8):
+def _grid(side, rng, p=0.8, diagonals=False):
     x = np.arange(side * side).reshape(side, side) + 1
     s, d = [], []
-    for a, b in ((x[:, :-1], x[:, 1:]), (x[:, 1:], x[:, :-1]), (x[:-1], x[1:]), (x[1:], x[:-1])):
+    pairs = [(x[:, :-1], x[:, 1:]), (x[:, 1:], x[:, :-1]), (x[:-1], x[1:]), (x[1:], x[:-1])]
+    if diagonals:   # more than four arcs per vertex and direction
+        pairs += [(x[:-1, :-1], x[1:, 1:]), (x[1:, 1:], x[:-1, :-1])]
+    for a, b in pairs:
         keep = rng.random(a.shape) < p
         s.append(a[keep])
         d.append(b[keep])
@@ -61,18 +64,19 @@ def test_communities(k, size, between):
     _run(g, [np.arange(g.V) // size])
 
 
-@pytest.mark.parametrize("side", [150, 700])
-def test_high_diameter(side):
-    """Low-degree graphs whose search ends within the bound, is given up, or
-    is given the longer one."""
+@pytest.mark.parametrize("side,diagonals", [(150, False), (700, False), (100, True), (900, True)])
+def test_high_diameter(side, diagonals):
+    """Low-degree graphs, which are searched to the end, and others, whose
+    search ends within the bound, is given up, or is given the longer one."""
     rng = np.random.default_rng(side)
-    g = _grid(side, rng)
+    g = _grid(side, rng, 0.6 if diagonals else 0.8, diagonals)
     _run(g, [np.arange(g.V) * 16 // g.V, rng.integers(0, 16, g.V)])
 
 
 def test_search_keeps_its_bound(monkeypatch, capfd):
-    """On a grid in blocks of rows no level past the sixteenth is run."""
-    g = _grid(1000, np.random.default_rng(1), p=0.7)
+    """On a grid with diagonals in blocks of rows no level past the sixteenth
+    is run."""
+    g = _grid(1200, np.random.default_rng(1), p=0.6, diagonals=True)
     monkeypatch.setenv("SCC_TRACE_LEVELS", "1")
     with scc.Context(0) as ctx:
         ctx.upload(g)
