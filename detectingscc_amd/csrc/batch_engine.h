@@ -43,7 +43,7 @@ class BatchEngine {
     scc_status launch(const std::vector<uint32_t> &idx, const std::vector<uint32_t> &cfg,
                       const std::vector<int> &block, double *ms, std::vector<double> *lat_ms,
                       uint32_t *launches);
-    scc_status spread_labels(const uint32_t *packed, uint64_t words, uint32_t *lab, uint32_t *const *each);
+    scc_status spread_labels(const uint32_t *packed, uint64_t words, uint32_t *lab);
 
     int dev = 0;
     hipStream_t s1 = nullptr, stream2 = nullptr;
@@ -75,6 +75,7 @@ class BatchEngine {
     static constexpr uint64_t kLabelBlock = 1 << 18;
     uint32_t *h_label = nullptr;
     uint64_t label_words = 0;
+    std::vector<uint32_t> label_host;   // the packed labels of a server's batch
     hipEvent_t ev[3] = {nullptr, nullptr, nullptr};   // start, end of each stream
     int occ[3] = {0, 0, 0};                           // workgroups per CU at 1,024, 512 and 256 lanes
     std::vector<uint32_t> stage;        // host staging of the row arrays
